@@ -81,7 +81,7 @@ def draw(rng):
     if kind == "weight_quant":
         return {"kind": kind, "n": _spread(rng, 576, 36864, 64), "k": _spread(rng, 512, 7168, 128), "dtype": dtype}
     experts, topk = rng.choice([(256, 8), (256, 8), (128, 8), (64, 6), (40, 6), (32, 5), (8, 2)])
-    dim, inter = _spread(rng, 1024, 7168, 128), rng.choice([128, 256, 256, 384, 512, 1024])
+    dim, inter = _spread(rng, 1024, 7168, 256), rng.choice([128, 256, 256, 384, 512, 1024])
     most = min(8192, _MOE_MOST // (topk * dim * inter))
     return {"kind": kind, "tokens": _spread(rng, 1, most), "experts": experts, "topk": topk, "dim": dim, "inter": inter,
             "dtype": dtype}
