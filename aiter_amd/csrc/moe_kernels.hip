@@ -1883,6 +1883,8 @@ size_t moe_workspace_bytes(const MoeArgs& a)
 {
     const size_t slots = (size_t)a.max_padded;
     size_t       b     = 0;
+    if(moe_prefill_wanted(a))
+        return moe_prefill_workspace_bytes(a);
     b += align_up(slots * a.inter * 2);          // activation product, bf16
     b += align_up(slots * a.inter);              // the same as fp8
     b += align_up(slots * scale_floats_per_slot(a) * 4); // its scales, or the row records that hold them
@@ -1895,6 +1897,26 @@ size_t moe_workspace_bytes(const MoeArgs& a)
         b += align_up((size_t)a.M * (a.dim / 128) * 4); // their scales
     }
     return b;
+}
+
+// out[token] += the token's rows, weighted, in slot order
+static hipError_t launch_combine(const MoeArgs& a, const uint16_t* y, bool y32, const int32_t* where, hipStream_t stream)
+{
+    if(!y32 && (a.dim & 7) == 0 && (a.out_stride & 7) == 0 && ((uintptr_t)a.out & 15) == 0 && ((uintptr_t)y & 15) == 0)
+    {
+        const dim3 grid8((unsigned)a.M, (unsigned)((a.dim / 8 + 255) / 256));
+        auto combine8 = a.out_dtype == In16::bf16 ? moe_combine8_kernel<In16::bf16> : moe_combine8_kernel<In16::fp16>;
+        hipLaunchKernelGGL(combine8, grid8, dim3(256), 0, stream, (const uint16_t*)y, a.sorted_weights, where, a.sorted_ids,
+                           a.num_valid, a.max_padded, (uint16_t*)a.out, a.M, a.topk, a.dim, a.out_stride);
+        return hipGetLastError();
+    }
+    const dim3 cgrid((unsigned)a.M, (unsigned)((a.dim / 4 + 255) / 256));
+    auto combine = a.out_dtype == In16::bf16
+                       ? (y32 ? moe_combine_kernel<In16::bf16, true> : moe_combine_kernel<In16::bf16, false>)
+                       : (y32 ? moe_combine_kernel<In16::fp16, true> : moe_combine_kernel<In16::fp16, false>);
+    hipLaunchKernelGGL(combine, cgrid, dim3(256), 0, stream, (const void*)y, a.sorted_weights, where, a.sorted_ids,
+                       a.num_valid, a.max_padded, (uint16_t*)a.out, a.M, a.topk, a.dim, a.out_stride);
+    return hipGetLastError();
 }
 
 hipError_t launch_fmoe_blockscale(const MoeArgs& a, hipStream_t stream, const char** why)
@@ -1910,6 +1932,14 @@ hipError_t launch_fmoe_blockscale(const MoeArgs& a, hipStream_t stream, const ch
     hipError_t    e     = workspace_acquire(ctx, lock, WsKind::moe_layer, moe_workspace_bytes(a), false, &block);
     if(e != hipSuccess)
         return e;
+    if(moe_prefill_wanted(a))
+    {
+        uint16_t* rows  = nullptr;
+        int32_t*  where = nullptr;
+        if((e = launch_moe_prefill_gemms(a, stream, block, &rows, &where)) != hipSuccess)
+            return e;
+        return launch_combine(a, rows, false, where, stream);
+    }
     uint8_t* ws = (uint8_t*)block;
     const size_t slots = (size_t)a.max_padded;
     uint16_t*    h16   = (uint16_t*)ws;
@@ -2145,21 +2175,7 @@ hipError_t launch_fmoe_blockscale(const MoeArgs& a, hipStream_t stream, const ch
                            stream, d);
     }
 
-    if(!y32 && (a.dim & 7) == 0 && (a.out_stride & 7) == 0 && ((uintptr_t)a.out & 15) == 0 && ((uintptr_t)y & 15) == 0)
-    {
-        const dim3 grid8((unsigned)a.M, (unsigned)((a.dim / 8 + 255) / 256));
-        auto combine8 = a.out_dtype == In16::bf16 ? moe_combine8_kernel<In16::bf16> : moe_combine8_kernel<In16::fp16>;
-        hipLaunchKernelGGL(combine8, grid8, dim3(256), 0, stream, (const uint16_t*)y, a.sorted_weights, where, a.sorted_ids,
-                           a.num_valid, a.max_padded, (uint16_t*)a.out, a.M, a.topk, a.dim, a.out_stride);
-        return hipGetLastError();
-    }
-    const dim3 cgrid((unsigned)a.M, (unsigned)((a.dim / 4 + 255) / 256));
-    auto combine = a.out_dtype == In16::bf16
-                       ? (y32 ? moe_combine_kernel<In16::bf16, true> : moe_combine_kernel<In16::bf16, false>)
-                       : (y32 ? moe_combine_kernel<In16::fp16, true> : moe_combine_kernel<In16::fp16, false>);
-    hipLaunchKernelGGL(combine, cgrid, dim3(256), 0, stream, (const void*)y, a.sorted_weights, where, a.sorted_ids,
-                       a.num_valid, a.max_padded, (uint16_t*)a.out, a.M, a.topk, a.dim, a.out_stride);
-    return hipGetLastError();
+    return launch_combine(a, y, y32, where, stream);
 }
 
 } // namespace fp8bs

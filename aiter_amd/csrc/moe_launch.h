@@ -70,9 +70,16 @@ struct MoeArgs
     int32_t        down_staged;    // second GEMM: 0 = 16-bit rows stored straight from the lanes, else through LDS as whole lines
     int32_t        gate_ring;      // first GEMM, pairs of blocks: 0 = every K block requested and waited for in turn, else weights two K blocks ahead through LDS
                                    // (where its tables fit); 0 = choose
+    int32_t        tiles128;       // the kernels of moe_prefill.hip (tiles of up to 128 rows of one expert): 1 / 0, -1 = choose
     int64_t        lda, out_stride;
     int            device_id;
 };
+// moe_prefill.hip: whether this call takes its kernels, their scratch, and the launches up to the second GEMM's rows
+// (bf16, by sorted slot) and the sorted position of each (token, slot) pair
+bool       moe_prefill_wanted(const MoeArgs& a);
+size_t     moe_prefill_workspace_bytes(const MoeArgs& a);
+hipError_t launch_moe_prefill_gemms(const MoeArgs& a, hipStream_t stream, void* scratch, uint16_t** rows, int32_t** where);
+
 hipError_t launch_fmoe_blockscale(const MoeArgs& a, hipStream_t stream, const char** why);
 
 } // namespace fp8bs

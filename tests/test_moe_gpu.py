@@ -384,6 +384,34 @@ def test_fmoe_rows_through_lds_give_the_same_bits(tokens, dim, inter, experts, t
     assert_close(run_moe(p, kernel_name="down=rows"), reference(p), "rows through LDS")
 
 
+@pytest.mark.parametrize("tokens,dim,inter,experts,topk,block", [
+    (70, 256, 128, 3, 2, 32),     # tiles of one and two blocks; two K blocks of the first GEMM, one of the second
+    (97, 768, 256, 2, 2, 32),     # 97 rows: a last block of one row; six K blocks (the scale windows' last is half used)
+    (129, 1280, 384, 2, 1, 64),   # ten K blocks; the second GEMM's ring with three
+    (260, 512, 1024, 2, 2, 128),  # full tiles, and blocks that are all padding inside a sorted block; ring with eight
+    (33, 8448, 256, 1, 1, 32),    # 66 K blocks: past one window of w_scale
+])
+def test_fmoe_tiles_of_rows(tokens, dim, inter, experts, topk, block):
+    # tiles of up to 128 rows of one expert (what large batches take), against the oracle; fp8 and 16-bit tokens give the
+    # same bits, and so does a second run
+    p = make_moe(tokens, dim, inter, experts, topk, seed=tokens + dim)
+    w1 = aiter_amd.shuffle_weight(p["w1q"].view(torch.uint8)).view(dtypes.fp8)
+    w2 = aiter_amd.shuffle_weight(p["w2q"].view(torch.uint8)).view(dtypes.fp8)
+    for act, name in ((0, "silu"), (1, "gelu")):
+        outs = []
+        for x16 in (False, True, False):
+            s_ids, s_w, s_e, nv, out = aiter_amd.moe_sorting(p["ti"].to(DEV), p["tw"].to(DEV), experts, dim, torch.bfloat16,
+                                                             block_size=block)
+            aiter_amd.fmoe_fp8_blockscale_g1u1(out, p["x"].to(DEV) if x16 else p["aq"].to(DEV), w1, w2, s_ids, s_w, s_e, nv,
+                                               topk, None if x16 else p["asc"].t().contiguous().to(DEV), p["w1s"], p["w2s"],
+                                               "tiles=1", 128, 128, None, act, block)
+            torch.cuda.synchronize()
+            outs.append(out)
+        assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+        assert torch.equal(outs[0].view(torch.int16), outs[2].view(torch.int16))
+        assert_close(outs[0], reference(p, name), f"tiles, {name}")
+
+
 @pytest.mark.parametrize("block", [64, 128])
 def test_fmoe_pairs_of_blocks_in_arrays_sorted_in_larger_blocks(block):
     # sorted in blocks of 64 or 128 rows, the kernels' 32-row blocks of one sorted block share an expert id:
