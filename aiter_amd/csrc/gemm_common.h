@@ -89,6 +89,7 @@ struct PrefillPlan
     int   splits;
     float us;
     int   tile_n; // 256, 192 or 128 columns per tile
+    bool  ring;   // two K ranges, one after the other on gemm_ring.hip's tiles
 };
 PrefillPlan gemm_prefill_plan(const GemmKernelParams& p, int cus);
 // want_splits: K ranges per tile; 0 lets the launcher choose, 1 keeps a tile in one workgroup.
@@ -96,6 +97,7 @@ PrefillPlan gemm_prefill_plan(const GemmKernelParams& p, int cus);
 hipError_t launch_gemm_prefill(const GemmKernelParams& p, In16 out_dtype, const LaunchCtx& ctx, int want_splits,
                                int want_tile_n = 0);
 bool       gemm_prefill_supports(const GemmKernelParams& p);
+hipError_t launch_gemm_ring(const GemmKernelParams& p, In16 out_dtype, const LaunchCtx& ctx, int kb_per_range, int device, int cus);
 hipError_t launch_gemm_decode(const GemmKernelParams& p, In16 out_dtype, int split_k_log2, const LaunchCtx& ctx,
                               const char* tuning = nullptr);
 bool       gemm_decode_supports(const GemmKernelParams& p);

@@ -569,12 +569,15 @@ bool gemm_prefill_supports(const GemmKernelParams& p)
 // 144 workgroups: 100 us; 1536 x 7168 x 2048, 168 workgroups: 36 us).  K
 // ranges over s workgroups per tile cost 4 us plus the parked tiles' traffic, (2 s - 1) x 256 KiB
 // per tile at about 5 TB/s (2048 x 4096 x 7168: 89.8 us as one range, 77-80 us as two).
-// 256 x 128 tiles: 6 us per round and 1.2 us per K block, rising to 1.4 us when the workgroups of a round
-// cover all compute units (a compute unit takes in its 48 KiB per K block no faster than the wide
-// tile's 64 KiB: what the narrow tile buys is workgroups, not speed; 1024 x 7168 x 2048: 26.4 us
-// against 34.4, 256 x 24576 x 1536: 22.5 against 30.9, 2048 x 4096 x 7168: 84.0 against 78.8 with
-// the wide tile's K ranges).
-constexpr float kFixed128 = 6.f, kIter128 = 1.2f;
+// 256 x 128 tiles are gemm_ring.hip's: 7 us and, per K block, 0.7 us with few workgroups, 0.9 us with one on every compute unit
+// (modelled / measured: 2048 x 4096 x 7168 57 / 58, 3001 x 2112 x 7168 55 / 55, 1500 x 4096 x 7168 55 / 52, 3001 x 2112 x 2048
+// 21 / 19, 2048 x 3072 x 1536 17 / 17, 1024 x 2112 x 7168 49 / 45).  One round only.
+static float ring_cost(const GemmKernelParams& p, int cus, int tiles128)
+{
+    return 7.f + (float)p.kblocks * (0.7f + 0.2f * (float)tiles128 / (float)cus);
+}
+// ... and a parked first range (2048 x 4096 x 7168 70 us, 3001 x 2112 x 7168 64)
+constexpr float kRingFold = 11.f;
 
 static float plan_cost(const GemmKernelParams& p, int cus, int bn, int s)
 {
@@ -583,8 +586,6 @@ static float plan_cost(const GemmKernelParams& p, int cus, int bn, int s)
     const int   rounds = (items + cus - 1) / cus;
     const float share  = (float)items / (float)(rounds * cus);
     const int   kb     = (p.kblocks + s - 1) / s;
-    if(bn == 128)
-        return (float)rounds * (kFixed128 + (float)kb * (kIter128 + (share > 0.44f ? (share - 0.44f) * 0.35f : 0.f)));
     if(bn == 192) // 56 KiB and 24 MFMA slots per K block: 1.4 us (4096 x 2112 x 7168, 176 workgroups: 86.9 us;
                   // 2048 x 2112 x 7168 as 88 tiles x 2 K ranges: 60.3 us against 73.1 with the wide tile),
                   // 1.5 us with a workgroup on every compute unit (8192 x 1536 x 7168, 256 tiles: 93 us)
@@ -599,7 +600,7 @@ PrefillPlan gemm_prefill_plan(const GemmKernelParams& p, int cus)
 {
     const int tiles = ((p.M + kBM - 1) / kBM) * ((p.N + 255) / 256);
     cus             = std::max(cus, 1);
-    PrefillPlan best{1, plan_cost(p, cus, 256, 1), 256};
+    PrefillPlan best{1, plan_cost(p, cus, 256, 1), 256, false};
     for(int s = 2; s <= 3; ++s)
     {
         // (below 64 tiles the model is off: 1024 x 2112 x 7168, 36 tiles x 3, takes 67 us where it
@@ -608,14 +609,7 @@ PrefillPlan gemm_prefill_plan(const GemmKernelParams& p, int cus)
             break;
         const float c = plan_cost(p, cus, 256, s);
         if(c < best.us * 0.97f)
-            best = PrefillPlan{s, c, 256};
-    }
-    // half-width tiles where the wide ones leave at least half of the compute units without a workgroup
-    if(tiles * 2 <= cus)
-    {
-        const float c = plan_cost(p, cus, 128, 1);
-        if(c < best.us * 0.97f)
-            best = PrefillPlan{1, c, 128};
+            best = PrefillPlan{s, c, 256, false};
     }
     // 192-wide tiles: no ragged last column where they divide N and 256 does not (N = 2112: a
     // ninth column of tiles that is three quarters empty against eleven full ones), and often a better
@@ -632,8 +626,19 @@ PrefillPlan gemm_prefill_plan(const GemmKernelParams& p, int cus)
                 break;
             const float c = plan_cost(p, cus, 192, s);
             if(c < best.us * 0.97f)
-                best = PrefillPlan{s, c, 192};
+                best = PrefillPlan{s, c, 192, false};
         }
+    }
+    // One round of 256 x 128 tiles.  A plan of two K ranges stays one (its sums are part of what its name says) and
+    // is only carried out on them.
+    const int t128 = ((p.M + kBM - 1) / kBM) * ((p.N + 127) / 128);
+    if(t128 <= cus)
+    {
+        const float c = ring_cost(p, cus, t128) + (best.splits == 2 ? kRingFold : 0.f);
+        if(best.splits == 1 && c < best.us * 0.97f)
+            best = PrefillPlan{1, c, 128, false};
+        else if(best.splits == 2 && c < best.us * 0.97f)
+            best = PrefillPlan{2, c, best.tile_n, true};
     }
     return best;
 }
@@ -724,6 +729,16 @@ hipError_t launch_gemm_prefill(const GemmKernelParams& p, In16 out_dtype, const 
                            : (want_splits > 0 ? 256 : plan.tile_n);
     const int splits = want_splits > 0 ? want_splits : (bn == plan.tile_n ? plan.splits : 1);
     const bool chosen = want_splits <= 0;
+    if(bn == 128 && splits == 1)
+        return launch_gemm_ring(p, out_dtype, ctx, 0, device, cus);
+    // (a caller that may not allocate gets one K range where the plan's two, in the kernel that takes a workgroup for
+    // each, would not fit the fixed buffer)
+    if(chosen && plan.ring && bn == plan.tile_n && splits == 2)
+    {
+        const size_t tiles = (size_t)((p.M + kBM - 1) / kBM) * ((p.N + bn - 1) / bn);
+        const bool   one   = ctx.static_only && tiles * 2 * kBM * bn * 4 > kStaticPartialBytes;
+        return launch_gemm_ring(p, out_dtype, ctx, one ? 0 : (p.kblocks + 1) / 2, device, cus);
+    }
     return bn == 128   ? launch_prefill_nw<4>(p, out_dtype, ctx, splits, chosen, device, cus)
            : bn == 192 ? launch_prefill_nw<6>(p, out_dtype, ctx, splits, chosen, device, cus)
                        : launch_prefill_nw<8>(p, out_dtype, ctx, splits, chosen, device, cus);

@@ -153,14 +153,16 @@ __device__ __forceinline__ void ring_fetch(lds_byte_ptr smem3, const RingSource<
 //
 // SG: w_scale blocks per wave (fragments 0, 1 and 2, 3 may belong to different 128-row blocks).
 // busy: false for a wave whose rows are all padding: it multiplies nothing.
+// kb_start: the first K block that the fetching waves bring in; a tile's blocks may be multiplied in several calls that
+// follow one another (kb_lo > kb_start continues where the call before stopped), for sums of their own.
 template <int WN, bool SHUF, bool XS4, int SG>
 __device__ __forceinline__ void ring_multiply(lds_byte_ptr smem3, const RingSource<WN>& src, int wave, int lane, int kb_lo,
-                                              int kb_hi, bool busy, float (&acc)[kRingFrags][4][4])
+                                              int kb_hi, bool busy, float (&acc)[kRingFrags][4][4], int kb_start)
 {
     using T = RingTile<WN>;
     if(!busy)
     {
-        for(int kb = kb_lo; kb <= kb_hi; ++kb)
+        for(int kb = kb_lo + (kb_lo > kb_start ? 1 : 0); kb <= kb_hi; ++kb)
             __syncthreads();
         return;
     }
@@ -192,7 +194,8 @@ __device__ __forceinline__ void ring_multiply(lds_byte_ptr smem3, const RingSour
 #pragma unroll
     for(int g = 0; g < SG; ++g)
         ws_vec[g] = load_ws_window(src.ws_row[g], kb_lo & ~63);
-    __syncthreads();
+    if(kb_lo == kb_start)
+        __syncthreads();
 
 #define FP8BS_MFMA(P, A, B) asm volatile("v_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, 0" : "=&v"(P) : "v"(A), "v"(B))
 #define FP8BS_FMA4(ACC, P, S)                                                              \
@@ -204,7 +207,7 @@ __device__ __forceinline__ void ring_multiply(lds_byte_ptr smem3, const RingSour
         asm volatile("v_fmac_f32 %0, %1, %2" : "+v"((ACC)[3]) : "v"((P)[3]), "v"(S));      \
     } while(0)
 
-    uint32_t stage = 0; // of K block kb
+    uint32_t stage = (uint32_t)((kb_lo - kb_start) % kRingStages) * T::kStageBytes; // of K block kb
 
     // The instruction stream is that of gemm_prefill.hip with four weight fragments: 16 MFMA slots per K block, the FMAs
     // that fold a product into the accumulators two slots behind its MFMA; the tiles of fragments 2 and 3 are issued

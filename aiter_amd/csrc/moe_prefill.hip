@@ -220,7 +220,7 @@ __global__ __launch_bounds__(kRingThreads) void moe_prefill_gate_up_kernel(Prefi
 
         float acc[kRingFrags][4][4];
         zero_acc(acc);
-        ring_multiply<4, true, true, 2>(smem3, src, wave, lane, 0, p.kblocks, wm * 64 < rows, acc);
+        ring_multiply<4, true, true, 2>(smem3, src, wave, lane, 0, p.kblocks, wm * 64 < rows, acc, 0);
 
         typedef u32x2 __attribute__((address_space(3)))*       lds_u2_ptr;
         typedef const u32x4 __attribute__((address_space(3)))* lds_u4_ptr;
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(kRingThreads) void moe_prefill_down_ring_kernel(Pre
 
         float acc[kRingFrags][4][4];
         zero_acc(acc);
-        ring_multiply<4, true, true, 1>(smem3, src, wave, lane, 0, p.kblocks, wm * 64 < rows, acc);
+        ring_multiply<4, true, true, 1>(smem3, src, wave, lane, 0, p.kblocks, wm * 64 < rows, acc, 0);
 
         const uint32_t ebase = (uint32_t)wave * (64u * kPitch);
         typedef u32x2 __attribute__((address_space(3)))*       lds_u2_ptr;

@@ -540,3 +540,33 @@ def test_prefill_kernel_k_ranges_across_workgroups(m, n, k, name):
     assert (outs[0].view(torch.int16) != tile.view(torch.int16)).float().mean().item() < 0.02
     rows = torch.tensor(sorted({0, 1, 255, m // 2, m - 1}), device=DEV)
     _check_rows_against_f64(outs[0], xq, wq, xs, ws, rows, f"{name or 'auto'} {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (2048, 4096, 7168),  # 256 tiles of 256 x 128: one on every compute unit
+    (1500, 4112, 7040),  # ragged rows and columns, 55 K blocks as 28 + 27
+    (300, 16384, 7168),  # a last row of tiles with 44 rows: waves without any
+    (1790, 4092, 6784),  # output rows that are not 16-byte aligned, 53 K blocks
+])
+@pytest.mark.parametrize("layout", ["plain", "preshuffled"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_two_k_ranges_one_after_the_other(m, n, k, layout, dtype):
+    # the library's own choice runs a plan of two K ranges in one workgroup per 256 x 128 tile; the plan asked for by
+    # name takes a workgroup per range: the same additions, so the same bits
+    shuffled = layout == "preshuffled"
+    n = n // 16 * 16 if shuffled else n
+    plan = _ffi.gemm_choice(m, n, k, shuffled)
+    assert plan == "prefill_256x256:s=2"
+    xq, wq, xs, ws = _gpu_problem(m, n, k, seed=m + n + k, outliers=True)
+    outs = [torch.full((m, n), float("nan"), dtype=dtype, device=DEV) for _ in range(3)]
+    if shuffled:
+        xs = xs.t().contiguous().t()
+        wq = aiter_amd.shuffle_weight(wq.view(torch.uint8)).view(wq.dtype)
+        for out, name in zip(outs, ("", plan, "")):
+            aiter_amd.gemm_a8w8_blockscale_bpreshuffle_ck(xq, wq, xs, ws, out, name)
+    else:
+        for out, name in zip(outs, ("", plan, "")):
+            aiter_amd.gemm_a8w8_blockscale_ck(xq, wq, xs, ws, out, splitK=-1, kernelName=name)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    assert torch.equal(outs[0].view(torch.int16), outs[2].view(torch.int16))
