@@ -214,21 +214,6 @@ __device__ __forceinline__ void encode16_slow(const float (&v)[16], uint32_t mm,
     scale = s;
 }
 
-// largest |x| of 16 values as a float; a NaN (which fmaxf would drop) turns it into +inf, which
-// sends the group to the slow path
-__device__ __forceinline__ float amax16(const float (&v)[16])
-{
-    float m  = 0.0f;
-    bool  un = false;
-#pragma unroll
-    for(int i = 0; i < 16; i += 2)
-    {
-        m = fmaxf(fmaxf(m, fabsf(v[i])), fabsf(v[i + 1]));
-        un |= __builtin_isunordered(v[i], v[i + 1]);
-    }
-    return un ? __builtin_inff() : m;
-}
-
 // m: the group's amax, for which amax_allows_fast_path holds
 __device__ __forceinline__ void encode16_fast(const float (&v)[16], float m, u32x4& codes, float& scale)
 {

@@ -54,6 +54,17 @@ def test_special_blocks():
     assert ws[0, 0].item() == 1.0
 
 
+@pytest.mark.parametrize("n,k", [(31, 128), (97, 384), (161, 640)])
+def test_special_block_beside_an_ordinary_one(n, k):
+    # two blocks share a workgroup; an odd last one has it to itself
+    w = tr.make_weight(n, k, seed=n)
+    w[n - 1, k - 1] = float("nan")
+    if k > 128:
+        w[3, k - 130] = float("inf")
+        w[: min(n, 128), :128] *= 1e-30
+    check(w, f"[{n},{k}]")
+
+
 def test_strided_rows_and_guard_bands():
     n, k = 200, 256
     full = tr.make_weight(n, k + 128, seed=3)
