@@ -57,6 +57,26 @@ def test_topk_softmax_ties_go_to_the_lower_index():
     assert torch.equal(ids.cpu(), rids) and torch.allclose(w.cpu(), rw, rtol=2e-6)
 
 
+@pytest.mark.parametrize("experts", [63, 64, 65, 128, 129, 256, 257, 512, 513, 1024])
+def test_topk_softmax_at_the_edges_of_a_lane_s_share(experts):
+    g = torch.Generator().manual_seed(experts)
+    gating = torch.randn(70, experts, generator=g) * 3
+    gating[1] = -float("inf")
+    gating[1, experts - 1] = -1e30      # one expert that counts, the others at weight 0
+    gating[2, ::2] = float("nan")       # a NaN is never selected
+    gating[3] = -0.0
+    w, ids = aiter_amd.fused_topk(torch.empty(70, 16, device=DEV), gating.to(DEV), 8, True)
+    torch.cuda.synchronize()
+    p = torch.softmax(torch.where(gating.isnan(), -float("inf"), gating).double(), dim=-1)
+    order = torch.sort(p.float(), dim=-1, descending=True, stable=True).indices  # ties: lower index first
+    assert ids.cpu()[1].tolist() == [experts - 1] + list(range(7))
+    assert ids.cpu()[2].tolist() == order[2, :8].tolist() and ids.cpu()[3].tolist() == list(range(8))
+    rest = [0] + list(range(4, 70))
+    rw, rids = tr.fused_topk_ref(gating[rest], 8, True)
+    assert torch.equal(ids.cpu()[rest], rids)
+    assert torch.allclose(w.cpu()[rest], rw, rtol=2e-6, atol=1e-8)
+
+
 def test_topk_softmax_rejects_what_it_cannot_do():
     with pytest.raises(RuntimeError, match="experts"):
         aiter_amd.fused_topk(torch.empty(2, 8, device=DEV), torch.zeros(2, 2000, device=DEV), 2, True)
@@ -117,6 +137,22 @@ def test_moe_sorting_expert_mask_and_local_tokens():
     check_sorting(ids, w, 32, expert_mask=mask)
     check_sorting(ids, w, 32, num_local_tokens=57)
     check_sorting(ids, w, 32, expert_mask=mask, num_local_tokens=0)
+
+
+@pytest.mark.parametrize("tokens,experts,topk,block", [
+    (513, 256, 8, 32),    # 17 chunks: the smallest sort in three launches
+    (700, 65, 6, 16),     # a second set of 64 experts with one in it
+    (9000, 1000, 8, 64),  # 71 long chunks, 16 sets of experts
+    (70000, 40, 6, 32),   # 411 chunks: two steps of the scan
+])
+def test_moe_sorting_in_three_launches(tokens, experts, topk, block):
+    g = torch.Generator().manual_seed(tokens)
+    ids = torch.rand(tokens, experts, generator=g).topk(topk, dim=-1).indices.to(torch.int32)
+    w = torch.rand(tokens, topk, generator=g)
+    mask = (torch.arange(experts) % 3 != 1).to(torch.int32)
+    check_sorting(ids, w, experts, block=block)
+    check_sorting(ids, w, experts, block=block, expert_mask=mask, num_local_tokens=tokens - 300)
+    check_sorting(ids, w, experts, block=block, num_local_tokens=0)
 
 
 def test_moe_sorting_strided_inputs_and_repeat_calls():
