@@ -17,6 +17,11 @@ import torch
 
 from .dtypes import aiter_tensor_t, shared_descriptor
 
+try:  # built beside the library; without it calls take the ctypes route below, 3 us slower
+    from . import _bridge
+except ImportError:
+    _bridge = None
+
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "libaiter_fp8bs.so")
 
@@ -89,6 +94,8 @@ def load_library():
             fn = getattr(lib, name)
             fn.argtypes = argtypes + [ctypes.c_void_p]
             fn.restype = ctypes.c_int
+            if _bridge is not None:
+                _bridge.bind(name, ctypes.cast(fn, ctypes.c_void_p).value)
         _lib = lib
     return _lib
 
@@ -107,8 +114,17 @@ def _current_stream(device_index):
 
 def call(name: str, *args):
     """Call entry point ``name``.  torch tensors become descriptors, None stays NULL, str is
-    encoded; the current stream of the first GPU tensor's device is appended."""
-    lib = load_library()
+    encoded; the current stream of the first GPU tensor's device is appended.
+
+    Plain tensors and numbers go through the native bridge; it answers None, with nothing called,
+    where an argument is anything else."""
+    lib = _lib or load_library()
+    if _bridge is not None:
+        status = _bridge.call(name, *args)
+        if status == 0:
+            return None
+        if status is not None:
+            _raise(lib, name, status)
     fn = getattr(lib, name)
     c_args, keep, device = [], [], None
     for a in args:
@@ -128,11 +144,15 @@ def call(name: str, *args):
     lib.aiter_clear_last_error()
     status = fn(*c_args)
     if status != 0:
-        raw = lib.aiter_get_last_error()
-        msg = raw.decode(errors="replace") if raw else f"ctypes status={status}"
-        lib.aiter_clear_last_error()
-        raise RuntimeError(f"{name} failed: {msg}")
+        _raise(lib, name, status)
     return None
+
+
+def _raise(lib, name, status):
+    raw = lib.aiter_get_last_error()
+    msg = raw.decode(errors="replace") if raw else f"ctypes status={status}"
+    lib.aiter_clear_last_error()
+    raise RuntimeError(f"{name} failed: {msg}")
 
 
 def gemm_kernel_names():

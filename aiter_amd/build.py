@@ -1,7 +1,8 @@
 """Builds ``libaiter_fp8bs.so`` (the C-ABI library) in-tree with hipcc for gfx950.
 
 Usage: ``python -m aiter_amd.build`` (always recompiles), or ``build_library()`` from Python.
-The library has no torch / Python dependency; it links only against the HIP runtime.
+The library has no torch / Python dependency; it links only against the HIP runtime.  The bridge
+(``_bridge.so``), through which this package calls it, is a Python extension of its own.
 """
 
 from __future__ import annotations
@@ -73,5 +74,30 @@ def build_library(verbose: bool = False) -> str:
     return LIB_PATH
 
 
+BRIDGE_PATH = os.path.join(PKG_DIR, "_bridge.so")
+
+
+def build_bridge() -> str:
+    """Compile the Python extension that calls the library with torch tensors. Returns its path."""
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    tmp = BRIDGE_PATH + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-I", sysconfig.get_paths()["include"], "-isystem", os.path.join(root, "include"),
+           "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           "-isystem", os.path.join(os.path.dirname(os.path.dirname(hipcc())), "include"),
+           os.path.join(CSRC, "bridge.cpp"), "-o", tmp,
+           "-L", os.path.join(root, "lib"), "-ltorch_python", "-lc10_hip", "-lc10", "-ltorch_cpu"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for bridge.cpp:\n{proc.stderr}")
+    os.replace(tmp, BRIDGE_PATH)
+    return BRIDGE_PATH
+
+
 if __name__ == "__main__":
     print(build_library(verbose=True))
+    print(build_bridge())

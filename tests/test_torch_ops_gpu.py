@@ -84,3 +84,43 @@ def test_compiled_expert_layer_equals_eager():
     eager = expert_layer(*args)
     got = torch.compile(expert_layer, backend="aot_eager", fullgraph=True)(*args)
     assert torch.equal(eager, got)
+
+
+def test_native_bridge_and_ctypes_route_call_alike():
+    # plain tensors go through the bridge; a subclass, which it declines, through ctypes: same call, same errors
+    from aiter_amd import _ffi
+
+    assert _ffi._bridge is not None, "aiter_amd/_bridge.so is not built"
+
+    class Sub(torch.Tensor):
+        pass
+
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(48, 1024, generator=g).bfloat16().to("cuda:0")
+    gain = torch.ones(1024, dtype=torch.bfloat16, device="cuda:0")
+    results = []
+    for cast in (lambda t: t, lambda t: t.as_subclass(Sub)):
+        y = torch.empty(48, 1024, dtype=dtypes.fp8, device="cuda:0")
+        s = torch.empty(48, 8, device="cuda:0")
+        assert _ffi._bridge.call("rmsnorm_quant", cast(y), x, s, gain, 1e-6, 128, False, False) in (0, None)
+        _ffi.call("rmsnorm_quant", cast(y), x, s, gain, 1e-6, 128, False, False)
+        results.append((y.view(torch.uint8).clone(), s.clone()))
+        with pytest.raises(RuntimeError, match="rmsnorm_quant failed: .*group"):
+            _ffi.call("rmsnorm_quant", cast(y), x, s, gain, 1e-6, 48, False, False)
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+    # on another stream, and with what neither route takes
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        y = torch.empty(48, 1024, dtype=dtypes.fp8, device="cuda:0")
+        s = torch.empty(48, 8, device="cuda:0")
+        _ffi.call("rmsnorm_quant", y, x, s, gain, 1e-6, 128, False, False)
+    side.synchronize()
+    assert torch.equal(y.view(torch.uint8), results[0][0])
+    import ctypes
+
+    with pytest.raises(ctypes.ArgumentError):
+        _ffi.call("rmsnorm_quant", y, x, s, gain, 1e-6, "128", False, False)
+    with pytest.raises((ctypes.ArgumentError, TypeError)):
+        _ffi.call("rmsnorm_quant", y, x, s, gain, 1e-6, 128, False)
+    with pytest.raises(TypeError, match="dtype"):
+        _ffi.call("rmsnorm_quant", y, x.double(), s, gain, 1e-6, 128, False, False)
