@@ -629,16 +629,17 @@ PrefillPlan gemm_prefill_plan(const GemmKernelParams& p, int cus)
                 best = PrefillPlan{s, c, 192, false};
         }
     }
-    // One round of 256 x 128 tiles.  A plan of two K ranges stays one (its sums are part of what its name says) and
-    // is only carried out on them.
+    // One round of 256 x 128 tiles, K in one range (two ranges / one: 256 x 24576 x 7168 77 / 58 us, 700 x 7168 x 7168 63 / 49,
+    // 1500 x 4096 x 7168 73 / 52).  From 2048 rows on a plan of two ranges stays one, though 2048 x 4096 x 7168 would take 58
+    // us: what the library reports there has been two ranges, callers name it, and its bits follow from it.  It is then
+    // carried out on the same tiles, one range after the other (79 -> 70 us).
     const int t128 = ((p.M + kBM - 1) / kBM) * ((p.N + 127) / 128);
     if(t128 <= cus)
     {
-        const float c = ring_cost(p, cus, t128) + (best.splits == 2 ? kRingFold : 0.f);
-        if(best.splits == 1 && c < best.us * 0.97f)
-            best = PrefillPlan{1, c, 128, false};
-        else if(best.splits == 2 && c < best.us * 0.97f)
-            best = PrefillPlan{2, c, best.tile_n, true};
+        const bool  two = best.splits == 2 && p.M >= 2048;
+        const float c   = ring_cost(p, cus, t128) + (two ? kRingFold : 0.f);
+        if(c < best.us * 0.97f && (two || best.splits == 1 || p.M < 2048))
+            best = two ? PrefillPlan{2, c, best.tile_n, true} : PrefillPlan{1, c, 128, false};
     }
     return best;
 }
