@@ -998,7 +998,7 @@ int fmoe_fp8_blockscale_g1u1(aiter_tensor_t* out, aiter_tensor_t* input, aiter_t
         // the reference's names pick among its tuned kernels; here "nt=1|2|4" pins the first GEMM's
         // columns per workgroup, "dw=" / "dc=" / "down=rows" pick the second GEMM that writes rows
         // (and its shape), "down=cols" the one that sums per token in LDS, "pair=0|1" whether consecutive
-        // blocks of one expert are multiplied in pairs, "tail=0" keeps the first GEMM's last blocks as wide as the rest, "stage=0" stores the second GEMM's 16-bit rows straight from the lanes instead of through LDS, "ring=0" has the first GEMM's pairs of blocks request and wait for every K block in turn instead of keeping the weights two K blocks ahead; "tiles=1" takes the kernels for many rows per expert (moe_prefill.hip), "tiles=0" and every hint above the block-wise ones; several hints are joined by commas; anything else
+        // blocks of one expert are multiplied in pairs, "tail=0" keeps the first GEMM's last blocks as wide as the rest, "stage=0" stores the second GEMM's 16-bit rows straight from the lanes instead of through LDS, "ring=0" has the first GEMM's pairs of blocks request and wait for every K block in turn instead of keeping the weights two K blocks ahead; "tiles=1" takes the kernels for many rows per expert (moe_prefill.hip), "tiles=0" and every hint above the block-wise ones; "out=write" stores the sums instead of adding them onto out; several hints are joined by commas; anything else
         // means choose
         a.gate_tiles     = 0;
         a.down_waves     = 0;
@@ -1009,6 +1009,7 @@ int fmoe_fp8_blockscale_g1u1(aiter_tensor_t* out, aiter_tensor_t* input, aiter_t
         a.down_staged    = -1;
         a.gate_ring      = -1;
         a.tiles128       = -1;
+        a.overwrite      = 0;
         for(const char* hint = kernel_name; hint && *hint;)
         {
             const char*  end = strchr(hint, ',');
@@ -1016,7 +1017,12 @@ int fmoe_fp8_blockscale_g1u1(aiter_tensor_t* out, aiter_tensor_t* input, aiter_t
             auto         is  = [&](const char* word) { return len == strlen(word) && strncmp(hint, word, len) == 0; };
             const int tiles128 = a.tiles128;
             a.tiles128         = 0;
-            if(len > 3 && strncmp(hint, "nt=", 3) == 0)
+            if(is("out=write"))
+            {
+                a.overwrite = 1;
+                a.tiles128  = tiles128; // (says nothing about the kernels)
+            }
+            else if(len > 3 && strncmp(hint, "nt=", 3) == 0)
                 a.gate_tiles = atoi(hint + 3);
             else if(len > 3 && strncmp(hint, "dw=", 3) == 0)
             {

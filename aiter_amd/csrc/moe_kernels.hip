@@ -1650,7 +1650,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const void* __restrict
                                                           const int32_t* __restrict__ sorted_ids,
                                                           const int32_t* __restrict__ num_valid, int32_t max_padded,
                                                           uint16_t* __restrict__ out, int32_t M, int32_t topk,
-                                                          int32_t dim, int64_t out_stride)
+                                                          int32_t dim, int64_t out_stride, int32_t overwrite)
 {
     const int quads = dim / 4;
     const int token = blockIdx.x;
@@ -1682,7 +1682,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const void* __restrict
         }
     }
     uint16_t*   dst  = out + (size_t)token * out_stride + (size_t)q * 4;
-    const u32x2 prev = *(const u32x2*)dst;
+    const u32x2 prev = overwrite ? u32x2{0u, 0u} : *(const u32x2*)dst;
     float       o[4];
     if constexpr(DT == In16::bf16)
     {
@@ -1709,7 +1709,7 @@ __global__ __launch_bounds__(256) void moe_combine8_kernel(const uint16_t* __res
                                                            const int32_t* __restrict__ sorted_ids,
                                                            const int32_t* __restrict__ num_valid, int32_t max_padded,
                                                            uint16_t* __restrict__ out, int32_t M, int32_t topk,
-                                                           int32_t dim, int64_t out_stride)
+                                                           int32_t dim, int64_t out_stride, int32_t overwrite)
 {
     const int octs  = dim / 8;
     const int token = blockIdx.x;
@@ -1747,7 +1747,7 @@ __global__ __launch_bounds__(256) void moe_combine8_kernel(const uint16_t* __res
             }
     }
     uint16_t*   dst  = out + (size_t)token * out_stride + (size_t)q * 8;
-    const u32x4 prev = *(const u32x4*)dst;
+    const u32x4 prev = overwrite ? u32x4{0u, 0u, 0u, 0u} : *(const u32x4*)dst;
     u32x4       res;
 #pragma unroll
     for(int c = 0; c < 4; ++c)
@@ -1766,6 +1766,14 @@ __global__ __launch_bounds__(256) void moe_combine8_kernel(const uint16_t* __res
         res[c] = pack2<DT>(lo + acc[2 * c], hi + acc[2 * c + 1]);
     }
     *(u32x4*)dst = res;
+}
+
+// out = 0, for a caller that wants it written where the kernels that follow add onto it (dim a multiple of 4)
+__global__ __launch_bounds__(256) void moe_zero_rows_kernel(uint16_t* __restrict__ out, int32_t dim, int64_t out_stride)
+{
+    const int q = blockIdx.y * 256 + threadIdx.x;
+    if(q < dim / 4)
+        *(u32x2*)(out + (size_t)blockIdx.x * out_stride + (size_t)q * 4) = u32x2{0u, 0u};
 }
 
 size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -1928,7 +1936,7 @@ static hipError_t launch_combine(const MoeArgs& a, const uint16_t* y, bool y32, 
         const dim3 grid8((unsigned)a.M, (unsigned)((a.dim / 8 + 255) / 256));
         auto combine8 = a.out_dtype == In16::bf16 ? moe_combine8_kernel<In16::bf16> : moe_combine8_kernel<In16::fp16>;
         hipLaunchKernelGGL(combine8, grid8, dim3(256), 0, stream, (const uint16_t*)y, a.sorted_weights, where, a.sorted_ids,
-                           a.num_valid, a.max_padded, (uint16_t*)a.out, a.M, a.topk, a.dim, a.out_stride);
+                           a.num_valid, a.max_padded, (uint16_t*)a.out, a.M, a.topk, a.dim, a.out_stride, a.overwrite);
         return hipGetLastError();
     }
     const dim3 cgrid((unsigned)a.M, (unsigned)((a.dim / 4 + 255) / 256));
@@ -1936,14 +1944,19 @@ static hipError_t launch_combine(const MoeArgs& a, const uint16_t* y, bool y32, 
                        ? (y32 ? moe_combine_kernel<In16::bf16, true> : moe_combine_kernel<In16::bf16, false>)
                        : (y32 ? moe_combine_kernel<In16::fp16, true> : moe_combine_kernel<In16::fp16, false>);
     hipLaunchKernelGGL(combine, cgrid, dim3(256), 0, stream, (const void*)y, a.sorted_weights, where, a.sorted_ids,
-                       a.num_valid, a.max_padded, (uint16_t*)a.out, a.M, a.topk, a.dim, a.out_stride);
+                       a.num_valid, a.max_padded, (uint16_t*)a.out, a.M, a.topk, a.dim, a.out_stride, a.overwrite);
     return hipGetLastError();
 }
 
 hipError_t launch_fmoe_blockscale(const MoeArgs& a, hipStream_t stream, const char** why)
 {
-    if(a.M == 0 || a.max_padded == 0)
+    if(a.M == 0)
         return hipSuccess;
+    if(a.overwrite && (a.max_padded == 0 || (!moe_prefill_wanted(a) && down_by_columns(a))))
+        hipLaunchKernelGGL(moe_zero_rows_kernel, dim3((unsigned)a.M, (unsigned)((a.dim / 4 + 255) / 256)), dim3(256), 0, stream,
+                           (uint16_t*)a.out, a.dim, a.out_stride);
+    if(a.max_padded == 0)
+        return hipGetLastError();
     LaunchCtx ctx;
     ctx.device_id = a.device_id;
     ctx.stream    = stream;

@@ -71,6 +71,7 @@ struct MoeArgs
     int32_t        gate_ring;      // first GEMM, pairs of blocks: 0 = every K block requested and waited for in turn, else weights two K blocks ahead through LDS
                                    // (where its tables fit); 0 = choose
     int32_t        tiles128;       // the kernels of moe_prefill.hip (tiles of up to 128 rows of one expert): 1 / 0, -1 = choose
+    int32_t        overwrite;      // 1: `out` is written, whatever it held; 0: accumulated into
     int64_t        lda, out_stride;
     int            device_id;
 };

@@ -490,6 +490,39 @@ def test_fmoe_is_deterministic_and_accumulates_into_out():
     assert ((got - q).norm() / q.norm()).item() < 1e-2  # one more bf16 rounding, of base + result
 
 
+@pytest.mark.parametrize("hint", ["tiles=1", "tiles=0,down=rows", "down=cols"])
+@pytest.mark.parametrize("tokens,local", [(48, None), (48, 20), (300, None), (300, 0)])
+def test_fmoe_that_writes_out_instead_of_adding(hint, tokens, local):
+    # whatever `out` held: the bits of the sum added onto zeros; tokens without a sorted row come back as zeros
+    p = make_moe(tokens, 1024, 256, 16, 4, seed=tokens)
+    w1 = aiter_amd.shuffle_weight(p["w1q"].view(torch.uint8)).view(dtypes.fp8)
+    w2 = aiter_amd.shuffle_weight(p["w2q"].view(torch.uint8)).view(dtypes.fp8)
+    n = torch.tensor([local], dtype=torch.int32, device=DEV) if local is not None else None
+    s_ids, s_w, s_e, nv, added = aiter_amd.moe_sorting(p["ti"].to(DEV), p["tw"].to(DEV), 16, 1024, torch.bfloat16,
+                                                       num_local_tokens=n)
+    written = torch.full((tokens, 1024), float("nan"), dtype=torch.bfloat16, device=DEV)
+    for out, name in ((added, hint), (written, hint + ",out=write"), (written, "out=write," + hint)):
+        aiter_amd.fmoe_fp8_blockscale_g1u1(out, p["aq"].to(DEV), w1, w2, s_ids, s_w, s_e, nv, 4,
+                                           p["asc"].t().contiguous().to(DEV), p["w1s"], p["w2s"], name)
+        torch.cuda.synchronize()
+        assert out is added or torch.equal(added.view(torch.int16), written.view(torch.int16))
+    if local is not None:
+        assert not written[local:].any().item()
+
+
+@pytest.mark.parametrize("tokens", [2047, 2048, 2300])
+def test_fused_moe_on_both_sides_of_writing_its_result(tokens):
+    p = make_moe(tokens, 512, 128, 8, 2, seed=tokens)
+    w1 = aiter_amd.shuffle_weight(p["w1q"].view(torch.uint8)).view(dtypes.fp8)
+    w2 = aiter_amd.shuffle_weight(p["w2q"].view(torch.uint8)).view(dtypes.fp8)
+    tw, ti = p["tw"].to(DEV), p["ti"].to(DEV)
+    got = aiter_amd.fused_moe(p["x"], w1, w2, tw, ti, quant_type=aiter_amd.QuantType.per_1x128, w1_scale=p["w1s"], w2_scale=p["w2s"])
+    s_ids, s_w, s_e, nv, out = aiter_amd.moe_sorting(ti, tw, 8, 512, torch.bfloat16)
+    aiter_amd.fmoe_fp8_blockscale_g1u1(out, p["x"], w1, w2, s_ids, s_w, s_e, nv, 2, None, p["w1s"], p["w2s"])
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), out.view(torch.int16))
+
+
 def test_fmoe_gelu_fp16_out_and_16bit_input():
     p = make_moe(20, 512, 128, 8, 2, seed=4, w_std=0.05)
     assert_close(run_moe(p, activation=aiter_amd.ActivationType.Gelu), reference(p, "gelu"), "gelu")
