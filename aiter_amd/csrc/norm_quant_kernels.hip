@@ -228,7 +228,7 @@ hipError_t launch_group_quant(const QuantArgs& a, hipStream_t stream)
 }
 
 // ---------------------------------------------------------------- weight-side 128x128 block quant
-// One workgroup per two neighbouring 128x128 blocks of a [N, K] weight matrix: one scale per block, codes by the
+// One workgroup per two (one) neighbouring 128x128 blocks of a [N, K] weight matrix: one scale per block, codes by the
 // same exact division as the activation quant.  Rows past N count as zeros (they do not move the
 // amax), as in the torch formulation that zero-pads ragged blocks
 // (op_tests/multigpu_tests/test_dispatch_combine.py:180-204 applies pertoken_quant,
@@ -246,12 +246,9 @@ struct WeightQuantKernelParams
     int64_t         ldw, ldq; // row strides in elements
 };
 
-constexpr int kWeightBlocks = 2;
-
-template <In16 DT>
-__global__ __launch_bounds__(256 * kWeightBlocks) void weight_block_quant_kernel(WeightQuantKernelParams p)
+template <In16 DT, int NB> // NB: blocks per workgroup
+__global__ __launch_bounds__(256 * NB) void weight_block_quant_kernel(WeightQuantKernelParams p)
 {
-    constexpr int       NB = kWeightBlocks;
     __shared__ uint32_t pattern_max[NB], bits_max[NB];
     const int  t = threadIdx.x, unit = t % (8 * NB), blk = unit >> 3;
     const int  n = blockIdx.y * 128 + t / (8 * NB); // first of this lane's four rows, 32 apart
@@ -329,11 +326,15 @@ hipError_t launch_weight_block_quant(const WeightQuantArgs& a, hipStream_t strea
     p.K     = (int32_t)a.K;
     p.ldw   = a.ldw;
     p.ldq   = a.ldq;
-    const dim3 grid((unsigned)((a.K / 128 + kWeightBlocks - 1) / kWeightBlocks), (unsigned)((a.N + 127) / 128));
-    if(a.dtype == In16::bf16)
-        hipLaunchKernelGGL(weight_block_quant_kernel<In16::bf16>, grid, dim3(256 * kWeightBlocks), 0, stream, p);
-    else
-        hipLaunchKernelGGL(weight_block_quant_kernel<In16::fp16>, grid, dim3(256 * kWeightBlocks), 0, stream, p);
+    // an odd number of K blocks leaves half of a row's last workgroup idle: with few of them that costs more than the longer
+    // row pieces give (one / two blocks per workgroup: 13568 x 1408 13.5 /
+    // 14.8 us, 40000 x 384 11.8 / 14.7, 30000 x 1920 32.9 / 36.1; 30000 x 2176, 17 K blocks, 39 either way)
+    const unsigned kblocks = (unsigned)(a.K / 128);
+    const int      nb      = (kblocks & 1) && kblocks < 16 ? 1 : 2;
+    const bool     bf      = a.dtype == In16::bf16;
+    auto kernel = nb == 1 ? (bf ? weight_block_quant_kernel<In16::bf16, 1> : weight_block_quant_kernel<In16::fp16, 1>)
+                          : (bf ? weight_block_quant_kernel<In16::bf16, 2> : weight_block_quant_kernel<In16::fp16, 2>);
+    hipLaunchKernelGGL(kernel, dim3((kblocks + nb - 1) / nb, (unsigned)((a.N + 127) / 128)), dim3(256 * nb), 0, stream, p);
     return hipGetLastError();
 }
 
