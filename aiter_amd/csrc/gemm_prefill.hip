@@ -22,9 +22,9 @@ namespace {
 constexpr int kBM = 256, kThreads = 512;
 constexpr int kStages = 2;
 constexpr int kGroupN = 4; // n tiles swept together by consecutive workgroups
-// The tile is 256 (m) x NW * 32 (n): NW = 8 weight fragments per wave for the 256 x 256 tile, 4 for the
-// 256 x 128 one (twice the workgroups where the wide tiles leave compute units idle), 6 for the
-// 256 x 192 one (N = 2112 = 11 x 192: no ragged last column of tiles).
+// The tile is 256 (m) x NW * 32 (n): NW = 8 weight fragments per wave for the 256 x 256 tile, 6 for the
+// 256 x 192 one (N = 2112 = 11 x 192: no ragged last column of tiles), 4 for a 256 x 128 tile whose K ranges
+// a caller asks for by name ("prefill_256x128:s=2"; in one range that tile is gemm_ring.hip's).
 constexpr int tile_n(int nw) { return nw * 32; }
 constexpr int slab_bytes(int nw) { return (kBM + tile_n(nw)) * 128; } // weight rows, then 256 activation rows
 constexpr int stage_bytes(int nw) { return slab_bytes(nw) + kBM * 4; } // + this K block's x_scale for the 256 rows
