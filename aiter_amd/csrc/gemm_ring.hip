@@ -52,7 +52,7 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmKernelParam
         const int tn     = group * kGroupN + (within - tm * gn);
         const int m0 = tm * T::kBM, n0 = tn * T::kBN;
 
-        RingSource<WN> src;
+        RingSource<T> src;
         src.wq      = p.wq;
         src.xq      = p.xq;
         src.xs      = (const uint8_t*)p.xs;
@@ -76,14 +76,15 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmKernelParam
                     src.goff[i] = min((uint32_t)m0 + v.row - (uint32_t)T::kBN, (uint32_t)p.M - 1u) * (uint32_t)p.lda + v.chunk * 16u;
             }
             src.xs_goff = min((uint32_t)m0 + 64u * (uint32_t)(f % T::kWM) + (uint32_t)lane, (uint32_t)p.M - 1u) * (uint32_t)p.xs_m * 4u;
-            ring_fetch<WN, SHUF, XS4>(smem3, src, f, 0, p.kblocks);
+            ring_fetch<T, SHUF, XS4>(smem3, src, f);
             __syncthreads();
             continue;
         }
-        float          acc[kRingFrags][4][4];
+        float          acc[T::kFrags][4][4];
         const uint32_t nb = min((uint32_t)(n0 + wn * 64) >> 7, (uint32_t)((p.N + 127) / 128 - 1));
         src.ws_row[0] = src.ws_row[1] = p.ws + (size_t)nb * p.kblocks;
         const bool busy = m0 + wm * 64 < p.M && n0 + wn * 64 < p.N;
+        float      ws_vec[1] = {ring_ws_window<0>(src.ws_row[0], p.kblocks, 0, lane)};
         auto zero = [&] {
 #pragma unroll
             for(int q = 0; q < 16; ++q)
@@ -99,19 +100,24 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmKernelParam
             const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
                 (uint8_t*)parked + (size_t)blockIdx.x * kParkedBytes, 0, (int)kParkedBytes, 0x00020000);
             const int at = t * 4;
-            ring_multiply<WN, SHUF, XS4, 1>(smem3, src, wave, lane, 0, fold_kb, busy, acc, 0);
+            ring_multiply<T, SHUF, XS4, 1>(smem3, src, wave, lane, 0, fold_kb, busy, ws_vec, acc);
 #pragma unroll
             for(int q = 0; q < 64; ++q)
                 __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[q >> 4][(q >> 2) & 3][q & 3]), rsrc, at, q * 2048, 0);
             zero();
-            ring_multiply<WN, SHUF, XS4, 1>(smem3, src, wave, lane, fold_kb, p.kblocks, busy, acc, 0);
+            ring_multiply<T, SHUF, XS4, 1>(smem3, src, wave, lane, fold_kb, p.kblocks, busy, ws_vec, acc);
+            // (all requested before the first is added: left to itself the compiler may wait for them one by one)
+            float back[64];
 #pragma unroll
             for(int q = 0; q < 64; ++q)
-                acc[q >> 4][(q >> 2) & 3][q & 3] =
-                    __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, at, q * 2048, 0)) + acc[q >> 4][(q >> 2) & 3][q & 3];
+                back[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, at, q * 2048, 0));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for(int q = 0; q < 64; ++q)
+                acc[q >> 4][(q >> 2) & 3][q & 3] = back[q] + acc[q >> 4][(q >> 2) & 3][q & 3];
         }
         else
-            ring_multiply<WN, SHUF, XS4, 1>(smem3, src, wave, lane, 0, p.kblocks, busy, acc, 0);
+            ring_multiply<T, SHUF, XS4, 1>(smem3, src, wave, lane, 0, p.kblocks, busy, ws_vec, acc);
 
         const uint32_t ebase = (uint32_t)wave * (64u * kOutPitch);
         typedef u32x2 __attribute__((address_space(3)))*       lds_u2_ptr;
@@ -119,7 +125,7 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmKernelParam
 #pragma unroll
         for(int j = 0; j < 4; ++j)
 #pragma unroll
-            for(int i = 0; i < kRingFrags; ++i)
+            for(int i = 0; i < T::kFrags; ++i)
                 *(lds_u2_ptr)(smem3 + ebase + (uint32_t)(j * 16 + l16) * kOutPitch + (uint32_t)(i * 16 + kg * 4) * 2u) =
                     u32x2{pack2<DT>(acc[i][j][0], acc[i][j][1]), pack2<DT>(acc[i][j][2], acc[i][j][3])};
         const int  col    = (lane & 7) * 8;

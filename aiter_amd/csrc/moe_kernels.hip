@@ -640,9 +640,8 @@ __device__ __forceinline__ PairOfBlocks pair_of_blocks(const MoeGemmParams& p, c
 // the "B" operand, so a lane ends up with 4 consecutive columns of one row.
 // waves per workgroup of the first GEMM: each keeps one K block of its tiles in flight, and a
 // workgroup that has a compute unit to itself (the last units of a launch) should still stream at
-// the unit's share of HBM
-constexpr int kGateUpWaves = 8;
-constexpr int kChipCus     = 256;
+// the unit's share of HBM (kGateUpWaves of them)
+constexpr int kChipCus = 256;
 
 // The eight waves' sums of a block meet in LDS, all MT row tiles at once: red[row tile][wave][n tile][lane][c]
 // (MT x NT x 16 KiB), and wave NT j + i adds up the pair (gate tile i, up tile NT + i) of row tile j in wave

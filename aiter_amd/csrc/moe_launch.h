@@ -39,6 +39,10 @@ struct MoeSortArgs
 // *why receives a static message when scratch memory cannot be had
 hipError_t launch_moe_sorting(const MoeSortArgs& a, hipStream_t stream, const char** why);
 
+// The first GEMM's sums, in every kernel: one chain per wave of the block-wise kernel, which takes every kGateUpWaves-th K
+// block, and the chains added in wave order.
+constexpr int kGateUpWaves = 8;
+
 struct MoeArgs
 {
     const uint8_t* xq;  // [M][dim] fp8 (row stride lda), or null when x16 is given

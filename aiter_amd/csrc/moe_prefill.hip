@@ -1,16 +1,16 @@
 // Block-scale mixture of experts, many rows per expert: the two grouped GEMMs on 128-row tiles.
 //
-// DeepSeek-V3's routed experts (256, top-8, dim 7168, inter 256), the layer on 2048 / 4096 / 8192 tokens: 541 / 930 / 1714 us
-// block by block, 448 / 623 / 947 in tiles.
+// DeepSeek-V3's routed experts (256, top-8, dim 7168, inter 256), the layer on 2048 / 8192 tokens: 553 / 1724 us block by
+// block, 515 / 1040 in tiles, with the same bits.
 //
 // The kernels of moe_kernels.hip walk the sorted rows in blocks of 32 (or pairs of them) and stream an expert's weights
 // once per block: right while the weights are what the layer reads, but with hundreds of rows per expert the same
 // weights pass through the caches many times and the matrix pipes wait.  Here the sorted rows are cut into tiles of up
 // to 128 rows of one expert, and
-//   moe_prefill_gate_up  multiplies a tile by 128 gate and 128 up rows with the three-stage ring of gemm_ring.h, applies
-//                        the activation, and quantises the product 1x128 in the same kernel;
-//   moe_prefill_down     keeps a tile's activation rows in registers (K = inter_dim of one or two K blocks) and streams
-//                        the expert's down weights past them straight into operand registers; longer K takes the ring.
+//   moe_prefill_gate_up  multiplies a tile by 128 gate and 128 up rows, 64 and 64 at a time, with the ring of gemm_ring.h,
+//                        applies the activation, and quantises the product 1x128 in the same kernel;
+//   moe_prefill_down     keeps a tile's activation rows in LDS (K = inter_dim of one or two K blocks) and streams the
+//                        expert's down weights past them straight into operand registers; longer K takes the ring.
 // The per-token sum is moe_kernels.hip's.
 #include "gemm_ring.h"
 #include "moe_launch.h"
@@ -115,13 +115,14 @@ __global__ __launch_bounds__(1024) void moe_prefill_prep_kernel(PrepParams p)
         p.tiles[0] = carry_tiles;
 }
 
-// [K/128][M] scales, as the entry point takes them with fp8 tokens, to rows of `stride` floats
+// [K/128][M] scales, as the quantiser and the entry point have them, to rows of `stride` floats in the order in which the
+// first GEMM takes its K blocks
 __global__ __launch_bounds__(256) void moe_scale_rows_kernel(const float* __restrict__ in, float* __restrict__ out, int32_t M,
                                                              int32_t kblocks, int32_t stride)
 {
-    const int m = blockIdx.x * 256 + threadIdx.x, kb = blockIdx.y;
+    const int m = blockIdx.x * 256 + threadIdx.x, pos = blockIdx.y;
     if(m < M)
-        out[(size_t)m * stride + kb] = in[(size_t)kb * M + m];
+        out[(size_t)m * stride + pos] = in[(size_t)ring_kblock<kGateUpWaves>(pos, kblocks) * M + m];
 }
 
 // Items (tile, part of its columns) in tile order.  Each of the 8 XCDs takes a contiguous eighth of them, and its
@@ -143,10 +144,11 @@ __device__ __forceinline__ float prefill_activate(float g)
     return ACT == 0 ? g / (1.f + expf(-g)) : 0.5f * g * (1.f + erff(g * 0.70710678118654752f));
 }
 
-__device__ __forceinline__ void zero_acc(float (&acc)[kRingFrags][4][4])
+template <int NF>
+__device__ __forceinline__ void zero_acc(float (&acc)[NF][4][4])
 {
 #pragma unroll
-    for(int i = 0; i < kRingFrags; ++i)
+    for(int i = 0; i < NF; ++i)
 #pragma unroll
         for(int j = 0; j < 4; ++j)
 #pragma unroll
@@ -154,20 +156,34 @@ __device__ __forceinline__ void zero_acc(float (&acc)[kRingFrags][4][4])
                 acc[i][j][r] = 0.f;
 }
 
-// First GEMM, activation and quantisation: item = (tile, 128 columns of the product).  The ring's 256 weight rows are 128
-// gate and 128 up rows, dealt out so that each wave holds 32 gate columns and the 32 up columns that belong to them: the
-// activation product is formed in registers.  It is rounded to bf16, as it would be stored, and a row's 128 columns --
-// one group of the quantiser -- meet in LDS.
-// 8192 tokens (256 rows per expert, about 1300 items of 0.94 us per K block): 345 us = 1.4 PFLOP/s of the rows' own work,
-// where the block-wise kernel takes 826; with the loads issued by the multiplying waves it took 544.
-constexpr uint32_t kHPitch = 272; // bytes per row of the bf16 product in LDS
+// First GEMM, activation and quantisation: item = (tile, 128 columns of the product), in two halves of 64 columns, each a
+// 128 x 128 tile of the ring: its weight rows are 64 gate and 64 up rows, dealt out so that a wave holds 16 gate columns and
+// the 16 up columns that belong to them, and the activation product is formed in registers.  It is rounded to bf16, as it
+// would be stored, and a row's 128 columns -- one group of the quantiser -- meet in LDS: the first half's wait behind the
+// ring while the second is multiplied, the second's land where the stages were.
+//
+// The sums are those of the block-wise kernel: kGateUpWaves chains of every kGateUpWaves-th K block, added one after the
+// other.  An fp8 code of the product follows from a sum's last bits now and then, so that the order is part of the result, and
+// one chain over all K blocks is the less precise of the two.  That takes a second set of sums per wave, and with it half the
+// columns per tile: 32 KiB taken in per K block where a 256 x 128 tile takes 48 for twice the products.  Bound by that
+// intake: 8192 tokens (256 rows per expert) 445 us, where the block-wise kernel takes 826 and 256 x 128 tiles with one chain
+// 345.  (No 256 x 128 tile holds both sets: 168 registers per wave of twelve; parked in memory they would add 256 KiB of
+// intake per chain.)
+constexpr uint32_t kHPitch = 144; // bytes per row of half a product (64 columns, bf16) in LDS
+using GateUpTile = RingTile<4, 2>;
+constexpr size_t kGateUpLds = GateUpTile::lds_bytes(true) + kTileRows * kHPitch;
+static_assert(kGateUpLds <= 160 * 1024 && kTileRows * kHPitch <= GateUpTile::kWindows, "LDS");
 template <int ACT>
 __global__ __launch_bounds__(kRingThreads) void moe_prefill_gate_up_kernel(PrefillParams p)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-    using T = RingTile<4>;
+    using T = GateUpTile;
+    constexpr int C = kGateUpWaves;
     static_assert(T::kBM == kTileRows, "a tile's rows");
+    typedef u32x2 __attribute__((address_space(3)))*       lds_u2_ptr;
+    typedef const u32x4 __attribute__((address_space(3)))* lds_u4_ptr;
     const lds_byte_ptr smem3 = (lds_byte_ptr)smem;
+    auto h_lds = [&](int half) -> lds_byte_ptr { return smem3 + (half == 0 ? (uint32_t)T::lds_bytes(true) : 0u); };
     const int groups = p.inter / 128;
     Items     it     = items_of_workgroup(p.tiles[0] * groups);
     for(; it.at < it.end; it.at += it.step)
@@ -187,7 +203,7 @@ __global__ __launch_bounds__(kRingThreads) void moe_prefill_gate_up_kernel(Prefi
             const int id = p.sorted_ids[first + min(row, rows - 1)] & 0xffffff;
             return (uint32_t)(id < p.M ? id : 0);
         };
-        RingSource<4> src;
+        RingSource<T> src;
         src.wq      = p.w + (size_t)expert * (size_t)p.N * (size_t)p.K;
         src.xq      = p.xq;
         src.xs      = (const uint8_t*)p.xs;
@@ -202,15 +218,19 @@ __global__ __launch_bounds__(kRingThreads) void moe_prefill_gate_up_kernel(Prefi
                 const RingUnit v = ring_unit(i, f, lane);
                 if(i < T::kWLoads)
                 {
-                    const uint32_t q   = v.u >> 1; // slab tile q: multiplying wave q / 4's fragment q % 4
-                    const uint32_t col = (uint32_t)grp * 8u + (q >> 2) * 2u + (q & 1u) + ((q & 2u) ? (uint32_t)p.inter >> 4 : 0u);
+                    const uint32_t q   = v.u >> 1; // slab tile q: multiplying wave q / 2's gate (even) or up tile
+                    const uint32_t col = (uint32_t)grp * 8u + (q >> 1) + ((q & 1u) ? (uint32_t)p.inter >> 4 : 0u);
                     src.goff[i]        = col * 16u * (uint32_t)p.K + (v.u & 1u) * 1024u + (uint32_t)lane * 16u;
                 }
                 else
                     src.goff[i] = token_of((int)v.row - T::kBN) * (uint32_t)p.lda + v.chunk * 16u;
             }
             src.xs_goff = token_of(64 * (f & 1) + lane) * (uint32_t)p.xs_stride * 4u;
-            ring_fetch<4, true, true>(smem3, src, f, 0, p.kblocks);
+            ring_fetch<T, true, true, C>(smem3, src, f);
+#pragma unroll
+            for(int i = 0; i < T::kWLoads; ++i)
+                src.goff[i] += 64u * (uint32_t)p.K; // four tiles on: the other half of the columns
+            ring_fetch<T, true, true, C>(smem3, src, f);
             __syncthreads();
             __syncthreads();
             continue;
@@ -218,24 +238,35 @@ __global__ __launch_bounds__(kRingThreads) void moe_prefill_gate_up_kernel(Prefi
         src.ws_row[0] = p.wsc + ((size_t)expert * (p.N / 128) + grp) * p.kblocks;
         src.ws_row[1] = src.ws_row[0] + (size_t)groups * p.kblocks;
 
-        float acc[kRingFrags][4][4];
-        zero_acc(acc);
-        ring_multiply<4, true, true, 2>(smem3, src, wave, lane, 0, p.kblocks, wm * 64 < rows, acc, 0);
-
-        typedef u32x2 __attribute__((address_space(3)))*       lds_u2_ptr;
-        typedef const u32x4 __attribute__((address_space(3)))* lds_u4_ptr;
+#pragma nounroll
+        for(int half = 0; half < 2; ++half)
+        {
+            float acc[T::kFrags][4][4], sum[T::kFrags][4][4];
+            float ws_vec[2] = {ring_ws_window<C>(src.ws_row[0], p.kblocks, 0, lane), ring_ws_window<C>(src.ws_row[1], p.kblocks, 0, lane)};
+            zero_acc(sum);
+            const int chains = min(p.kblocks, C);
+#pragma nounroll
+            for(int r = 0; r < chains; ++r)
+            {
+                zero_acc(acc);
+                ring_multiply<T, true, true, 2, C>(smem3, src, wave, lane, ring_first_position<C>(r, p.kblocks),
+                                                   ring_first_position<C>(r + 1, p.kblocks), wm * 64 < rows, ws_vec, acc);
 #pragma unroll
-        for(int j = 0; j < 4; ++j)
+                for(int q = 0; q < 16 * T::kFrags; ++q)
+                    sum[q >> 4][(q >> 2) & 3][q & 3] += acc[q >> 4][(q >> 2) & 3][q & 3];
+            }
+            const lds_byte_ptr h_at = h_lds(half) + (uint32_t)(wm * 64 + l16) * kHPitch + (uint32_t)(wn * 16 + kg * 4) * 2u;
 #pragma unroll
-            for(int i = 0; i < 2; ++i)
+            for(int j = 0; j < 4; ++j)
             {
                 float h[4];
 #pragma unroll
                 for(int r = 0; r < 4; ++r)
-                    h[r] = prefill_activate<ACT>(acc[i][j][r]) * acc[2 + i][j][r];
-                *(lds_u2_ptr)(smem3 + (uint32_t)(wm * 64 + j * 16 + l16) * kHPitch + (uint32_t)(wn * 32 + i * 16 + kg * 4) * 2u) =
+                    h[r] = prefill_activate<ACT>(sum[0][j][r]) * sum[1][j][r];
+                *(lds_u2_ptr)(h_at + (uint32_t)j * 16u * kHPitch) =
                     u32x2{pack2<In16::bf16>(h[0], h[1]), pack2<In16::bf16>(h[2], h[3])};
             }
+        }
         __syncthreads();
         // eight lanes per row, 16 columns each
 #pragma unroll
@@ -244,8 +275,9 @@ __global__ __launch_bounds__(kRingThreads) void moe_prefill_gate_up_kernel(Prefi
             const int row = (u * kRingMulThreads + t) >> 3, part = t & 7;
             if(row >= rows) // (uniform over a row's eight lanes)
                 continue;
-            const u32x4 lo = *(lds_u4_ptr)(smem3 + (uint32_t)row * kHPitch + (uint32_t)part * 32u);
-            const u32x4 hi = *(lds_u4_ptr)(smem3 + (uint32_t)row * kHPitch + (uint32_t)part * 32u + 16u);
+            const lds_byte_ptr at = h_lds(part >> 2) + (uint32_t)row * kHPitch + (uint32_t)(part & 3) * 32u;
+            const u32x4 lo = *(lds_u4_ptr)at;
+            const u32x4 hi = *(lds_u4_ptr)(at + 16u);
             float       v[16], scale;
             unpack8<In16::bf16>(lo, v);
             unpack8<In16::bf16>(hi, v + 8);
@@ -279,7 +311,7 @@ __global__ __launch_bounds__(kRingThreads) void moe_prefill_down_ring_kernel(Pre
         const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
         const int l16 = lane & 15, kg = lane >> 4;
         const int wn = wave & 3, wm = wave >> 2;
-        RingSource<4> src;
+        RingSource<T> src;
         src.wq      = p.w + (size_t)expert * (size_t)p.N * (size_t)p.K;
         src.xq      = p.xq + (size_t)first * p.K;
         src.xs      = (const uint8_t*)(p.xs + (size_t)first * p.xs_stride);
@@ -298,15 +330,15 @@ __global__ __launch_bounds__(kRingThreads) void moe_prefill_down_ring_kernel(Pre
                     src.goff[i] = min(v.row - (uint32_t)T::kBN, (uint32_t)rows - 1u) * (uint32_t)p.K + v.chunk * 16u;
             }
             src.xs_goff = min(64u * (f & 1) + lane, (uint32_t)rows - 1u) * (uint32_t)p.xs_stride * 4u;
-            ring_fetch<4, true, true>(smem3, src, f, 0, p.kblocks);
+            ring_fetch<T, true, true>(smem3, src, f);
             __syncthreads();
             continue;
         }
         src.ws_row[0] = src.ws_row[1] = p.wsc + ((size_t)expert * (p.N / 128) + (n0 + wn * 64) / 128) * p.kblocks;
 
-        float acc[kRingFrags][4][4];
+        float acc[T::kFrags][4][4], ws_vec[1] = {ring_ws_window<0>(src.ws_row[0], p.kblocks, 0, lane)};
         zero_acc(acc);
-        ring_multiply<4, true, true, 1>(smem3, src, wave, lane, 0, p.kblocks, wm * 64 < rows, acc, 0);
+        ring_multiply<T, true, true, 1>(smem3, src, wave, lane, 0, p.kblocks, wm * 64 < rows, ws_vec, acc);
 
         const uint32_t ebase = (uint32_t)wave * (64u * kPitch);
         typedef u32x2 __attribute__((address_space(3)))*       lds_u2_ptr;
@@ -314,7 +346,7 @@ __global__ __launch_bounds__(kRingThreads) void moe_prefill_down_ring_kernel(Pre
 #pragma unroll
         for(int j = 0; j < 4; ++j)
 #pragma unroll
-            for(int i = 0; i < kRingFrags; ++i)
+            for(int i = 0; i < T::kFrags; ++i)
                 *(lds_u2_ptr)(smem3 + ebase + (uint32_t)(j * 16 + l16) * kPitch + (uint32_t)(i * 16 + kg * 4) * 2u) =
                     u32x2{pack2<In16::bf16>(acc[i][j][0], acc[i][j][1]), pack2<In16::bf16>(acc[i][j][2], acc[i][j][3])};
         const int col = (lane & 7) * 8;
@@ -483,18 +515,22 @@ bool moe_prefill_wanted(const MoeArgs& a)
     if(a.tiles128 >= 0)
         return a.tiles128 != 0;
     // From where the tiles win: enough rows per expert that the block-wise kernels' repeated passes over the weights cost
-    // more than a tile's padding, and enough items for the chip (an expert's last tile is half full on average).  Measured
-    // on both sides, us block by block / in tiles (experts, topk, dim, inter):
-    //   (256, 8, 7168, 256)  32 rows per expert 362 / 388, 48: 450 / 429, 64: 541 / 448, 256: 1714 / 947
-    //   (128, 8, 4096, 384)  32: 158 / 166, 48: 190 / 175, 128: 378 / 245
-    //   (256, 8, 2048, 512)  16: 181 / 189, 24: 195 / 194, 32: 223 / 210, 256: 1041 / 478
-    //   (64, 6, 2048, 1024)  16: 107 / 101, 64: 179 / 124, 512: 964 / 349   (K of the second GEMM beyond four K blocks:
-    //                        the block-wise kernel has nothing in flight while it multiplies)
-    //   (32, 5, 4096, 256)   48 (56 items): 60 / 73, 64 (64): 75 / 74, 128: 102 / 79
-    //   (8, 2, 1024, 256)    256 (40 items): 38 / 43, 512 (72): 51 / 47
+    // more than a tile's padding, and enough items for the chip (an expert's last tile is half full on average).  Fewer rows
+    // do with many items, whose last round of workgroups matters less, and with a longer K of the second GEMM.  Measured on
+    // both sides, us block by block / in tiles (experts, topk, dim, inter):
+    //   (256, 8, 7168, 256)  rows per expert 48 (448 items): 468 / 490, 52: 494 / 479, 64: 553 / 515, 256: 1724 / 1044
+    //   (128, 8, 7168, 256)  64 (256): 294 / 319, 80 (288): 342 / 341, 96: 385 / 343
+    //   (256, 8, 3072, 128)  64 (256): 181 / 198, 80 (288): 215 / 206, 128: 299 / 236
+    //   (32, 5, 4096, 256)   96 (80): 92 / 106, 112 (88): 109 / 108, 160: 137 / 113
+    //   (8, 2, 1024, 256)    512 (72): 69 / 73, 640 (88): 72 / 72, 1024: 87 / 75
+    //   (128, 8, 4096, 384)  48 (336): 208 / 214, 56 (360): 231 / 212, 128: 392 / 291
+    //   (256, 8, 2048, 512)  32 (768): 241 / 254, 40 (832): 273 / 255, 256: 1055 / 609
+    //   (64, 6, 7168, 512)   48 (224): 238 / 275, 64 (256): 283 / 291, 80: 328 / 296
+    //   (32, 8, 7168, 1024)  32 (192): 182 / 182, 48 (224): 207 / 192, 128: 414 / 285
     const double rows  = (double)a.M * a.topk / a.experts;
     const double items = ((double)a.M * a.topk / kTileRows + 0.5 * a.experts) * (a.inter / 128);
-    return rows >= (a.inter > 512 ? 16.0 : a.inter > 256 ? 28.0 : 48.0) && items >= 60.0;
+    const double least = items >= 400.0 ? (a.inter > 256 ? 40.0 : 52.0) : a.inter > 512 ? 48.0 : a.inter > 256 ? 56.0 : 80.0;
+    return rows >= least && items >= 88.0;
 }
 
 size_t moe_prefill_workspace_bytes(const MoeArgs& a)
@@ -503,7 +539,7 @@ size_t moe_prefill_workspace_bytes(const MoeArgs& a)
     size_t       b     = align_up(slots * a.inter) + align_up(slots * row_floats(a.inter / 128) * 4) + align_up(slots * a.dim * 2) +
                align_up((size_t)a.M * a.topk * 4) + tiles_bytes(a) + align_up((size_t)a.M * row_floats(a.dim / 128) * 4);
     if(a.x16)
-        b += align_up((size_t)a.M * a.dim);
+        b += align_up((size_t)a.M * a.dim) + align_up((size_t)a.M * (a.dim / 128) * 4);
     return b;
 }
 
@@ -524,29 +560,31 @@ hipError_t launch_moe_prefill_gemms(const MoeArgs& a, hipStream_t stream, void* 
     PrepParams pp{a.sorted_ids, a.sorted_expert_ids, a.num_valid, tiles, *where, a.M, a.topk, a.experts, a.max_padded, a.max_blocks, a.expert_shift};
     hipLaunchKernelGGL(moe_prefill_prep_kernel, dim3(1 + (a.max_padded + 1023) / 1024), dim3(1024), 0, stream, pp);
 
-    const uint8_t* xq  = a.xq;
-    int64_t        lda = a.lda;
+    const uint8_t* xq    = a.xq;
+    const float*   xs_in = a.xs;
+    int64_t        lda   = a.lda;
     if(a.x16)
     {
         uint8_t*  q = take((size_t)a.M * a.dim);
+        float*    s = (float*)take((size_t)a.M * (a.dim / 128) * 4);
         QuantArgs qa{};
         qa.x                = a.x16;
         qa.y                = q;
-        qa.scale            = xs;
+        qa.scale            = s;
         qa.rows             = a.M;
         qa.groups_per_row   = a.dim / 128;
         qa.group            = 128;
         qa.num_rows_factor  = 1;
         qa.dtype            = a.x16_dtype;
-        qa.scale_row_stride = row_floats(a.dim / 128) == a.dim / 128 ? 0 : row_floats(a.dim / 128);
+        qa.transpose_scale  = true;
         if((e = launch_group_quant(qa, stream)) != hipSuccess)
             return e;
-        xq  = q;
-        lda = a.dim;
+        xq    = q;
+        xs_in = s;
+        lda   = a.dim;
     }
-    else
-        hipLaunchKernelGGL(moe_scale_rows_kernel, dim3((a.M + 255) / 256, a.dim / 128), dim3(256), 0, stream, a.xs, xs, a.M, a.dim / 128,
-                           row_floats(a.dim / 128));
+    hipLaunchKernelGGL(moe_scale_rows_kernel, dim3((a.M + 255) / 256, a.dim / 128), dim3(256), 0, stream, xs_in, xs, a.M, a.dim / 128,
+                       row_floats(a.dim / 128));
 
     static std::atomic<bool> ready[5][64];
     constexpr size_t kRingLds = RingTile<4>::lds_bytes(true);
@@ -569,9 +607,9 @@ hipError_t launch_moe_prefill_gemms(const MoeArgs& a, hipStream_t stream, void* 
     g.kblocks    = a.dim / 128;
     g.slots      = a.max_padded;
     auto gate_up = a.activation == 0 ? moe_prefill_gate_up_kernel<0> : moe_prefill_gate_up_kernel<1>;
-    if((e = raise_lds((const void*)gate_up, kRingLds, a.device_id, ready[a.activation == 0 ? 0 : 4])) != hipSuccess)
+    if((e = raise_lds((const void*)gate_up, kGateUpLds, a.device_id, ready[a.activation == 0 ? 0 : 4])) != hipSuccess)
         return e;
-    hipLaunchKernelGGL(gate_up, dim3(256), dim3(kRingThreads), kRingLds, stream, g);
+    hipLaunchKernelGGL(gate_up, dim3(256), dim3(kRingThreads), kGateUpLds, stream, g);
 
     PrefillParams d = g;
     d.xq        = hq;

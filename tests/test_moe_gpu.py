@@ -448,6 +448,23 @@ def test_fmoe_tiles_of_rows(tokens, dim, inter, experts, topk, block):
         assert_close(outs[0], reference(p, name), f"tiles, {name}")
 
 
+@pytest.mark.parametrize("tokens,dim,inter,experts,topk", [
+    (2800, 768, 128, 8, 4),    # six K blocks: fewer than the chains that their sums are made of
+    (1100, 1024, 256, 8, 8),   # eight: one per chain
+    (1000, 2304, 384, 8, 4),   # eighteen: chains of two and of three
+    (300, 7168, 256, 8, 4),    # seven per chain
+    (520, 8448, 512, 2, 2),    # 66 K blocks: past one window of w_scale
+])
+@pytest.mark.parametrize("act", [aiter_amd.ActivationType.Silu, aiter_amd.ActivationType.Gelu])
+def test_fmoe_tiles_add_up_as_the_block_wise_kernels_do(tokens, dim, inter, experts, topk, act):
+    # more than 32 MiB of rows, which both keep in 16 bits: the order of every sum is the same, so the bits are
+    p = make_moe(tokens, dim, inter, experts, topk, seed=tokens + dim)
+    want = run_moe(p, activation=act, bf16_input=True, kernel_name="tiles=0,down=rows")
+    for bf16_input in (True, False):
+        got = run_moe(p, activation=act, bf16_input=bf16_input, kernel_name="tiles=1")
+        assert torch.equal(want.view(torch.int16), got.view(torch.int16))
+
+
 @pytest.mark.parametrize("block", [64, 128])
 def test_fmoe_pairs_of_blocks_in_arrays_sorted_in_larger_blocks(block):
     # sorted in blocks of 64 or 128 rows, the kernels' 32-row blocks of one sorted block share an expert id:
