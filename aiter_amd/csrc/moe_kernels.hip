@@ -1780,12 +1780,6 @@ __global__ __launch_bounds__(256) void moe_zero_rows_kernel(uint16_t* __restrict
 
 size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 
-// The second GEMM's rows wait in memory for the per-token sum: in fp32 while the real rows
-// (tokens x topk) take at most 32 MiB -- the decode regime, where the bf16 rounding of rows that
-// largely cancel in the sum is avoided at no measurable cost -- and in bf16 beyond, where writing
-// them between the weight reads costs 5 % of the layer's time in fp32.
-bool rows_in_f32(const MoeArgs& a) { return (size_t)a.M * a.topk * a.dim * 4 <= ((size_t)32 << 20); }
-
 // Walkers per K block of moe_down_cols_kernel: two where their tables ([2 walkers][2 tiles][inter/128]
 // [tokens + 16][16] fp32) and the unit list (16 bytes per block) fit the LDS the kernel may ask for and the
 // workgroup stays within four waves, else one.
@@ -1797,10 +1791,18 @@ int cols_walkers(const MoeArgs& a)
     return (2 * one + (size_t)a.max_blocks * 16 <= kColsLdsBytes && 2 * kblocks <= 4) ? 2 : 1;
 }
 
+} // namespace
+
+// The second GEMM's rows wait in memory for the per-token sum: in fp32 while the real rows
+// (tokens x topk) take at most 32 MiB -- the decode regime, where the bf16 rounding of rows that
+// largely cancel in the sum is avoided at no measurable cost -- and in bf16 beyond, where writing
+// them between the weight reads costs 5 % of the layer's time in fp32.
+bool moe_rows_in_f32(const MoeArgs& a) { return (size_t)a.M * a.topk * a.dim * 4 <= ((size_t)32 << 20); }
+
 // Decode-size batches take the second GEMM that owns output columns and sums per token in LDS
 // (moe_down_cols_kernel): its tables and its unit list have to fit the LDS.  Beyond, rows go through
 // memory and moe_combine_kernel adds them.  down_mode 1 / 2 force the one / the other (2 only where it fits).
-bool down_by_columns(const MoeArgs& a)
+bool moe_down_by_columns(const MoeArgs& a)
 {
     const int  kblocks = a.inter / 128;
     const bool fits    = kblocks <= 4 && (size_t)kColsTiles * kblocks * (a.M + 16) * 64 <= kColsTableBytes &&
@@ -1812,8 +1814,6 @@ bool down_by_columns(const MoeArgs& a)
     // fit) 2 % slower at 288-320 tokens
     return a.down_mode == 2 || cols_walkers(a) == 2;
 }
-
-} // namespace
 
 template <typename T>
 static void launch_topk(const TopkSoftmaxArgs& a, hipStream_t stream)
@@ -1919,7 +1919,7 @@ size_t moe_workspace_bytes(const MoeArgs& a)
     b += align_up(slots * a.inter * 2);          // activation product, bf16
     b += align_up(slots * a.inter);              // the same as fp8
     b += align_up(slots * scale_floats_per_slot(a) * 4); // its scales, or the row records that hold them
-    b += align_up(slots * a.dim * (rows_in_f32(a) ? 4 : 2)); // second GEMM's rows
+    b += align_up(slots * a.dim * (moe_rows_in_f32(a) ? 4 : 2)); // second GEMM's rows
     b += align_up((size_t)a.M * a.topk * 4);     // sorted position of each (token, slot)
     b += align_up((size_t)a.max_blocks * 4);     // real rows of each block
     if(a.x16)
@@ -1941,7 +1941,7 @@ static auto combine8_kernel(int topk)
 }
 
 // out[token] += the token's rows, weighted, in slot order
-static hipError_t launch_combine(const MoeArgs& a, const uint16_t* y, bool y32, const int32_t* where, hipStream_t stream)
+static hipError_t launch_combine(const MoeArgs& a, const void* y, bool y32, const int32_t* where, hipStream_t stream)
 {
     if(!y32 && (a.dim & 7) == 0 && (a.out_stride & 7) == 0 && ((uintptr_t)a.out & 15) == 0 && ((uintptr_t)y & 15) == 0)
     {
@@ -1964,7 +1964,7 @@ hipError_t launch_fmoe_blockscale(const MoeArgs& a, hipStream_t stream, const ch
 {
     if(a.M == 0)
         return hipSuccess;
-    if(a.overwrite && (a.max_padded == 0 || (!moe_prefill_wanted(a) && down_by_columns(a))))
+    if(a.overwrite && (a.max_padded == 0 || (!moe_prefill_wanted(a) && moe_down_by_columns(a))))
         hipLaunchKernelGGL(moe_zero_rows_kernel, dim3((unsigned)a.M, (unsigned)((a.dim / 4 + 255) / 256)), dim3(256), 0, stream,
                            (uint16_t*)a.out, a.dim, a.out_stride);
     if(a.max_padded == 0)
@@ -1980,11 +1980,11 @@ hipError_t launch_fmoe_blockscale(const MoeArgs& a, hipStream_t stream, const ch
         return e;
     if(moe_prefill_wanted(a))
     {
-        uint16_t* rows  = nullptr;
+        void*     rows  = nullptr;
         int32_t*  where = nullptr;
         if((e = launch_moe_prefill_gemms(a, stream, block, &rows, &where)) != hipSuccess)
             return e;
-        return launch_combine(a, rows, false, where, stream);
+        return launch_combine(a, rows, moe_rows_in_f32(a), where, stream);
     }
     uint8_t* ws = (uint8_t*)block;
     const size_t slots = (size_t)a.max_padded;
@@ -1994,14 +1994,14 @@ hipError_t launch_fmoe_blockscale(const MoeArgs& a, hipStream_t stream, const ch
     ws += align_up(slots * a.inter);
     float* hs = (float*)ws;
     ws += align_up(slots * scale_floats_per_slot(a) * 4);
-    const bool y32 = rows_in_f32(a);
+    const bool y32 = moe_rows_in_f32(a);
     uint16_t*  y   = (uint16_t*)ws;
     ws += align_up(slots * a.dim * (y32 ? 4 : 2));
     int32_t* where = (int32_t*)ws; // sorted position of each (token, slot) pair; stale where the pair is not routed here
     ws += align_up((size_t)a.M * a.topk * 4);
     uint32_t* block_mask = (uint32_t*)ws;
     ws += align_up((size_t)a.max_blocks * 4);
-    const bool cols = down_by_columns(a);
+    const bool cols = moe_down_by_columns(a);
 
     const uint8_t* xq = a.xq;
     const float*   xs = a.xs;

@@ -36,7 +36,7 @@ struct PrefillParams
     const int32_t* tiles;  // [0] the number of tiles, then from [2] on {first block, blocks | expert << 8} each
     uint8_t*       hq;     // gate/up: codes of the activation product [slots][inter]
     float*         hs;     // and their scales [slots][hs_stride]
-    uint16_t*      y;      // down: rows [slots][N], bf16
+    void*          y;      // down: rows [slots][N], bf16 or fp32
     int64_t        lda;
     int32_t        M, K, N, inter, kblocks, slots, xs_stride, hs_stride;
     int32_t        col_splits; // down from registers: parts a tile's columns are cut into
@@ -291,12 +291,15 @@ __global__ __launch_bounds__(kRingThreads) void moe_prefill_gate_up_kernel(Prefi
     }
 }
 
-// Second GEMM on the ring, for K of three and more K blocks: item = (tile, 256 columns).
+// Second GEMM on the ring, for K of three and more K blocks: item = (tile, 256 columns).  F32: rows kept in fp32.
+template <bool F32>
 __global__ __launch_bounds__(kRingThreads) void moe_prefill_down_ring_kernel(PrefillParams p)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     using T = RingTile<4>;
-    constexpr uint32_t kPitch = 144; // bytes per row of a wave's 64 x 64 output block in LDS
+    constexpr uint32_t kSize = F32 ? 4 : 2, kPitch = 64 * kSize + 16; // bytes per row of a wave's 64 x 64 output block in LDS
+    constexpr int      kLanes = 4 * kSize;                            // lanes that store a row of it, 16 bytes each
+    static_assert(8 * 64 * kPitch <= T::kWindows, "LDS");
     const lds_byte_ptr smem3 = (lds_byte_ptr)smem;
     const int parts = p.N / T::kBN;
     Items     it    = items_of_workgroup(p.tiles[0] * parts);
@@ -341,22 +344,28 @@ __global__ __launch_bounds__(kRingThreads) void moe_prefill_down_ring_kernel(Pre
         ring_multiply<T, true, true, 1>(smem3, src, wave, lane, 0, p.kblocks, wm * 64 < rows, ws_vec, acc);
 
         const uint32_t ebase = (uint32_t)wave * (64u * kPitch);
+        typedef f32x4 __attribute__((address_space(3)))*       lds_f4_ptr;
         typedef u32x2 __attribute__((address_space(3)))*       lds_u2_ptr;
         typedef const u32x4 __attribute__((address_space(3)))* lds_u4_ptr;
 #pragma unroll
         for(int j = 0; j < 4; ++j)
 #pragma unroll
             for(int i = 0; i < T::kFrags; ++i)
-                *(lds_u2_ptr)(smem3 + ebase + (uint32_t)(j * 16 + l16) * kPitch + (uint32_t)(i * 16 + kg * 4) * 2u) =
-                    u32x2{pack2<In16::bf16>(acc[i][j][0], acc[i][j][1]), pack2<In16::bf16>(acc[i][j][2], acc[i][j][3])};
-        const int col = (lane & 7) * 8;
+            {
+                const lds_byte_ptr at = smem3 + ebase + (uint32_t)(j * 16 + l16) * kPitch + (uint32_t)(i * 16 + kg * 4) * kSize;
+                if constexpr(F32)
+                    *(lds_f4_ptr)at = f32x4{acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+                else
+                    *(lds_u2_ptr)at = u32x2{pack2<In16::bf16>(acc[i][j][0], acc[i][j][1]), pack2<In16::bf16>(acc[i][j][2], acc[i][j][3])};
+            }
+        const int piece = lane % kLanes;
 #pragma unroll
-        for(int c = 0; c < 8; ++c)
+        for(int c = 0; c < kLanes; ++c)
         {
-            const int   row = c * 8 + (lane >> 3);
-            const u32x4 v   = *(lds_u4_ptr)(smem3 + ebase + (uint32_t)row * kPitch + (uint32_t)col * 2u);
+            const int   row = c * (64 / kLanes) + lane / kLanes;
+            const u32x4 v   = *(lds_u4_ptr)(smem3 + ebase + (uint32_t)row * kPitch + (uint32_t)piece * 16u);
             if(wm * 64 + row < rows)
-                *(u32x4*)(p.y + (size_t)(first + wm * 64 + row) * p.N + n0 + wn * 64 + col) = v;
+                *(u32x4*)((uint8_t*)p.y + ((size_t)(first + wm * 64 + row) * p.N + n0 + wn * 64) * kSize + piece * 16) = v;
         }
         __syncthreads();
     }
@@ -369,21 +378,24 @@ __global__ __launch_bounds__(kRingThreads) void moe_prefill_down_ring_kernel(Pre
 // takes is requests in flight, 16 KiB per wave here.  8192 tokens: 295 us for 0.94 GB of rows and 0.47 GB of weights (4.8
 // TB/s, a plain copy runs at 5.1); with the rows in registers and one weight tile ahead 367 us, block by block 583.
 constexpr int      kDownWaves = 4;
-constexpr uint32_t kDownPitch = 144;
+constexpr uint32_t down_pitch(bool f32) { return f32 ? 272u : 144u; }
 constexpr uint32_t down_x_bytes(int kb) { return (uint32_t)kb * kTileRows * 128u; }
-constexpr uint32_t down_lds_bytes(int kb) { return down_x_bytes(kb) + (uint32_t)kb * kTileRows * 4u + kDownWaves * 16u * kDownPitch; }
+constexpr uint32_t down_lds_bytes(int kb, bool f32) { return down_x_bytes(kb) + (uint32_t)kb * kTileRows * 4u + kDownWaves * 16u * down_pitch(f32); }
 
-template <int KB>
+template <int KB, bool F32>
 __global__ __launch_bounds__(64 * kDownWaves, 2) void moe_prefill_down_kernel(PrefillParams p)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    constexpr uint32_t kSize = F32 ? 4 : 2, kPitch = down_pitch(F32);
+    constexpr int      kLanes = 4 * kSize; // lanes that store 64 columns of a row, 16 bytes each
     typedef float __attribute__((address_space(3)))*       lds_float_ptr;
+    typedef f32x4 __attribute__((address_space(3)))*       lds_f4_ptr;
     typedef u32x2 __attribute__((address_space(3)))*       lds_u2_ptr;
     typedef const u32x4 __attribute__((address_space(3)))* lds_u4_ptr;
     typedef const i32x4 __attribute__((address_space(3)))* lds_i4_ptr;
     const lds_byte_ptr smem3 = (lds_byte_ptr)smem;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), l16 = lane & 15, kg = lane >> 4;
-    const lds_byte_ptr  stage  = smem3 + down_x_bytes(KB) + KB * kTileRows * 4 + (uint32_t)wave * (16u * kDownPitch);
+    const lds_byte_ptr  stage  = smem3 + down_x_bytes(KB) + KB * kTileRows * 4 + (uint32_t)wave * (16u * kPitch);
     const lds_float_ptr xs_lds = (lds_float_ptr)(smem3 + down_x_bytes(KB)); // [KB][rows]
     const uint32_t sw     = lds_swizzle((uint32_t)l16);
     const uint32_t lo_off = (uint32_t)l16 * 128u + (((2u * kg) ^ sw) << 4);
@@ -440,16 +452,19 @@ __global__ __launch_bounds__(64 * kDownWaves, 2) void moe_prefill_down_kernel(Pr
                         for(int c = 0; c < 4; ++c)
                             acc[c] = __builtin_fmaf(prod[c], sc[kb], acc[c]);
                     }
-                    *(lds_u2_ptr)(stage + (uint32_t)l16 * kDownPitch + (uint32_t)(i * 16 + kg * 4) * 2u) =
-                        u32x2{pack2<In16::bf16>(acc[0], acc[1]), pack2<In16::bf16>(acc[2], acc[3])};
+                    const lds_byte_ptr at = stage + (uint32_t)l16 * kPitch + (uint32_t)(i * 16 + kg * 4) * kSize;
+                    if constexpr(F32)
+                        *(lds_f4_ptr)at = acc;
+                    else
+                        *(lds_u2_ptr)at = u32x2{pack2<In16::bf16>(acc[0], acc[1]), pack2<In16::bf16>(acc[2], acc[3])};
                 }
                 // (a wave's LDS operations complete in the order they were issued)
 #pragma unroll
-                for(int h = 0; h < 2; ++h)
+                for(int h = 0; h < kLanes / 4; ++h)
                 {
-                    const int   row = h * 8 + (lane >> 3), c = lane & 7;
-                    const u32x4 v   = *(lds_u4_ptr)(stage + (uint32_t)row * kDownPitch + (uint32_t)c * 16u);
-                    *(u32x4*)(p.y + (size_t)(first + j * 16 + row) * p.N + g * 64 + c * 8) = v;
+                    const int   row = h * (64 / kLanes) + lane / kLanes, c = lane % kLanes;
+                    const u32x4 v   = *(lds_u4_ptr)(stage + (uint32_t)row * kPitch + (uint32_t)c * 16u);
+                    *(u32x4*)((uint8_t*)p.y + ((size_t)(first + j * 16 + row) * p.N + g * 64) * kSize + c * 16) = v;
                 }
             }
         };
@@ -514,43 +529,48 @@ bool moe_prefill_wanted(const MoeArgs& a)
         return false;
     if(a.tiles128 >= 0)
         return a.tiles128 != 0;
+    if(moe_down_by_columns(a)) // few tokens, whose sums never leave fp32
+        return false;
     // From where the tiles win: enough rows per expert that the block-wise kernels' repeated passes over the weights cost
     // more than a tile's padding, and enough items for the chip (an expert's last tile is half full on average).  Fewer rows
-    // do with many items, whose last round of workgroups matters less, and with a longer K of the second GEMM.  Measured on
-    // both sides, us block by block / in tiles (experts, topk, dim, inter):
+    // do with many items, whose last round of workgroups matters less (unless the rows are kept in fp32), and with a longer K
+    // of the second GEMM.  Measured on both sides, us block by block / in tiles (experts, topk, dim, inter):
     //   (256, 8, 7168, 256)  rows per expert 48 (448 items): 468 / 490, 52: 494 / 479, 64: 553 / 515, 256: 1724 / 1044
     //   (128, 8, 7168, 256)  64 (256): 294 / 319, 80 (288): 342 / 341, 96: 385 / 343
     //   (256, 8, 3072, 128)  64 (256): 181 / 198, 80 (288): 215 / 206, 128: 299 / 236
     //   (32, 5, 4096, 256)   96 (80): 92 / 106, 112 (88): 109 / 108, 160: 137 / 113
-    //   (8, 2, 1024, 256)    512 (72): 69 / 73, 640 (88): 72 / 72, 1024: 87 / 75
+    //   (8, 2, 1024, 256)    640 (88, fp32 rows): 72 / 75, 768 (104): 79 / 75, 1024: 88 / 77
     //   (128, 8, 4096, 384)  48 (336): 208 / 214, 56 (360): 231 / 212, 128: 392 / 291
     //   (256, 8, 2048, 512)  32 (768): 241 / 254, 40 (832): 273 / 255, 256: 1055 / 609
     //   (64, 6, 7168, 512)   48 (224): 238 / 275, 64 (256): 283 / 291, 80: 328 / 296
-    //   (32, 8, 7168, 1024)  32 (192): 182 / 182, 48 (224): 207 / 192, 128: 414 / 285
+    //   (32, 8, 7168, 1024)  32 (192, fp32 rows): 183 / 198, 48 (224): 207 / 192, 128: 414 / 291
+    //   (64, 6, 2048, 1024)  40 (416, fp32 rows): 150 / 158, 48 (448): 162 / 158, 64: 204 / 174
     const double rows  = (double)a.M * a.topk / a.experts;
     const double items = ((double)a.M * a.topk / kTileRows + 0.5 * a.experts) * (a.inter / 128);
-    const double least = items >= 400.0 ? (a.inter > 256 ? 40.0 : 52.0) : a.inter > 512 ? 48.0 : a.inter > 256 ? 56.0 : 80.0;
-    return rows >= least && items >= 88.0;
+    const bool   many  = items >= 400.0 && !moe_rows_in_f32(a);
+    const double least = many ? (a.inter > 256 ? 40.0 : 52.0) : a.inter > 512 ? 48.0 : a.inter > 256 ? 56.0 : 80.0;
+    return rows >= least && items >= 92.0;
 }
 
 size_t moe_prefill_workspace_bytes(const MoeArgs& a)
 {
     const size_t slots = (size_t)a.max_padded;
-    size_t       b     = align_up(slots * a.inter) + align_up(slots * row_floats(a.inter / 128) * 4) + align_up(slots * a.dim * 2) +
+    size_t       b     = align_up(slots * a.inter) + align_up(slots * row_floats(a.inter / 128) * 4) + align_up(slots * a.dim * (moe_rows_in_f32(a) ? 4 : 2)) +
                align_up((size_t)a.M * a.topk * 4) + tiles_bytes(a) + align_up((size_t)a.M * row_floats(a.dim / 128) * 4);
     if(a.x16)
         b += align_up((size_t)a.M * a.dim) + align_up((size_t)a.M * (a.dim / 128) * 4);
     return b;
 }
 
-hipError_t launch_moe_prefill_gemms(const MoeArgs& a, hipStream_t stream, void* scratch, uint16_t** rows, int32_t** where)
+hipError_t launch_moe_prefill_gemms(const MoeArgs& a, hipStream_t stream, void* scratch, void** rows, int32_t** where)
 {
     uint8_t*     ws    = (uint8_t*)scratch;
     auto         take  = [&](size_t bytes) { uint8_t* at = ws; ws += align_up(bytes); return at; };
     const size_t slots = (size_t)a.max_padded;
     uint8_t*  hq = take(slots * a.inter);
     float*    hs = (float*)take(slots * row_floats(a.inter / 128) * 4);
-    uint16_t* y  = (uint16_t*)take(slots * a.dim * 2);
+    const bool f32 = moe_rows_in_f32(a);
+    void*     y  = take(slots * a.dim * (f32 ? 4 : 2));
     *where = (int32_t*)take((size_t)a.M * a.topk * 4);
     *rows  = y;
     int32_t* tiles = (int32_t*)take(tiles_bytes(a));
@@ -586,7 +606,7 @@ hipError_t launch_moe_prefill_gemms(const MoeArgs& a, hipStream_t stream, void* 
     hipLaunchKernelGGL(moe_scale_rows_kernel, dim3((a.M + 255) / 256, a.dim / 128), dim3(256), 0, stream, xs_in, xs, a.M, a.dim / 128,
                        row_floats(a.dim / 128));
 
-    static std::atomic<bool> ready[5][64];
+    static std::atomic<bool> ready[8][64];
     constexpr size_t kRingLds = RingTile<4>::lds_bytes(true);
     PrefillParams    g{};
     g.xq         = xq;
@@ -607,7 +627,7 @@ hipError_t launch_moe_prefill_gemms(const MoeArgs& a, hipStream_t stream, void* 
     g.kblocks    = a.dim / 128;
     g.slots      = a.max_padded;
     auto gate_up = a.activation == 0 ? moe_prefill_gate_up_kernel<0> : moe_prefill_gate_up_kernel<1>;
-    if((e = raise_lds((const void*)gate_up, kGateUpLds, a.device_id, ready[a.activation == 0 ? 0 : 4])) != hipSuccess)
+    if((e = raise_lds((const void*)gate_up, kGateUpLds, a.device_id, ready[a.activation == 0 ? 0 : 1])) != hipSuccess)
         return e;
     hipLaunchKernelGGL(gate_up, dim3(256), dim3(kRingThreads), kGateUpLds, stream, g);
 
@@ -626,18 +646,19 @@ hipError_t launch_moe_prefill_gemms(const MoeArgs& a, hipStream_t stream, void* 
     {
         // each wave of an item walks about seven groups of columns: enough to amortise the tile's rows, and enough items
         d.col_splits = std::max(1, a.dim / 64 / (7 * kDownWaves));
-        const int    inst = d.kblocks;
-        const size_t lds  = down_lds_bytes(inst);
-        auto kernel = inst == 1 ? moe_prefill_down_kernel<1> : moe_prefill_down_kernel<2>;
-        if((e = raise_lds((const void*)kernel, lds, a.device_id, ready[inst])) != hipSuccess)
+        const size_t lds = down_lds_bytes(d.kblocks, f32);
+        auto kernel = d.kblocks == 1 ? (f32 ? moe_prefill_down_kernel<1, true> : moe_prefill_down_kernel<1, false>)
+                                     : (f32 ? moe_prefill_down_kernel<2, true> : moe_prefill_down_kernel<2, false>);
+        if((e = raise_lds((const void*)kernel, lds, a.device_id, ready[(f32 ? 3 : 1) + d.kblocks])) != hipSuccess)
             return e;
         hipLaunchKernelGGL(kernel, dim3(512), dim3(64 * kDownWaves), lds, stream, d);
     }
     else
     {
-        if((e = raise_lds((const void*)moe_prefill_down_ring_kernel, kRingLds, a.device_id, ready[3])) != hipSuccess)
+        auto kernel = f32 ? moe_prefill_down_ring_kernel<true> : moe_prefill_down_ring_kernel<false>;
+        if((e = raise_lds((const void*)kernel, kRingLds, a.device_id, ready[f32 ? 7 : 6])) != hipSuccess)
             return e;
-        hipLaunchKernelGGL(moe_prefill_down_ring_kernel, dim3(256), dim3(kRingThreads), kRingLds, stream, d);
+        hipLaunchKernelGGL(kernel, dim3(256), dim3(kRingThreads), kRingLds, stream, d);
     }
     return hipGetLastError();
 }

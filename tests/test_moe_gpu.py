@@ -465,6 +465,31 @@ def test_fmoe_tiles_add_up_as_the_block_wise_kernels_do(tokens, dim, inter, expe
         assert torch.equal(want.view(torch.int16), got.view(torch.int16))
 
 
+@pytest.mark.parametrize("tokens,dim,inter,experts,topk", [
+    (97, 512, 128, 3, 2),     # the second GEMM with its rows in LDS, one K block and two
+    (682, 2048, 256, 64, 6),
+    (247, 2304, 512, 32, 5),  # its ring, four K blocks and eight
+    (171, 2048, 1024, 64, 6),
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_fmoe_tiles_keep_few_rows_in_fp32(tokens, dim, inter, experts, topk, dtype):
+    # up to 32 MiB the rows wait for the per-token sum in fp32: rounded to bf16 first, an fp16 result would be eight times
+    # as far off.  The same sums as block by block, so the same bits, by the library's own choice too
+    p = make_moe(tokens, dim, inter, experts, topk, seed=tokens + dim, w_std=0.05)
+    want = run_moe(p, dtype=dtype, bf16_input=True, kernel_name="tiles=0,down=rows")
+    got = run_moe(p, dtype=dtype, bf16_input=True, kernel_name="tiles=1")
+    assert torch.equal(want.view(torch.int16), got.view(torch.int16))
+    if tokens > 600 or inter > 256:  # (else the column kernel's choice)
+        assert torch.equal(want.view(torch.int16), run_moe(p, dtype=dtype, bf16_input=True).view(torch.int16))
+
+
+def test_fmoe_tiles_leave_few_tokens_to_the_column_kernel():
+    # 500 tokens, top-16: rows and items enough for tiles, but the column kernel's tables still fit: it sums in fp32
+    p = make_moe(500, 512, 128, 64, 16, seed=5)
+    want = run_moe(p, bf16_input=True, kernel_name="down=cols")
+    assert torch.equal(want.view(torch.int16), run_moe(p, bf16_input=True).view(torch.int16))
+
+
 @pytest.mark.parametrize("block", [64, 128])
 def test_fmoe_pairs_of_blocks_in_arrays_sorted_in_larger_blocks(block):
     # sorted in blocks of 64 or 128 rows, the kernels' 32-row blocks of one sorted block share an expert id:
