@@ -14,6 +14,7 @@
 // The per-token sum is moe_kernels.hip's.
 #include "gemm_ring.h"
 #include "moe_launch.h"
+#include "moe_rules.h"
 #include "quant_stage.h"
 
 #include <algorithm>
@@ -25,6 +26,7 @@ namespace {
 
 constexpr int kTileBlocks = 4;                // sorted blocks of 32 rows per tile
 constexpr int kTileRows   = 32 * kTileBlocks; // = RingTile<4>::kBM
+static_assert(kTileRows == kTileRowsOfExpert, "the rule counts such tiles");
 
 struct PrefillParams
 {
@@ -531,25 +533,9 @@ bool moe_prefill_wanted(const MoeArgs& a)
         return a.tiles128 != 0;
     if(moe_down_by_columns(a)) // few tokens, whose sums never leave fp32
         return false;
-    // From where the tiles win: enough rows per expert that the block-wise kernels' repeated passes over the weights cost
-    // more than a tile's padding, and enough items for the chip (an expert's last tile is half full on average).  Fewer rows
-    // do with many items, whose last round of workgroups matters less (unless the rows are kept in fp32), and with a longer K
-    // of the second GEMM.  Measured on both sides, us block by block / in tiles (experts, topk, dim, inter):
-    //   (256, 8, 7168, 256)  rows per expert 48 (448 items): 468 / 490, 52: 494 / 479, 64: 553 / 515, 256: 1724 / 1044
-    //   (128, 8, 7168, 256)  64 (256): 294 / 319, 80 (288): 342 / 341, 96: 385 / 343
-    //   (256, 8, 3072, 128)  64 (256): 181 / 198, 80 (288): 215 / 206, 128: 299 / 236
-    //   (32, 5, 4096, 256)   96 (80): 92 / 106, 112 (88): 109 / 108, 160: 137 / 113
-    //   (8, 2, 1024, 256)    640 (88, fp32 rows): 72 / 75, 768 (104): 79 / 75, 1024: 88 / 77
-    //   (128, 8, 4096, 384)  48 (336): 208 / 214, 56 (360): 231 / 212, 128: 392 / 291
-    //   (256, 8, 2048, 512)  32 (768): 241 / 254, 40 (832): 273 / 255, 256: 1055 / 609
-    //   (64, 6, 7168, 512)   48 (224): 238 / 275, 64 (256): 283 / 291, 80: 328 / 296
-    //   (32, 8, 7168, 1024)  32 (192, fp32 rows): 183 / 198, 48 (224): 207 / 192, 128: 414 / 291
-    //   (64, 6, 2048, 1024)  40 (416, fp32 rows): 150 / 158, 48 (448): 162 / 158, 64: 204 / 174
-    const double rows  = (double)a.M * a.topk / a.experts;
-    const double items = ((double)a.M * a.topk / kTileRows + 0.5 * a.experts) * (a.inter / 128);
-    const bool   many  = items >= 400.0 && !moe_rows_in_f32(a);
-    const double least = many ? (a.inter > 256 ? 40.0 : 52.0) : a.inter > 512 ? 48.0 : a.inter > 256 ? 56.0 : 80.0;
-    return rows >= least && items >= 92.0;
+    const int64_t pairs = (int64_t)a.M * a.topk;
+    const int64_t all   = routed_experts(pairs, a.topk, a.block_rows << a.expert_shift, a.max_padded, a.experts);
+    return tiles_win(pairs, all, a.experts, a.inter, moe_rows_in_f32(a));
 }
 
 size_t moe_prefill_workspace_bytes(const MoeArgs& a)

@@ -1,0 +1,48 @@
+// When the expert layer takes the kernels for many rows per expert (moe_prefill.hip).  Plain C++ (no HIP), so that the rule can
+// be compiled and tested on the host.
+#pragma once
+
+#include <stdint.h>
+
+namespace fp8bs {
+
+constexpr int kTileRowsOfExpert = 128; // most rows of one expert in a tile
+
+// The experts that the tokens' `pairs` = tokens x topk were routed to, of which `experts` are held here.  An expert-parallel
+// rank sorts with all of them and holds a part; how many pairs are its own only the device knows, but the sorted arrays are
+// sized for every expert's last block (pairs + all x unit - topk slots; padded: that in whole blocks).
+inline int64_t routed_experts(int64_t pairs, int topk, int unit, int64_t padded, int experts)
+{
+    const int64_t all = (padded - pairs + topk + unit - 1) / unit;
+    return all > experts ? all : experts;
+}
+
+// Tiles win where an expert has enough rows that the block-wise kernels' repeated passes over its weights cost more than a
+// tile's padding, and where there are enough items (a tile's 128 columns of the product; an expert's last tile is half full
+// on average) for the chip.  Fewer rows do with many items, whose last round of workgroups matters less (unless the rows are
+// kept in fp32), and with a longer K of the second GEMM.  Measured on both sides, us block by block / in tiles (experts,
+// topk, dim, inter):
+//   (256, 8, 7168, 256)  rows per expert 48 (448 items): 468 / 490, 52: 494 / 479, 64: 553 / 515, 256: 1724 / 1044
+//   (128, 8, 7168, 256)  64 (256): 294 / 319, 80 (288): 342 / 341, 96: 385 / 343
+//   (256, 8, 3072, 128)  64 (256): 181 / 198, 80 (288): 215 / 206, 128: 299 / 236
+//   (32, 5, 4096, 256)   96 (80): 92 / 106, 112 (88): 109 / 108, 160: 137 / 113
+//   (8, 2, 1024, 256)    640 (88, fp32 rows): 72 / 75, 768 (104): 79 / 75, 1024: 88 / 77
+//   (128, 8, 4096, 384)  48 (336): 208 / 214, 56 (360): 231 / 212, 128: 392 / 291
+//   (256, 8, 2048, 512)  32 (768): 241 / 254, 40 (832): 273 / 255, 256: 1055 / 609
+//   (64, 6, 7168, 512)   48 (224): 238 / 275, 64 (256): 283 / 291, 80: 328 / 296
+//   (32, 8, 7168, 1024)  32 (192, fp32 rows): 183 / 198, 48 (224): 207 / 192, 128: 414 / 291
+//   (64, 6, 2048, 1024)  40 (416, fp32 rows): 150 / 158, 48 (448): 162 / 158, 64: 204 / 174
+//   (16, 4, 4096, 2048)  32 (192, fp32 rows): 121 / 112, 128: 284 / 180
+//   (32 held of 256, 8, 7168, 2048)  2: 245 / 273, 16 (320): 293 / 299, 32 (384): 396 / 319, 256: 1635 / 815
+//   (64 held of 256, 8, 4096, 1024)  16: 187 / 219, 32 (384): 226 / 229, 64: 337 / 252
+// `all`: the experts that the pairs are spread over, as routed_experts says.
+inline bool tiles_win(int64_t pairs, int64_t all, int experts, int inter, bool rows_f32)
+{
+    const double rows  = (double)pairs / (double)all;
+    const double items = (rows * experts / kTileRowsOfExpert + 0.5 * experts) * (inter / 128);
+    const bool   many  = items >= 400.0 && !rows_f32;
+    const double least = inter > 1024 ? 32.0 : many ? (inter > 256 ? 40.0 : 52.0) : inter > 512 ? 48.0 : inter > 256 ? 56.0 : 80.0;
+    return rows >= least && items >= 92.0;
+}
+
+} // namespace fp8bs

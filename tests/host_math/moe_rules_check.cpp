@@ -1,0 +1,51 @@
+// Host check of the rule by which the expert layer takes its kernels for many rows per expert (aiter_amd/csrc/moe_rules.h).
+// Prints OK or the first failed expectation.
+#include "../../aiter_amd/csrc/moe_rules.h"
+
+#include <cstdio>
+#include <initializer_list>
+
+#define EXPECT(cond)                                                                             \
+    do                                                                                           \
+    {                                                                                            \
+        if(!(cond))                                                                              \
+        {                                                                                        \
+            std::printf("FAILED line %d: %s (tokens %d, experts %d)\n", __LINE__, #cond, m, e);  \
+            return 1;                                                                            \
+        }                                                                                        \
+    } while(0)
+
+using namespace fp8bs;
+
+// slots as the sort's arrays are sized, in whole blocks
+static int64_t padded(int64_t pairs, int topk, int unit, int all) { return (pairs + (int64_t)all * unit - topk) / unit * unit; }
+
+int main()
+{
+    int m = 0, e = 0;
+    for(int unit : {32, 64, 128})
+        for(int topk : {1, 2, 5, 8})
+            for(m = 1; m < 9000; m += 37)
+                for(int all : {8, 33, 256, 1000})
+                    for(int held : {1, all / 8, all / 2, all})
+                    {
+                        const int64_t pairs = (int64_t)m * topk, p = padded(pairs, topk, unit, all);
+                        e = held;
+                        EXPECT(routed_experts(pairs, topk, unit, p, e) == all);
+                        // arrays that say less than the weights: the experts held are the least there are
+                        EXPECT(routed_experts(pairs, topk, unit, pairs / unit * unit, 1000) == 1000);
+                        // a rank that holds a part of the experts sees the rows per expert of the whole: no more tiles than
+                        // with all of them, whatever its own part
+                        for(int inter : {128, 256, 512, 2048})
+                            if(tiles_win(pairs, all, e, inter, false))
+                                EXPECT(tiles_win(pairs, all, all, inter, false));
+                    }
+    // 32 of 256 experts held: a decode batch of 64 tokens has two rows per expert, not sixteen
+    e = 32;
+    for(m = 1; m <= 512; ++m)
+        EXPECT(!tiles_win((int64_t)m * 8, routed_experts((int64_t)m * 8, 8, 32, padded((int64_t)m * 8, 8, 32, 256), e), e, 2048, m < 147));
+    m = 8192;
+    EXPECT(tiles_win((int64_t)m * 8, 256, e, 256, false) && tiles_win((int64_t)m * 8, 256, 256, 256, false));
+    std::printf("OK\n");
+    return 0;
+}

@@ -37,6 +37,14 @@ def test_capture_lane_bookkeeping(tmp_path):
     assert out.returncode == 0 and out.stdout.startswith("OK"), out.stdout + out.stderr
 
 
+def test_expert_layer_rule_counts_rows_per_routed_expert(tmp_path):
+    """An expert-parallel rank holds a part of the experts its tokens are routed to: aiter_amd/csrc/moe_rules.h on the host."""
+    exe = str(tmp_path / "moe_rules_check")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-o", exe, os.path.join(HERE, "host_math", "moe_rules_check.cpp")])
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0 and out.stdout.startswith("OK"), out.stdout + out.stderr
+
+
 def test_kernel_choice_query_on_the_headline_shapes():
     """The shape rule that stands in for the reference's tuned-table lookup (get_CKGEMM_config,
     aiter/ops/gemm_op_a8w8.py:448-490) can be asked without a GPU."""

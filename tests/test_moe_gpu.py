@@ -483,6 +483,23 @@ def test_fmoe_tiles_keep_few_rows_in_fp32(tokens, dim, inter, experts, topk, dty
         assert torch.equal(want.view(torch.int16), run_moe(p, dtype=dtype, bf16_input=True).view(torch.int16))
 
 
+@pytest.mark.parametrize("tokens,inter", [(300, 256), (2500, 384)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_fmoe_tiles_on_an_expert_parallel_rank(tokens, inter, dtype):
+    # a third of the experts is held here: pairs routed to the others have no sorted row
+    p = make_moe(tokens, 1024, inter, 24, 4, seed=tokens, w_std=0.05)
+    mask = (torch.arange(24) % 3 == 1).to(torch.int32)
+    held = mask.nonzero().flatten().to(DEV)
+    for name in ("w1q", "w2q"):
+        p[name] = p[name].view(torch.uint8)[held].view(dtypes.fp8).contiguous()
+    for name in ("w1s", "w2s"):
+        p[name] = p[name][held].contiguous()
+    want = run_moe(p, dtype=dtype, expert_mask=mask, bf16_input=True, kernel_name="tiles=0,down=rows")
+    got = run_moe(p, dtype=dtype, expert_mask=mask, bf16_input=True, kernel_name="tiles=1")
+    assert torch.equal(want.view(torch.int16), got.view(torch.int16))
+    assert want.float().norm() > 0
+
+
 def test_fmoe_tiles_leave_few_tokens_to_the_column_kernel():
     # 500 tokens, top-16: rows and items enough for tiles, but the column kernel's tables still fit: it sums in fp32
     p = make_moe(500, 512, 128, 64, 16, seed=5)
