@@ -44,7 +44,7 @@ struct PrefillParams
     int32_t        col_splits; // down from registers: parts a tile's columns are cut into
 };
 
-// The tiles of the sorted rows, by one workgroup, and the position of each (token, slot) pair, by the others.
+// The tiles of the sorted rows, by one workgroup, and the position of each (token, slot) pair (-1: none), by the others.
 struct PrepParams
 {
     const int32_t* sorted_ids;
@@ -52,7 +52,7 @@ struct PrepParams
     const int32_t* num_valid;
     int32_t*       tiles;
     int32_t*       where;
-    int32_t        M, topk, experts, max_padded, max_blocks, expert_shift;
+    int32_t        M, topk, experts, max_padded, expert_shift;
 };
 __global__ __launch_bounds__(1024) void moe_prefill_prep_kernel(PrepParams p)
 {
@@ -64,8 +64,9 @@ __global__ __launch_bounds__(1024) void moe_prefill_prep_kernel(PrepParams p)
         if(at < valid_rows)
         {
             const int id = p.sorted_ids[at], token = id & 0xffffff, slot = (id >> 24) & 0xff;
-            if(token < p.M && slot < p.topk)
-                p.where[(size_t)token * p.topk + slot] = at;
+            const int e  = p.sorted_expert_ids[(at >> 5) >> p.expert_shift];
+            if(token < p.M && slot < p.topk) // (a block of an expert that is not held here has no tile, and its rows no sums)
+                p.where[(size_t)token * p.topk + slot] = e >= 0 && e < p.experts ? at : -1;
         }
         return;
     }
@@ -563,7 +564,7 @@ hipError_t launch_moe_prefill_gemms(const MoeArgs& a, hipStream_t stream, void* 
     float*   xs    = (float*)take((size_t)a.M * row_floats(a.dim / 128) * 4);
     hipError_t e;
 
-    PrepParams pp{a.sorted_ids, a.sorted_expert_ids, a.num_valid, tiles, *where, a.M, a.topk, a.experts, a.max_padded, a.max_blocks, a.expert_shift};
+    PrepParams pp{a.sorted_ids, a.sorted_expert_ids, a.num_valid, tiles, *where, a.M, a.topk, a.experts, a.max_padded, a.expert_shift};
     hipLaunchKernelGGL(moe_prefill_prep_kernel, dim3(1 + (a.max_padded + 1023) / 1024), dim3(1024), 0, stream, pp);
 
     const uint8_t* xq    = a.xq;

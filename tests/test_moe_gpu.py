@@ -500,6 +500,22 @@ def test_fmoe_tiles_on_an_expert_parallel_rank(tokens, inter, dtype):
     assert want.float().norm() > 0
 
 
+@pytest.mark.parametrize("block", [32, 128])
+def test_fmoe_tiles_skip_blocks_of_experts_that_are_not_held(block):
+    # sorted for six experts, weights for four: the other two's rows count for nothing, whatever an earlier call left behind
+    p = make_moe(200, 512, 128, 6, 2, seed=9)
+    w1 = aiter_amd.shuffle_weight(p["w1q"].view(torch.uint8)).view(dtypes.fp8)
+    w2 = aiter_amd.shuffle_weight(p["w2q"].view(torch.uint8)).view(dtypes.fp8)
+    ti, outs = p["ti"].to(DEV), []
+    for tw, held in ((p["tw"] * (p["ti"] < 4), 6), (p["tw"], 4)):
+        s_ids, s_w, s_e, nv, out = aiter_amd.moe_sorting(ti, tw.to(DEV), 6, 512, torch.bfloat16, block_size=block)
+        aiter_amd.fmoe_fp8_blockscale_g1u1(out, p["x"], w1[:held], w2[:held], s_ids, s_w, s_e, nv, 2, None, p["w1s"][:held],
+                                           p["w2s"][:held], "tiles=1", 128, 128, None, 0, block)
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
 def test_fmoe_tiles_leave_few_tokens_to_the_column_kernel():
     # 500 tokens, top-16: rows and items enough for tiles, but the column kernel's tables still fit: it sums in fp32
     p = make_moe(500, 512, 128, 64, 16, seed=5)
