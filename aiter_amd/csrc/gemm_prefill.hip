@@ -576,8 +576,9 @@ static float ring_cost(const GemmKernelParams& p, int cus, int tiles128)
 {
     return 7.f + (float)p.kblocks * (0.7f + 0.2f * (float)tiles128 / (float)cus);
 }
-// ... and a parked first range (2048 x 4096 x 7168 70 us, 3001 x 2112 x 7168 64)
-constexpr float kRingFold = 11.f;
+// ... and a parked first range (modelled / measured: 2048 x 4096 x 7168 63 / 63, 3001 x 2112 x 7168 61 / 53, 300 x 16384 x
+// 7168 54 / 55, 700 x 7168 x 7168 60 / 49, 256 x 24576 x 7168 61 / 72)
+constexpr float kRingFold = 6.f;
 
 static float plan_cost(const GemmKernelParams& p, int cus, int bn, int s)
 {
@@ -629,17 +630,18 @@ PrefillPlan gemm_prefill_plan(const GemmKernelParams& p, int cus)
                 best = PrefillPlan{s, c, 192, false};
         }
     }
-    // One round of 256 x 128 tiles, K in one range (two ranges / one: 256 x 24576 x 7168 77 / 58 us, 700 x 7168 x 7168 63 / 49,
-    // 1500 x 4096 x 7168 73 / 52).  From 2048 rows on a plan of two ranges stays one, though 2048 x 4096 x 7168 would take 58
-    // us: what the library reports there has been two ranges, callers name it, and its bits follow from it.  It is then
-    // carried out on the same tiles, one range after the other (79 -> 70 us).
+    // One round of 256 x 128 tiles.  They carry a plan out, they do not change its sums: two K ranges stay two, one after the
+    // other in a workgroup (us in the kernel with a workgroup per range / here: 2048 x 4096 x 7168 75 / 63, 2048 x 2304 x 7168
+    // 50 / 44, 700 x 7168 x 7168 58 / 49).  In one range they take 4-5 us less, with an error against 64 bits that is the same to
+    // seven digits; but a call's K ranges, and the bits that follow, are what the library says they are.
     const int t128 = ((p.M + kBM - 1) / kBM) * ((p.N + 127) / 128);
     if(t128 <= cus)
     {
-        const bool  two = best.splits == 2 && p.M >= 2048;
-        const float c   = ring_cost(p, cus, t128) + (two ? kRingFold : 0.f);
-        if(c < best.us * 0.97f && (two || best.splits == 1 || p.M < 2048))
-            best = two ? PrefillPlan{2, c, best.tile_n, true} : PrefillPlan{1, c, 128, false};
+        const float c = ring_cost(p, cus, t128) + (best.splits == 2 ? kRingFold : 0.f);
+        if(best.splits == 1 && c < best.us * 0.97f)
+            best = PrefillPlan{1, c, 128, false};
+        else if(best.splits == 2 && c < best.us * 0.97f)
+            best = PrefillPlan{2, c, best.tile_n, true};
     }
     return best;
 }

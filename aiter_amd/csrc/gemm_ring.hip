@@ -6,8 +6,8 @@
 // Bound by what a compute unit takes in: 48 KiB per K block, 0.75 us with few workgroups, 0.9 us with 256 (13 TB/s out of L2
 // over the chip; the matrix pipes need 0.45).  The two-stage tiles of gemm_prefill.hip wait for each K block's loads
 // instead (1.2-1.8 us).  us there / here: 3001 x 2112 x 2048 24.1 / 19.3, 2048 x 4096 x 3584 39.8 / 33.8,
-// 3000 x 2560 x 5120 59.5 / 43.1; two ranges: 3001 x 2112 x 7168 75 / 64, 2048 x 4096 x 7168 79 / 70,
-// 300 x 16384 x 7168 77 / 57.  With more than one round the 256 x 256 tile, 64 KiB for twice the products, is ahead again
+// 3000 x 2560 x 5120 59.5 / 43.1; two ranges: 3001 x 2112 x 7168 70 / 53, 2048 x 4096 x 7168 75 / 63,
+// 300 x 16384 x 7168 78 / 55.  With more than one round the 256 x 256 tile, 64 KiB for twice the products, is ahead again
 // (4096^3: 64 / 68).
 #include "gemm_ring.h"
 
@@ -96,7 +96,7 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmKernelParam
         if constexpr(FOLD)
         {
             // The second of two ranges of K blocks starts a sum of its own.  There are no 64 registers for the first
-            // one's: it waits in memory, each thread reads back what it wrote (10 us of 70 at 2048 x 4096 x 7168).
+            // one's: it waits in memory, each thread reads back what it wrote (5 us of 63 at 2048 x 4096 x 7168).
             const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
                 (uint8_t*)parked + (size_t)blockIdx.x * kParkedBytes, 0, (int)kParkedBytes, 0x00020000);
             const int at = t * 4;

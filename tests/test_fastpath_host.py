@@ -37,6 +37,17 @@ def test_capture_lane_bookkeeping(tmp_path):
     assert out.returncode == 0 and out.stdout.startswith("OK"), out.stdout + out.stderr
 
 
+def test_k_ranges_of_a_plan_do_not_depend_on_the_kernel_that_carries_them_out():
+    # two ranges of K are two sums: the choice is the same on both sides of any number of rows, and 256 x 128 tiles, which
+    # take the ranges one after the other, do not turn them into one
+    from aiter_amd import _ffi
+
+    for n, k in ((4096, 7168), (3504, 7040)):
+        assert {_ffi.gemm_choice(m, n, k) for m in range(1793, 2049, 15)} == {"prefill_256x256:s=2"}
+    for m, n, k in ((256, 24576, 7168), (300, 16384, 7168), (700, 7168, 7168), (1500, 4096, 7168), (2048, 2304, 7168)):
+        assert _ffi.gemm_choice(m, n, k).endswith(":s=2")
+
+
 def test_expert_layer_rule_counts_rows_per_routed_expert(tmp_path):
     """An expert-parallel rank holds a part of the experts its tokens are routed to: aiter_amd/csrc/moe_rules.h on the host."""
     exe = str(tmp_path / "moe_rules_check")

@@ -544,8 +544,11 @@ def test_prefill_kernel_k_ranges_across_workgroups(m, n, k, name):
 
 @pytest.mark.parametrize("m,n,k", [
     (2048, 4096, 7168),  # 256 tiles of 256 x 128: one on every compute unit
-    (2100, 3504, 7040),  # ragged rows and columns, 55 K blocks as 28 + 27
-    (2090, 3500, 6784),  # a last row of tiles with 42 rows: waves without any; output rows not 16-byte aligned, 53 K blocks
+    (1500, 4112, 7040),  # ragged rows and columns, 55 K blocks as 28 + 27
+    (300, 16384, 7168),  # a last row of tiles with 44 rows: waves without any
+    (1790, 4092, 6784),  # output rows that are not 16-byte aligned, 53 K blocks
+    (2100, 3504, 7040),  # the same on the other side of 2048 rows
+    (2090, 3500, 6784),
 ])
 @pytest.mark.parametrize("layout", ["plain", "preshuffled"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
