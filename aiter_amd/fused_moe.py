@@ -180,7 +180,7 @@ def fused_moe(hidden_states, w1, w2, topk_weight, topk_ids, expert_mask=None, ac
         topk_ids, topk_weight, num_experts, dim, dtype, block_m, expert_mask, num_local_tokens,
         moe_sorting_dispatch_policy, accumulate=not write_out)
     if write_out:
-        out = torch.empty((tokens, dim), dtype=dtype, device=topk_ids.device)
+        out = torch.empty((topk_ids.shape[0], dim), dtype=dtype, device=topk_ids.device)
     if hidden_states.dtype in (torch.bfloat16, torch.float16):
         a1, scale_t = hidden_states, None
     else:

@@ -598,6 +598,17 @@ def test_fused_moe_on_both_sides_of_writing_its_result(tokens):
     assert torch.equal(got.view(torch.int16), out.view(torch.int16))
 
 
+@pytest.mark.parametrize("tokens", [2047, 2048, 2300])
+@pytest.mark.parametrize("more", [-1, 1])
+def test_fused_moe_refuses_routing_of_another_number_of_tokens(tokens, more):
+    p = make_moe(tokens, 512, 128, 8, 2, seed=tokens)
+    w1 = aiter_amd.shuffle_weight(p["w1q"].view(torch.uint8)).view(dtypes.fp8)
+    w2 = aiter_amd.shuffle_weight(p["w2q"].view(torch.uint8)).view(dtypes.fp8)
+    rows = (torch.arange(tokens + more) % tokens)
+    with pytest.raises(RuntimeError, match="out must be"):
+        aiter_amd.fused_moe(p["x"], w1, w2, p["tw"][rows].to(DEV), p["ti"][rows].to(DEV), w1_scale=p["w1s"], w2_scale=p["w2s"])
+
+
 def test_fmoe_gelu_fp16_out_and_16bit_input():
     p = make_moe(20, 512, 128, 8, 2, seed=4, w_std=0.05)
     assert_close(run_moe(p, activation=aiter_amd.ActivationType.Gelu), reference(p, "gelu"), "gelu")
