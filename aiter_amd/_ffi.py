@@ -12,6 +12,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 
 import torch
 
@@ -19,8 +20,9 @@ from .dtypes import aiter_tensor_t, shared_descriptor
 
 try:  # built beside the library; without it calls take the ctypes route below, 3 us slower
     from . import _bridge
-except ImportError:
+except ImportError as _error:
     _bridge = None
+    _bridge_error = _error
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "libaiter_fp8bs.so")
@@ -96,6 +98,13 @@ def load_library():
             fn.restype = ctypes.c_int
             if _bridge is not None:
                 _bridge.bind(name, ctypes.cast(fn, ctypes.c_void_p).value)
+        if _bridge is None:
+            warnings.warn(
+                f"aiter_amd._bridge cannot be loaded ({_bridge_error}): calls from Python take 3 us longer; "
+                "build it for this torch with `python -m aiter_amd.build`",
+                RuntimeWarning,
+                stacklevel=2,
+            )
         _lib = lib
     return _lib
 

@@ -12,7 +12,7 @@ usable under functionalisation, which the reference's generic wrapper does not g
   itself;
 * an op never returns one of its inputs.
 
-Eager calls bypass the dispatcher (one ctypes call, no schema matching): only while a compiler is
+Eager calls bypass the dispatcher (one native call, no schema matching): only while a compiler is
 tracing does an entry point go through ``torch.ops.aiter``.
 """
 

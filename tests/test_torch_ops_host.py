@@ -105,3 +105,25 @@ def test_whole_graph_tracing_without_breaks():
         gm, _ = torch._dynamo.export(expert_layer)(*margs)
         called = [str(n.target) for n in gm.graph.nodes if n.op == "call_function" and "aiter" in str(n.target)]
         assert called == ["aiter.topk_softmax", "aiter.moe_sorting_fwd", "aiter.fmoe_fp8_blockscale_g1u1"]
+
+
+@pytest.mark.parametrize("missing", [False, True])
+def test_a_bridge_that_cannot_be_loaded_is_said(missing):
+    # the calls still work, by ctypes and slower: once, and with the reason
+    import subprocess
+    import sys
+
+    code = (
+        "import sys, warnings\n"
+        f"missing = {missing}\n"
+        "if missing: sys.modules['aiter_amd._bridge'] = None\n"
+        "import aiter_amd\n"
+        "from aiter_amd import _ffi\n"
+        "with warnings.catch_warnings(record=True) as seen:\n"
+        "    warnings.simplefilter('always')\n"
+        "    _ffi.gemm_choice(1, 512, 512), _ffi.gemm_choice(1, 512, 512)\n"
+        "text = [str(w.message) for w in seen if w.category is RuntimeWarning]\n"
+        "assert len(text) == missing and (not missing or '_bridge' in text[0]), text\n"
+    )
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert done.returncode == 0, done.stderr
