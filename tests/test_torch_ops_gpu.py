@@ -99,23 +99,37 @@ def test_native_bridge_and_ctypes_route_call_alike():
     x = torch.randn(48, 1024, generator=g).bfloat16().to("cuda:0")
     gain = torch.ones(1024, dtype=torch.bfloat16, device="cuda:0")
     results = []
-    for cast in (lambda t: t, lambda t: t.as_subclass(Sub)):
-        y = torch.empty(48, 1024, dtype=dtypes.fp8, device="cuda:0")
-        s = torch.empty(48, 8, device="cuda:0")
-        assert _ffi._bridge.call("rmsnorm_quant", cast(y), x, s, gain, 1e-6, 128, False, False) in (0, None)
-        _ffi.call("rmsnorm_quant", cast(y), x, s, gain, 1e-6, 128, False, False)
-        results.append((y.view(torch.uint8).clone(), s.clone()))
+    for cast, status in ((lambda t: t, 0), (lambda t: t.as_subclass(Sub), None)):  # None: declined, nothing called
+        outs = []
+        for call in (_ffi._bridge.call, _ffi.call):
+            y = torch.full((48, 1024), 7, dtype=torch.uint8, device="cuda:0").view(dtypes.fp8)
+            s = torch.full((48, 8), -1.0, device="cuda:0")
+            got = call("rmsnorm_quant", cast(y), x, s, gain, 1e-6, 128, False, False)
+            assert got == status if call is _ffi._bridge.call else got is None
+            outs.append((y.view(torch.uint8).clone(), s.clone()))
+        if status is None:
+            assert (outs[0][0] == 7).all() and (outs[0][1] == -1).all()
+            del outs[0]
+        results += outs
         with pytest.raises(RuntimeError, match="rmsnorm_quant failed: .*group"):
             _ffi.call("rmsnorm_quant", cast(y), x, s, gain, 1e-6, 48, False, False)
-    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
-    # on another stream, and with what neither route takes
-    side = torch.cuda.Stream()
-    with torch.cuda.stream(side):
+    assert len(results) == 3
+    for y8, scale in results[1:]:
+        assert torch.equal(results[0][0], y8) and torch.equal(results[0][1], scale)
+    assert not (results[0][0] == 7).all() and (results[0][1] > 0).all()
+    # on the current stream: the call waits for what that stream does before it, which takes a while
+    for cast in (lambda t: t, lambda t: t.as_subclass(Sub)):
+        late = torch.zeros_like(x)
         y = torch.empty(48, 1024, dtype=dtypes.fp8, device="cuda:0")
         s = torch.empty(48, 8, device="cuda:0")
-        _ffi.call("rmsnorm_quant", y, x, s, gain, 1e-6, 128, False, False)
-    side.synchronize()
-    assert torch.equal(y.view(torch.uint8), results[0][0])
+        side = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(50_000_000)
+            late.copy_(x)
+            _ffi.call("rmsnorm_quant", cast(y), late, s, gain, 1e-6, 128, False, False)
+        side.synchronize()
+        assert torch.equal(y.view(torch.uint8), results[0][0]) and torch.equal(s, results[0][1])
     import ctypes
 
     with pytest.raises(ctypes.ArgumentError):
