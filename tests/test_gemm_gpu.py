@@ -543,6 +543,29 @@ def test_prefill_kernel_k_ranges_across_workgroups(m, n, k, name):
 
 
 @pytest.mark.parametrize("m,n,k", [
+    (2100, 5000, 1024),  # 360 tiles of 256 x 128, the last ones ragged; x_scale four K blocks per load
+    (2560, 8192, 640),   # 640 tiles, up to three per workgroup; x_scale K block by K block
+])
+@pytest.mark.parametrize("layout", ["plain", "preshuffled"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_256x128_tiles_beyond_one_round(m, n, k, layout, dtype):
+    # by name the kernel takes any size: a workgroup's second tile lands where the first one's output was
+    n = n // 16 * 16 if layout == "preshuffled" else n
+    xq, wq, xs, ws = _gpu_problem(m, n, k, seed=m + n + k, outliers=True)
+    out = torch.full((m, n), float("nan"), dtype=dtype, device=DEV)
+    tile = torch.full_like(out, float("nan"))
+    aiter_amd.gemm_a8w8_blockscale_ck(xq, wq, xs, ws, tile, kernelName="tile_128x128")
+    if layout == "preshuffled":
+        xs = xs.t().contiguous().t()
+        wq = aiter_amd.shuffle_weight(wq.view(torch.uint8)).view(wq.dtype)
+        aiter_amd.gemm_a8w8_blockscale_bpreshuffle_ck(xq, wq, xs, ws, out, "prefill_256x128")
+    else:
+        aiter_amd.gemm_a8w8_blockscale_ck(xq, wq, xs, ws, out, splitK=-1, kernelName="prefill_256x128")
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), tile.view(torch.int16))
+
+
+@pytest.mark.parametrize("m,n,k", [
     (2048, 4096, 7168),  # 256 tiles of 256 x 128: one on every compute unit
     (1500, 4112, 7040),  # ragged rows and columns, 55 K blocks as 28 + 27
     (300, 16384, 7168),  # a last row of tiles with 44 rows: waves without any

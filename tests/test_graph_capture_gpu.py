@@ -98,10 +98,11 @@ def test_moe_under_graph_replay_with_changing_routing():
     replay_and_compare(build, refill, run)
 
 
-def test_moe_with_many_rows_per_expert_under_graph_replay():
+@pytest.mark.parametrize("tokens,dim,inter,experts,topk", [(400, 7168, 256, 4, 2), (1300, 1024, 256, 16, 8)])
+def test_moe_with_many_rows_per_expert_under_graph_replay(tokens, dim, inter, experts, topk):
     # 200 rows per expert: pairs of blocks (the first GEMM's LDS ring, 128 KiB of dynamic LDS), the second GEMM
-    # by rows (16-bit rows through LDS) and the separate per-token sum, with the routing redrawn per replay
-    tokens, dim, inter, experts, topk = 400, 7168, 256, 4, 2
+    # by rows (16-bit rows through LDS) and the separate per-token sum, with the routing redrawn per replay;
+    # 650 rows of 16 experts: the same layer in 128-row tiles
     g = torch.Generator(device=DEV).manual_seed(6)
     w1 = (torch.randn(experts * 2 * inter, dim, generator=g, device=DEV) * 0.1).bfloat16()
     w2 = (torch.randn(experts * dim, inter, generator=g, device=DEV) * 0.1).bfloat16()

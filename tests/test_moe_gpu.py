@@ -516,6 +516,23 @@ def test_fmoe_tiles_skip_blocks_of_experts_that_are_not_held(block):
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
 
 
+@pytest.mark.parametrize("tokens,dim,inter,experts,topk", [
+    (9000, 3584, 128, 8, 4),   # some 285 tiles: one item each of the first GEMM, two of the second, one K block
+    (4300, 7168, 256, 7, 4),   # two K blocks: 280 items and 560
+    (3000, 1024, 384, 6, 4),   # the ring for three K blocks: 300 items, then 400
+    (1200, 2048, 1024, 5, 4),  # for eight: 320 and 320
+    (1000, 2048, 1024, 5, 4),  # the same with rows in fp32: 270 and 270
+])
+def test_fmoe_tiles_with_more_items_than_workgroups(tokens, dim, inter, experts, topk):
+    # a workgroup's second item: its slabs land where the first one's results were.  256 workgroups, 512 of the second GEMM
+    # for one and two K blocks; the last tile of an expert is ragged
+    p = make_moe(tokens, dim, inter, experts, topk, seed=tokens)
+    want = run_moe(p, bf16_input=True, kernel_name="tiles=0,down=rows")
+    for _ in range(2):
+        got = run_moe(p, bf16_input=True, kernel_name="tiles=1")
+        assert torch.equal(want.view(torch.int16), got.view(torch.int16))
+
+
 def test_fmoe_tiles_leave_few_tokens_to_the_column_kernel():
     # 500 tokens, top-16: rows and items enough for tiles, but the column kernel's tables still fit: it sums in fp32
     p = make_moe(500, 512, 128, 64, 16, seed=5)
@@ -596,6 +613,17 @@ def test_fused_moe_on_both_sides_of_writing_its_result(tokens):
     aiter_amd.fmoe_fp8_blockscale_g1u1(out, p["x"], w1, w2, s_ids, s_w, s_e, nv, 2, None, p["w1s"], p["w2s"])
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int16), out.view(torch.int16))
+
+
+@pytest.mark.parametrize("tokens", [2047, 2048, 2300])
+def test_fused_moe_in_tiles_on_both_sides_of_writing_its_result(tokens):
+    # 16 experts, top-8: a thousand rows each.  Rows in fp32 up to 2048 tokens, in bf16 beyond
+    p = make_moe(tokens, 512, 512, 16, 8, seed=tokens)
+    w1 = aiter_amd.shuffle_weight(p["w1q"].view(torch.uint8)).view(dtypes.fp8)
+    w2 = aiter_amd.shuffle_weight(p["w2q"].view(torch.uint8)).view(dtypes.fp8)
+    got = aiter_amd.fused_moe(p["x"], w1, w2, p["tw"].to(DEV), p["ti"].to(DEV), w1_scale=p["w1s"], w2_scale=p["w2s"])
+    want = run_moe(p, bf16_input=True, kernel_name="tiles=0,down=rows")
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
 @pytest.mark.parametrize("tokens", [2047, 2048, 2300])
