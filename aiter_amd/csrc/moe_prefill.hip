@@ -40,7 +40,7 @@ struct PrefillParams
     float*         hs;     // and their scales [slots][hs_stride]
     void*          y;      // down: rows [slots][N], bf16 or fp32
     int64_t        lda;
-    int32_t        M, K, N, inter, kblocks, slots, xs_stride, hs_stride;
+    int32_t        M, K, N, inter, kblocks, xs_stride, hs_stride;
     int32_t        col_splits; // down from registers: parts a tile's columns are cut into
 };
 
@@ -612,7 +612,6 @@ hipError_t launch_moe_prefill_gemms(const MoeArgs& a, hipStream_t stream, void* 
     g.N          = 2 * a.inter;
     g.inter      = a.inter;
     g.kblocks    = a.dim / 128;
-    g.slots      = a.max_padded;
     auto gate_up = a.activation == 0 ? moe_prefill_gate_up_kernel<0> : moe_prefill_gate_up_kernel<1>;
     if((e = raise_lds((const void*)gate_up, kGateUpLds, a.device_id, ready[a.activation == 0 ? 0 : 1])) != hipSuccess)
         return e;
