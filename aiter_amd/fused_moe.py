@@ -173,7 +173,7 @@ def fused_moe(hidden_states, w1, w2, topk_weight, topk_ids, expert_mask=None, ac
         dtype = hidden_states.dtype if hidden_states.dtype in (torch.bfloat16, torch.float16) else torch.bfloat16
     num_experts = E if expert_mask is None else expert_mask.numel()
     # The result is ours to allocate: with many tokens the layer's last kernel writes it, instead of adding onto
-    # a buffer that the sort had to clear (the layer on 8192 / 2048 tokens: 1010 -> 955, 488 -> 475 us).  With few,
+    # a buffer that the sort had to clear (the layer on 8192 / 2048 tokens: 1081 -> 1038, 528 -> 517 us).  With few,
     # clearing it beside the sort costs nothing.
     write_out = tokens >= 2048 and expert_mask is None
     sorted_ids, sorted_weights, sorted_expert_ids, num_valid_ids, out = moe_sorting(

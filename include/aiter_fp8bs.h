@@ -304,8 +304,10 @@ int moe_sorting_fwd(aiter_tensor_t* topk_ids, aiter_tensor_t* topk_weights, aite
  *   (the sizes the reference has kernels for: hsa/gfx950/fmoe/silu/fmoe_bf16_blockscaleFp8_g1u1_silu.csv,
  *   column subGU_m) or 128;
  *   fc2_smooth_scale must be NULL; kernel_name names the reference's tuned kernels and is only a
- *   tuning hint here ("nt=1|2|4", "dw=2|4|8", "dc=2|4|8", "down=rows", "down=cols"; "out=write"
- *   stores the sums whatever out held; anything else: choose).
+ *   tuning hint here ("nt=1|2|4", "dw=2|4|8", "dc=2|4|8", "down=rows", "down=cols", "pair=0|1", "tail=0",
+ *   "stage=0", "ring=0", "tiles=0|1"; "out=write" stores the sums whatever out held; several joined by
+ *   commas; anything else: choose).  No hint changes a result but the second GEMM's ("down=cols" sums in
+ *   sorted order).
  * The product of the first GEMM is quantised 1x128 to fp8 for the second.  Each token's k
  * contributions are added in a fixed order (sorted order while the per-token tables of the second GEMM fit
  * the LDS, about 280 tokens at inter = 256; slot order beyond):
