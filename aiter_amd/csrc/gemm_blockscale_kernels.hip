@@ -14,6 +14,7 @@
 #include "fp8bs_launch.h"
 #include "gemm_common.h"
 #include <cstdio>
+#include <cstdlib>
 
 #include <string.h>
 
@@ -179,18 +180,22 @@ const char* gemm_kernel_names() { return kKernelNames; }
 // the compute units and up to 2.1 us when they cover all of them, against 0.8 us for a quarter of
 // the area: it wins once its tiles cover about half of the chip.  Near a tie it is preferred: it
 // gains more when the weights are still in the last-level cache.
+// That decides the K ranges, and with them the bits.  Where it means one range, one round of the 256 x 128 tiles of
+// gemm_ring.hip takes the place of mid_* tilings that are modelled no faster: the same sums (425 x 8896 x 2816: 31 us there, 20
+// here; 5712 x 704 x 3584: 37 and 23).
 static const char* automatic_choice(const GemmKernelParams& p)
 {
-    const float prefill_us = gemm_prefill_plan(p, 256).us; // fitted on a 256-CU part, like the mid model
+    const PrefillPlan plan = gemm_prefill_plan(p, 256); // fitted on a 256-CU part, like the mid model
     if(p.M <= 64 && gemm_decode_supports(p) && (!gemm_mid_supports(p) || gemm_mid_estimate_us(p) >= gemm_decode_estimate_us(p)))
         return "decode_stream";
-    if(gemm_mid_supports(p) && (!gemm_prefill_supports(p) || gemm_mid_estimate_us(p) * 1.03f < prefill_us))
-        return "mid_auto";
-    if(gemm_prefill_supports(p))
+    if(gemm_mid_supports(p) && (!gemm_prefill_supports(p) || gemm_mid_estimate_us(p) * 1.03f < plan.us_apart))
     {
-        const int bn = gemm_prefill_plan(p, 256).tile_n;
-        return bn == 128 ? "prefill_256x128" : bn == 192 ? "prefill_256x192" : "prefill_256x256";
+        if(gemm_prefill_supports(p) && gemm_mid_ranges(p) == 1 && gemm_ring_estimate_us(p, 256) <= gemm_mid_estimate_us(p) * 1.03f)
+            return "prefill_256x128";
+        return "mid_auto";
     }
+    if(gemm_prefill_supports(p))
+        return plan.tile_n == 128 ? "prefill_256x128" : plan.tile_n == 192 ? "prefill_256x192" : "prefill_256x256";
     return "tile_128x128";
 }
 
@@ -323,9 +328,10 @@ static hipError_t dispatch(const GemmArgs& a, const GemmKernelParams& p, hipStre
             return hipErrorInvalidValue;
         }
         // by name it keeps every tile in one workgroup (bitwise the result of the tile_* kernels)
-        // unless ":s=" pins the K ranges per tile; chosen automatically, the launcher decides.
+        // unless ":s=" pins the K ranges per tile; chosen automatically, the launcher decides -- but for
+        // 256 x 128 tiles, which may stand for a plan of another family.
         // splitK is a hint this kernel has no use for.
-        return launch_gemm_prefill(p, DT, ctx, k.splits > 0 ? k.splits : (named ? 1 : 0), named ? k.tile : 0);
+        return launch_gemm_prefill(p, DT, ctx, k.splits > 0 ? k.splits : (named ? 1 : 0), named || k.tile == 128 ? k.tile : 0);
     }
     *why = kUnknownName;
     return hipErrorInvalidValue;
@@ -368,10 +374,14 @@ void gemm_describe_choice(int64_t M, int64_t N, int64_t K, bool shuffled, char* 
     const char* name = automatic_choice(p);
     if(strcmp(name, "mid_auto") == 0)
         gemm_mid_describe(p, buf, n);
-    else if(strncmp(name, "prefill_", 8) == 0 && gemm_prefill_plan(p, 256).splits > 1)
-        snprintf(buf, n, "%s:s=%d", name, gemm_prefill_plan(p, 256).splits); // as on a 256-CU part
     else
-        snprintf(buf, n, "%s", name);
+    {
+        const PrefillPlan plan = gemm_prefill_plan(p, 256); // as on a 256-CU part
+        if(strncmp(name, "prefill_256x", 12) == 0 && atoi(name + 12) == plan.tile_n && plan.splits > 1)
+            snprintf(buf, n, "%s:s=%d", name, plan.splits);
+        else
+            snprintf(buf, n, "%s", name);
+    }
 }
 
 // "<kernel>;splitK=<n>": what the pair (kernelName, splitK) of a call resolves to for contiguous

@@ -89,8 +89,10 @@ struct PrefillPlan
     int   splits;
     float us;
     int   tile_n; // 256, 192 or 128 columns per tile
-    bool  ring;   // two K ranges, one after the other on gemm_ring.hip's tiles
+    bool  ring;   // carried out by gemm_ring.hip's tiles, two K ranges one after the other
+    float us_apart; // what the kernels with a workgroup per range would take
 };
+float gemm_ring_estimate_us(const GemmKernelParams& p, int cus); // one round, K in one range; huge beyond
 PrefillPlan gemm_prefill_plan(const GemmKernelParams& p, int cus);
 // want_splits: K ranges per tile; 0 lets the launcher choose, 1 keeps a tile in one workgroup.
 // want_tile_n: 256, 192 or 128 columns per tile; 0 lets the launcher choose (together with the K ranges).
@@ -108,4 +110,5 @@ bool       gemm_mid_supports(const GemmKernelParams& p);
 // modelled duration (us) of the best mid_* tiling, for the choice between kernel families
 void       gemm_mid_describe(const GemmKernelParams& g, char* buf, size_t n);
 float      gemm_mid_estimate_us(const GemmKernelParams& p);
+int        gemm_mid_ranges(const GemmKernelParams& p); // K ranges of the plan that the estimate is of
 } // namespace fp8bs

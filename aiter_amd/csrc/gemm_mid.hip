@@ -653,6 +653,7 @@ static MidPlan best_plan(const GemmKernelParams& g, int tile, size_t partial_cap
 }
 
 float gemm_mid_estimate_us(const GemmKernelParams& g) { return best_plan(g, 0).cost; }
+int   gemm_mid_ranges(const GemmKernelParams& g) { return best_plan(g, 0).splits; }
 
 // split_k_log2 < 0: choose.  tile: 0 = choose, else 128 (128x128), 64128 (64x128) or 64 (64x64).
 // splits > 0 pins the number of K ranges (any count, not only powers of two).

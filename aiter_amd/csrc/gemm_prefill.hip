@@ -569,16 +569,9 @@ bool gemm_prefill_supports(const GemmKernelParams& p)
 // 144 workgroups: 100 us; 1536 x 7168 x 2048, 168 workgroups: 36 us).  K
 // ranges over s workgroups per tile cost 4 us plus the parked tiles' traffic, (2 s - 1) x 256 KiB
 // per tile at about 5 TB/s (2048 x 4096 x 7168: 89.8 us as one range, 77-80 us as two).
-// 256 x 128 tiles are gemm_ring.hip's: 7 us and, per K block, 0.7 us with few workgroups, 0.9 us with one on every compute unit
-// (modelled / measured: 2048 x 4096 x 7168 57 / 58, 3001 x 2112 x 7168 55 / 55, 1500 x 4096 x 7168 55 / 52, 3001 x 2112 x 2048
-// 21 / 19, 2048 x 3072 x 1536 17 / 17, 1024 x 2112 x 7168 49 / 45).  One round only.
-static float ring_cost(const GemmKernelParams& p, int cus, int tiles128)
-{
-    return 7.f + (float)p.kblocks * (0.7f + 0.2f * (float)tiles128 / (float)cus);
-}
-// ... and a parked first range (modelled / measured: 2048 x 4096 x 7168 63 / 63, 3001 x 2112 x 7168 61 / 53, 300 x 16384 x
-// 7168 54 / 55, 700 x 7168 x 7168 60 / 49, 256 x 24576 x 7168 61 / 72)
-constexpr float kRingFold = 6.f;
+// 256 x 128 tiles, a workgroup per range and two stages: 6 us per round and 1.2 us per K block, rising to 1.4 us when the
+// workgroups of a round cover all compute units (1024 x 7168 x 2048: 26.4 us, 256 x 24576 x 1536: 22.5, 2048 x 4096 x 7168: 84.0).
+constexpr float kFixed128 = 6.f, kIter128 = 1.2f;
 
 static float plan_cost(const GemmKernelParams& p, int cus, int bn, int s)
 {
@@ -587,6 +580,8 @@ static float plan_cost(const GemmKernelParams& p, int cus, int bn, int s)
     const int   rounds = (items + cus - 1) / cus;
     const float share  = (float)items / (float)(rounds * cus);
     const int   kb     = (p.kblocks + s - 1) / s;
+    if(bn == 128)
+        return (float)rounds * (kFixed128 + (float)kb * (kIter128 + (share > 0.44f ? (share - 0.44f) * 0.35f : 0.f)));
     if(bn == 192) // 56 KiB and 24 MFMA slots per K block: 1.4 us (4096 x 2112 x 7168, 176 workgroups: 86.9 us;
                   // 2048 x 2112 x 7168 as 88 tiles x 2 K ranges: 60.3 us against 73.1 with the wide tile),
                   // 1.5 us with a workgroup on every compute unit (8192 x 1536 x 7168, 256 tiles: 93 us)
@@ -597,11 +592,28 @@ static float plan_cost(const GemmKernelParams& p, int cus, int bn, int s)
            (s > 1 ? 4.f + (float)tiles * (float)(2 * s - 1) * 0.05f : 0.f);
 }
 
+// One round of gemm_ring.hip's 256 x 128 tiles, K in one range: 7 us and, per K block, 0.7 us with few workgroups, 0.9 us with
+// one on every compute unit (modelled / measured: 2048 x 4096 x 7168 57 / 58, 3001 x 2112 x 7168 55 / 55, 1500 x 4096 x 7168
+// 55 / 52, 3001 x 2112 x 2048 21 / 19, 2048 x 3072 x 1536 17 / 17, 1024 x 2112 x 7168 49 / 45).
+float gemm_ring_estimate_us(const GemmKernelParams& p, int cus)
+{
+    const int tiles = ((p.M + kBM - 1) / kBM) * ((p.N + 127) / 128);
+    return tiles > cus ? 1e30f : 7.f + (float)p.kblocks * (0.7f + 0.2f * (float)tiles / (float)cus);
+}
+// ... and a parked first range (modelled / measured: 2048 x 4096 x 7168 63 / 63, 3001 x 2112 x 7168 61 / 53, 300 x 16384 x
+// 7168 54 / 55, 700 x 7168 x 7168 60 / 49, 256 x 24576 x 7168 61 / 72)
+constexpr float kRingFold = 6.f;
+
+// The tile and the K ranges are those of the kernels that take a workgroup per range: a call's sums, and with them its bits,
+// follow from that choice alone.  The ring's tiles then carry the plan out where they are faster.  They do not change the
+// ranges: two stay two, one after the other in a workgroup (us in the kernel with a workgroup per range / on the ring: 2048 x
+// 4096 x 7168 75 / 63, 2048 x 2304 x 7168 50 / 44, 700 x 7168 x 7168 58 / 49).  In one range they take 4-5 us less, with an
+// error against 64 bits that is the same to seven digits.
 PrefillPlan gemm_prefill_plan(const GemmKernelParams& p, int cus)
 {
     const int tiles = ((p.M + kBM - 1) / kBM) * ((p.N + 255) / 256);
     cus             = std::max(cus, 1);
-    PrefillPlan best{1, plan_cost(p, cus, 256, 1), 256, false};
+    PrefillPlan best{1, plan_cost(p, cus, 256, 1), 256, false, 0.f};
     for(int s = 2; s <= 3; ++s)
     {
         // (below 64 tiles the model is off: 1024 x 2112 x 7168, 36 tiles x 3, takes 67 us where it
@@ -610,7 +622,14 @@ PrefillPlan gemm_prefill_plan(const GemmKernelParams& p, int cus)
             break;
         const float c = plan_cost(p, cus, 256, s);
         if(c < best.us * 0.97f)
-            best = PrefillPlan{s, c, 256, false};
+            best = PrefillPlan{s, c, 256, false, 0.f};
+    }
+    // half-width tiles where the wide ones leave at least half of the compute units without a workgroup
+    if(tiles * 2 <= cus)
+    {
+        const float c = plan_cost(p, cus, 128, 1);
+        if(c < best.us * 0.97f)
+            best = PrefillPlan{1, c, 128, false, 0.f};
     }
     // 192-wide tiles: no ragged last column where they divide N and 256 does not (N = 2112: a
     // ninth column of tiles that is three quarters empty against eleven full ones), and often a better
@@ -627,21 +646,17 @@ PrefillPlan gemm_prefill_plan(const GemmKernelParams& p, int cus)
                 break;
             const float c = plan_cost(p, cus, 192, s);
             if(c < best.us * 0.97f)
-                best = PrefillPlan{s, c, 192, false};
+                best = PrefillPlan{s, c, 192, false, 0.f};
         }
     }
-    // One round of 256 x 128 tiles.  They carry a plan out, they do not change its sums: two K ranges stay two, one after the
-    // other in a workgroup (us in the kernel with a workgroup per range / here: 2048 x 4096 x 7168 75 / 63, 2048 x 2304 x 7168
-    // 50 / 44, 700 x 7168 x 7168 58 / 49).  In one range they take 4-5 us less, with an error against 64 bits that is the same to
-    // seven digits; but a call's K ranges, and the bits that follow, are what the library says they are.
-    const int t128 = ((p.M + kBM - 1) / kBM) * ((p.N + 127) / 128);
-    if(t128 <= cus)
+    best.us_apart = best.us;
+    const float c = gemm_ring_estimate_us(p, cus) + (best.splits == 2 ? kRingFold : 0.f);
+    if(best.splits <= 2 && (c < best.us * 0.97f || best.tile_n == 128)) // (256 x 128 tiles in one range are the ring's in any case)
     {
-        const float c = ring_cost(p, cus, t128) + (best.splits == 2 ? kRingFold : 0.f);
-        if(best.splits == 1 && c < best.us * 0.97f)
-            best = PrefillPlan{1, c, 128, false};
-        else if(best.splits == 2 && c < best.us * 0.97f)
-            best = PrefillPlan{2, c, best.tile_n, true};
+        best.us   = c;
+        best.ring = true;
+        if(best.splits == 1)
+            best.tile_n = 128;
     }
     return best;
 }

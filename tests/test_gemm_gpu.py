@@ -543,6 +543,31 @@ def test_prefill_kernel_k_ranges_across_workgroups(m, n, k, name):
 
 
 @pytest.mark.parametrize("m,n,k", [
+    (145, 19968, 4992),  # where the plan of wide tiles would be two ranges
+    (293, 12096, 7168),
+    (5712, 704, 3584),
+    (1631, 2496, 2432),
+])
+@pytest.mark.parametrize("layout", ["plain", "preshuffled"])
+def test_256x128_tiles_in_place_of_mid_tilings(m, n, k, layout):
+    # one range of K, chosen by its time on the mid_* tilings and carried out on 256 x 128 tiles: their bits, and what is reported
+    assert _ffi.gemm_choice(m, n, k, layout == "preshuffled") == "prefill_256x128"
+    xq, wq, xs, ws = _gpu_problem(m, n, k, seed=m + n + k, outliers=True)
+    outs = [torch.full((m, n), float("nan"), dtype=torch.float16, device=DEV) for _ in range(3)]
+    if layout == "preshuffled":
+        xs = xs.t().contiguous().t()
+        wq = aiter_amd.shuffle_weight(wq.view(torch.uint8)).view(wq.dtype)
+    for out, name in zip(outs, ("", "prefill_256x128", "mid_64x128:s=1")):
+        if layout == "preshuffled":
+            aiter_amd.gemm_a8w8_blockscale_bpreshuffle_ck(xq, wq, xs, ws, out, name)
+        else:
+            aiter_amd.gemm_a8w8_blockscale_ck(xq, wq, xs, ws, out, splitK=-1, kernelName=name)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    assert torch.equal(outs[0].view(torch.int16), outs[2].view(torch.int16))
+
+
+@pytest.mark.parametrize("m,n,k", [
     (2100, 5000, 1024),  # 360 tiles of 256 x 128, the last ones ragged; x_scale four K blocks per load
     (2560, 8192, 640),   # 640 tiles, up to three per workgroup; x_scale K block by K block
 ])
