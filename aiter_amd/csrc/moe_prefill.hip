@@ -536,7 +536,7 @@ bool moe_prefill_wanted(const MoeArgs& a)
         return false;
     const int64_t pairs = (int64_t)a.M * a.topk;
     const int64_t all   = routed_experts(pairs, a.topk, a.block_rows << a.expert_shift, a.max_padded, a.experts);
-    return tiles_win(pairs, all, a.experts, a.inter, moe_rows_in_f32(a));
+    return tiles_win(pairs, all, a.experts, a.inter);
 }
 
 size_t moe_prefill_workspace_bytes(const MoeArgs& a)

@@ -18,31 +18,30 @@ inline int64_t routed_experts(int64_t pairs, int topk, int unit, int64_t padded,
 }
 
 // Tiles win where an expert has enough rows that the block-wise kernels' repeated passes over its weights cost more than a
-// tile's padding, and where there are enough items (a tile's 128 columns of the product; an expert's last tile is half full
-// on average) for the chip.  Fewer rows do with many items, whose last round of workgroups matters less (unless the rows are
-// kept in fp32), and with a longer K of the second GEMM.  Measured on both sides, us block by block / in tiles (experts,
-// topk, dim, inter):
-//   (256, 8, 7168, 256)  rows per expert 48 (448 items): 468 / 490, 52: 494 / 479, 64: 553 / 515, 256: 1724 / 1044
+// tile's padding -- fewer with a longer K of the second GEMM, where those kernels have nothing in flight while they multiply --
+// and where there are enough items (a tile's 128 columns of the product; an expert's last tile is half full on average) for
+// the chip.  Over 1139 drawn layers (5 to 256 experts, 8 to 1200 rows each, dim 1024 to 7168) this takes 0.5 % longer than
+// the better of the two on average, 5 % and more in 43 and 23 % at worst.  us block by block / in tiles (experts, topk, dim,
+// inter):
+//   (256, 8, 3072, 128)  64 rows per expert (256 items): 181 / 198, 80 (288): 215 / 206, 128: 299 / 236
+//   (256, 8, 7168, 256)  48 (448): 468 / 490, 52: 494 / 479, 64: 553 / 515, 256: 1724 / 1044
 //   (128, 8, 7168, 256)  64 (256): 294 / 319, 80 (288): 342 / 341, 96: 385 / 343
-//   (256, 8, 3072, 128)  64 (256): 181 / 198, 80 (288): 215 / 206, 128: 299 / 236
 //   (32, 5, 4096, 256)   96 (80): 92 / 106, 112 (88): 109 / 108, 160: 137 / 113
-//   (8, 2, 1024, 256)    640 (88, fp32 rows): 72 / 75, 768 (104): 79 / 75, 1024: 88 / 77
+//   (8, 2, 1024, 256)    640 (88): 72 / 75, 768 (104): 79 / 75, 1024: 88 / 77
 //   (128, 8, 4096, 384)  48 (336): 208 / 214, 56 (360): 231 / 212, 128: 392 / 291
 //   (256, 8, 2048, 512)  32 (768): 241 / 254, 40 (832): 273 / 255, 256: 1055 / 609
 //   (64, 6, 7168, 512)   48 (224): 238 / 275, 64 (256): 283 / 291, 80: 328 / 296
-//   (32, 8, 7168, 1024)  32 (192, fp32 rows): 183 / 198, 48 (224): 207 / 192, 128: 414 / 291
-//   (64, 6, 2048, 1024)  40 (416, fp32 rows): 150 / 158, 48 (448): 162 / 158, 64: 204 / 174
-//   (16, 4, 4096, 2048)  32 (192, fp32 rows): 121 / 112, 128: 284 / 180
+//   (32, 8, 7168, 1024)  32 (192): 183 / 198, 48 (224): 207 / 192, 128: 414 / 291
+//   (16, 4, 4096, 2048)  32 (192): 121 / 112, 128: 284 / 180
 //   (32 held of 256, 8, 7168, 2048)  2: 245 / 273, 16 (320): 293 / 299, 32 (384): 396 / 319, 256: 1635 / 815
 //   (64 held of 256, 8, 4096, 1024)  16: 187 / 219, 32 (384): 226 / 229, 64: 337 / 252
 // `all`: the experts that the pairs are spread over, as routed_experts says.
-inline bool tiles_win(int64_t pairs, int64_t all, int experts, int inter, bool rows_f32)
+inline bool tiles_win(int64_t pairs, int64_t all, int experts, int inter)
 {
     const double rows  = (double)pairs / (double)all;
-    const double items = (rows * experts / kTileRowsOfExpert + 0.5 * experts) * (inter / 128);
-    const bool   many  = items >= 400.0 && !rows_f32;
-    const double least = inter > 1024 ? 32.0 : many ? (inter > 256 ? 40.0 : 52.0) : inter > 512 ? 48.0 : inter > 256 ? 56.0 : 80.0;
-    return rows >= least && items >= 92.0;
+    const double items = (rows / kTileRowsOfExpert + 0.5) * experts * (inter / 128);
+    const double least = inter <= 128 ? 80.0 : inter <= 256 ? 64.0 : inter <= 512 ? 40.0 : inter <= 1024 ? 28.0 : 24.0;
+    return rows >= least && items >= 80.0;
 }
 
 } // namespace fp8bs

@@ -37,15 +37,15 @@ int main()
                         // a rank that holds a part of the experts sees the rows per expert of the whole: no more tiles than
                         // with all of them, whatever its own part
                         for(int inter : {128, 256, 512, 2048})
-                            if(tiles_win(pairs, all, e, inter, false))
-                                EXPECT(tiles_win(pairs, all, all, inter, false));
+                            if(tiles_win(pairs, all, e, inter))
+                                EXPECT(tiles_win(pairs, all, all, inter));
                     }
     // 32 of 256 experts held: a decode batch of 64 tokens has two rows per expert, not sixteen
     e = 32;
     for(m = 1; m <= 512; ++m)
-        EXPECT(!tiles_win((int64_t)m * 8, routed_experts((int64_t)m * 8, 8, 32, padded((int64_t)m * 8, 8, 32, 256), e), e, 2048, m < 147));
+        EXPECT(!tiles_win((int64_t)m * 8, routed_experts((int64_t)m * 8, 8, 32, padded((int64_t)m * 8, 8, 32, 256), e), e, 2048));
     m = 8192;
-    EXPECT(tiles_win((int64_t)m * 8, 256, e, 256, false) && tiles_win((int64_t)m * 8, 256, 256, 256, false));
+    EXPECT(tiles_win((int64_t)m * 8, 256, e, 256) && tiles_win((int64_t)m * 8, 256, 256, 256));
     std::printf("OK\n");
     return 0;
 }
