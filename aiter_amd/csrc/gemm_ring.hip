@@ -1,7 +1,8 @@
 // Block-scale FP8 GEMM on 256 x 128 tiles: the three-stage ring of gemm_ring.h, four waves that fetch, eight that multiply.
 //
-// Runs the 256 x 128 plans of gemm_prefill.hip, and those of its plans with two K ranges per 256-wide tile whose 256 x 128
-// halves fill at most one round of workgroups; the additions are the plan's, so the bits are too.
+// Carries out, where it is faster and 256 x 128 tiles fill at most one round of workgroups, what was chosen for other
+// kernels: plans of gemm_prefill.hip with one or two K ranges, and mid_* tilings with one; the additions are the plan's, so the
+// bits are too.
 //
 // Bound by what a compute unit takes in: 48 KiB per K block, 0.75 us with few workgroups, 0.9 us with 256 (13 TB/s out of L2
 // over the chip; the matrix pipes need 0.45).  The two-stage tiles of gemm_prefill.hip wait for each K block's loads
