@@ -1,6 +1,5 @@
-// The multiply loop shared by the kernels whose workgroup tile is 256 x 128 or 128 x 128: eight waves multiply, with a
-// 64 (n) x 64 (m) or 32 x 64 block of the tile each; four more bring both operand slabs in by direct global->LDS loads, into
-// a ring of three or four stages.
+// The multiply loop shared by the kernels whose workgroup tile is 256 x 128: eight waves multiply, with a 64 (n) x 64 (m) block
+// of the tile each; four more bring both operand slabs in by direct global->LDS loads, into a ring of three stages.
 //
 // Why waves that only fetch.  A wave that issues a load is held at the issue while the memory pipeline's queue is full
 // (48 KiB are 768 cycles of it per K block), and with it the MFMAs behind: with the loads dealt out over the multiplying
@@ -9,10 +8,10 @@
 // Why three stages of a 256 x 128 tile.  A K block of it is 1024 matrix cycles per SIMD, 0.45-0.55 us; a slab load takes
 // 1-2 us from the last-level cache or HBM while every compute unit asks.  With two stages the loads of K block kb + 1 have
 // one K block of time to arrive and set the pace; with three they have two.  A stage is 48 KiB, so a tile of this
-// size is the largest for which three fit the 160 KiB.  128 x 128 tiles have stages of 32 KiB, and four of them.
+// size is the largest for which three fit the 160 KiB.
 //
-// Bound by, per K block of a compute unit: 48 (32) KiB taken in, 128 (96) KiB of fragments out of LDS (1024 cycles at 128
-// bytes a cycle, beside 384 for what the loads write), 128 (64) MFMAs (1024 cycles per SIMD).
+// Bound by, per K block of a compute unit: 48 KiB taken in, 128 KiB of fragments out of LDS (1024 cycles at 128
+// bytes a cycle, beside 384 for what the loads write), 128 MFMAs (1024 cycles per SIMD).
 #pragma once
 
 #include "gemm_common.h"
@@ -26,14 +25,13 @@ typedef const volatile float __attribute__((address_space(3)))* lds_f32_ptr;
 constexpr int kRingMulWaves = 8, kRingFetchWaves = 4;
 constexpr int kRingMulThreads = 64 * kRingMulWaves, kRingThreads = 64 * (kRingMulWaves + kRingFetchWaves);
 
-// WN: waves along n (2 or 4).  NF: weight fragments per multiplying wave (4 activation fragments in any case); the tile is
-// 16 NF WN (n) x 64 (8 / WN) (m).  NF = 2 leaves a wave the registers for a second set of sums, and the LDS a fourth stage.
-template <int WN, int NF = 4>
+// WN: waves along n (2 or 4); the tile is 64 WN (n) x 64 (8 / WN) (m).
+template <int WN>
 struct RingTile
 {
-    static constexpr int kWN = WN, kFrags = NF, kStages = NF == 2 ? 4 : 3;
-    static constexpr int kWM = 8 / WN, kBN = WN * 16 * NF, kBM = kWM * 64;
-    static constexpr int kSlabBytes  = (kBM + kBN) * 128;       // weight rows, then activation rows: 48 KiB (32 for 128 x 128)
+    static constexpr int kWN = WN, kFrags = 4, kStages = 3; // fragments of 16 weight rows per multiplying wave
+    static constexpr int kWM = 8 / WN, kBN = WN * 64, kBM = kWM * 64;
+    static constexpr int kSlabBytes  = (kBM + kBN) * 128;       // weight rows, then activation rows: 48 KiB
     static constexpr int kStageBytes = kSlabBytes + kBM * 4;    // + the K block's x_scale of the tile's rows
     static constexpr int kWindows    = kStages * kStageBytes;   // two windows of four K blocks of x_scale (XS4)
     static constexpr int kWindowBytes = kBM * 16;
@@ -53,33 +51,9 @@ struct RingSource
     uint32_t       goff[T::kLoads];
     uint32_t       xs_goff;                 // fetching waves 0 .. kWM - 1: this lane's row of x_scale
     uint32_t       xs_step;                 // bytes between two K blocks of x_scale (not XS4)
-    const float*   ws_row[2];               // w_scale of weight fragments 0, 1 and of 2, 3 (SG = 2; NF = 2: 0 and 1), [kblocks]
+    const float*   ws_row;                  // w_scale of the tile's columns of this wave, [kblocks]
     int            kblocks;
 };
-
-// The order in which a tile's K blocks pass.  C = 0: ascending.  C > 0: by their remainder modulo C, ascending inside a
-// remainder -- what C waves with every C-th K block each would add up, one wave's share after the other.  x_scale lies in
-// memory in that order, weights and activations do not.
-template <int C>
-__device__ __forceinline__ int ring_kblock(int pos, int kblocks)
-{
-    if constexpr(C == 0)
-        return pos;
-    else
-    {
-        const int q = kblocks / C, longer = (kblocks % C) * (q + 1); // the first kblocks % C remainders have one block more
-        const bool in = pos < longer;
-        const int  n = in ? q + 1 : max(q, 1), at = in ? pos : pos - longer;
-        const int  r = at / n;
-        return (in ? 0 : kblocks % C) + r + C * (at - r * n);
-    }
-}
-// where remainder r starts in that order
-template <int C>
-__device__ __forceinline__ int ring_first_position(int r, int kblocks)
-{
-    return r * (kblocks / C) + min(r, kblocks % C);
-}
 
 // One LDS-direct load: lane l's 16 (4) bytes land at M0 + 16 l (4 l).  From asm: the compiler models the builtin as a
 // flat access that may touch LDS and from then on waits for every outstanding LDS read in full.  The loads are
@@ -106,7 +80,7 @@ __device__ __forceinline__ RingUnit ring_unit(int i, int f, int lane)
     return RingUnit{u, r, ((uint32_t)lane & 7u) ^ lds_swizzle(r)};
 }
 
-// The fetching waves' half of a tile: its K blocks into the ring, in the order that C says.  f: 0 .. 3.
+// The fetching waves' half of a tile: its K blocks into the ring.  f: 0 .. 3.
 //
 // SHUF: weights pre-shuffled (16,16); a 16-row tile's K block is 2 KiB in fragment order and is copied as it lies.
 // XS4: x_scale rows are 16-byte aligned and come four K blocks per load (see gemm_prefill.hip for what that saves).
@@ -114,13 +88,12 @@ __device__ __forceinline__ RingUnit ring_unit(int i, int f, int lane)
 // Both halves pass the same barriers: one when the first K block is in LDS, one per K block, after which the next one is, and
 // the stage just multiplied is free.  At the last one every load has landed and every read is done: the LDS is free.  The
 // caller has a barrier between the last use of the LDS and this call.
-template <class T, bool SHUF, bool XS4, int C = 0>
+template <class T, bool SHUF, bool XS4>
 __device__ __forceinline__ void ring_fetch(lds_byte_ptr smem3, const RingSource<T>& src, int f)
 {
     constexpr int S = T::kStages;
     const bool xs_wave = f < T::kWM; // waves that fetch x_scale, 64 rows each
     const int  n = src.kblocks;
-    int        walk = 0; // C > 0: the K block at the position issued next
     auto issue_slabs = [&](int kb, uint32_t stage) {
         const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(smem3 + stage + f * 1024));
 #pragma unroll
@@ -130,58 +103,42 @@ __device__ __forceinline__ void ring_fetch(lds_byte_ptr smem3, const RingSource<
             ring_dma16(dst + (uint32_t)u * (kRingFetchWaves * 1024u), src.goff[u], (u < T::kWLoads ? src.wq : src.xq) + koff);
         }
     };
-    auto issue_xs = [&](int pos, uint32_t stage) {
+    auto issue_xs = [&](int kb, uint32_t stage) {
         if constexpr(XS4)
-            ring_dma16(__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(smem3 + T::kWindows + ((pos >> 2) & 1) * T::kWindowBytes + f * 1024)),
-                       src.xs_goff + (uint32_t)(pos & ~3) * 4u, src.xs);
+            ring_dma16(__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(smem3 + T::kWindows + ((kb >> 2) & 1) * T::kWindowBytes + f * 1024)),
+                       src.xs_goff + (uint32_t)(kb & ~3) * 4u, src.xs);
         else
             ring_dma4(__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(smem3 + stage + T::kSlabBytes + f * 256)),
-                      src.xs_goff + (uint32_t)pos * src.xs_step, src.xs);
+                      src.xs_goff + (uint32_t)kb * src.xs_step, src.xs);
     };
-    // The K block at position `pos` into `stage`; past the end the last block again, unused, so that every stage has its
-    // loads.  x_scale comes with each of them, or (XS4) with the one that opens a window of four.  `young` has a bit per
-    // stage, the youngest lowest: whether this wave's loads of it include one of x_scale.
-    uint32_t young = 0;
-    auto issue = [&](int pos, uint32_t stage) {
-        const int at = min(pos, n - 1);
-        issue_slabs(C == 0 ? at : walk, stage);
-        const bool xs = xs_wave && (!XS4 || ((at & 3) == 0 && at == pos));
-        if(xs)
+    // K block kb into `stage`; past the end the last block again, unused, so that every stage has its loads.  x_scale comes
+    // with each of them, or (XS4) with the one that opens a window of four.
+    bool with_xs = false; // whether this wave's loads of the youngest stage include one of x_scale
+    auto issue = [&](int kb, uint32_t stage) {
+        const int at = min(kb, n - 1);
+        issue_slabs(at, stage);
+        with_xs = xs_wave && (!XS4 || ((at & 3) == 0 && at == kb));
+        if(with_xs)
             issue_xs(at, stage);
-        young = young << 1 | (xs ? 1u : 0u);
-        if constexpr(C > 0)
-            if(pos + 1 < n)
-                walk = walk + C < n ? walk + C : walk % C + 1; // past the end: the next remainder
     };
-    // all but the S - 2 youngest stages' loads of this wave have landed
-    auto wait_but_youngest = [&] {
-        static_assert(T::kLoads * (S - 2) == 12 || T::kLoads * (S - 2) == 16, "the waits count the loads of S - 2 stages");
-        const int xs = __builtin_popcount(young & ((1u << (S - 2)) - 1u));
-        if constexpr(T::kLoads * (S - 2) == 12)
-        {
-            if(xs)
-                asm volatile("s_waitcnt vmcnt(13)" ::: "memory");
-            else
-                asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
-        }
-        else if(xs == 2)
-            asm volatile("s_waitcnt vmcnt(18)" ::: "memory");
-        else if(xs == 1)
-            asm volatile("s_waitcnt vmcnt(17)" ::: "memory");
+    auto wait_but_youngest = [&] { // all but the youngest stage's loads of this wave have landed
+        static_assert(T::kLoads == 12 && S == 3, "the waits count the loads of a stage");
+        if(with_xs)
+            asm volatile("s_waitcnt vmcnt(13)" ::: "memory");
         else
-            asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+            asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
     };
 #pragma unroll
     for(int s = 0; s < S - 1; ++s)
         issue(s, (uint32_t)s * T::kStageBytes);
     wait_but_youngest();
     __syncthreads();
-    uint32_t stage = (S - 1) * T::kStageBytes; // of position pos + S - 1
-    for(int pos = 0; pos < n; ++pos)
+    uint32_t stage = (S - 1) * T::kStageBytes; // of K block kb + S - 1
+    for(int kb = 0; kb < n; ++kb)
     {
-        issue(pos + S - 1, stage);
+        issue(kb + S - 1, stage);
         stage = stage == (S - 1u) * T::kStageBytes ? 0u : stage + (uint32_t)T::kStageBytes;
-        if(pos + 1 < n)
+        if(kb + 1 < n)
             wait_but_youngest();
         else
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -189,29 +146,27 @@ __device__ __forceinline__ void ring_fetch(lds_byte_ptr smem3, const RingSource<
     }
 }
 
-// w_scale for 64 consecutive positions from pos0 (a multiple of 64) on in one VGPR, lane = position: picked with
+// w_scale for 64 consecutive K blocks from kb0 (a multiple of 64) on in one VGPR, lane = K block: picked with
 // v_readlane, because a scalar load in the loop would share the LGKM counter with the LDS reads
-template <int C>
-__device__ __forceinline__ float ring_ws_window(const float* row, int kblocks, int pos0, int lane)
+__device__ __forceinline__ float ring_ws_window(const float* row, int kblocks, int kb0, int lane)
 {
-    return row[ring_kblock<C>(min(pos0 + lane, kblocks - 1), kblocks)];
+    return row[min(kb0 + lane, kblocks - 1)];
 }
 
 // The multiplying waves' half: acc[i][j] += this wave's share, weight fragment i, activation fragment j.  wave: 0 .. 7.
 //
-// lo, hi: positions in the order of K blocks.  A tile's K blocks may be multiplied in several calls that follow one another
-// (lo > 0 continues where the call before stopped), for sums of their own.
-// SG: w_scale blocks per wave (the first and the second half of the fragments may belong to different 128-row blocks).
-// ws_vec: ring_ws_window of each, of the window that `lo` lies in; handed on from call to call.
+// lo, hi: K blocks.  A tile's K blocks may be multiplied in several calls that follow one another (lo > 0 continues where the
+// call before stopped), for sums of their own.
+// ws_vec: ring_ws_window of the window that `lo` lies in; handed on from call to call.
 // busy: false for a wave whose rows are all padding: it multiplies nothing.
-template <class T, bool SHUF, bool XS4, int SG, int C = 0>
+template <class T, bool SHUF, bool XS4>
 __device__ __forceinline__ void ring_multiply(lds_byte_ptr smem3, const RingSource<T>& src, int wave, int lane, int lo, int hi,
-                                              bool busy, float (&ws_vec)[SG], float (&acc)[T::kFrags][4][4])
+                                              bool busy, float& ws_vec, float (&acc)[T::kFrags][4][4])
 {
     constexpr int NF = T::kFrags, H = NF / 2, D = 4 * H; // fragments H .. NF - 1 are deferred: D tiles
     if(!busy)
     {
-        for(int pos = lo + (lo > 0 ? 1 : 0); pos <= hi; ++pos)
+        for(int kb = lo + (lo > 0 ? 1 : 0); kb <= hi; ++kb)
             __syncthreads();
         return;
     }
@@ -246,9 +201,9 @@ __device__ __forceinline__ void ring_multiply(lds_byte_ptr smem3, const RingSour
         asm volatile("v_fmac_f32 %0, %1, %2" : "+v"((ACC)[3]) : "v"((P)[3]), "v"(S));      \
     } while(0)
 
-    uint32_t stage = (uint32_t)(lo % T::kStages) * T::kStageBytes; // of position pos
+    uint32_t stage = (uint32_t)(lo % T::kStages) * T::kStageBytes; // of K block kb
 
-    // The instruction stream is that of gemm_prefill.hip with NF weight fragments: 4 NF MFMA slots per K block, the FMAs
+    // The instruction stream is that of gemm_prefill.hip with four weight fragments: 4 NF MFMA slots per K block, the FMAs
     // that fold a product into the accumulators two slots behind its MFMA; the tiles of the upper half of the fragments are
     // issued behind the barrier, while the next K block's first fragments travel from LDS.  Where those notes speak of zero
     // fragments for the first K block's predecessor and the wait states ahead of the first MFMA, the same holds here.
@@ -263,12 +218,10 @@ __device__ __forceinline__ void ring_multiply(lds_byte_ptr smem3, const RingSour
 #pragma unroll
     for(int q = 0; q < NF; ++q)
         aw[q] = i32x8{0, 0, 0, 0, 0, 0, 0, 0};
-    float scp[SG][4]; // x_scale * w_scale of the previous K block
+    float scp[4]; // x_scale * w_scale of the previous K block
 #pragma unroll
-    for(int g = 0; g < SG; ++g)
-#pragma unroll
-        for(int j = 0; j < 4; ++j)
-            scp[g][j] = 0.f;
+    for(int j = 0; j < 4; ++j)
+        scp[j] = 0.f;
 #pragma unroll
     for(int q = 0; q < 4; ++q)
         asm volatile("" : "+v"(bx[q]));
@@ -280,36 +233,27 @@ __device__ __forceinline__ void ring_multiply(lds_byte_ptr smem3, const RingSour
     // LDS address of this lane's x_scale for m tile 0; tile j sits 64 (XS4: 256) bytes further
     const uint32_t xs_lds = XS4 ? (uint32_t)T::kWindows + ((uint32_t)wm * 64u + (uint32_t)l16) * 16u
                                 : (uint32_t)T::kSlabBytes + ((uint32_t)wm * 64u + (uint32_t)l16) * 4u;
-    auto xs_window_addr = [&](int pos) -> uint32_t { return (uint32_t)(((pos >> 2) & 1) * T::kWindowBytes + (pos & 3) * 4) + xs_lds; };
+    auto xs_window_addr = [&](int kb) -> uint32_t { return (uint32_t)(((kb >> 2) & 1) * T::kWindowBytes + (kb & 3) * 4) + xs_lds; };
     uint32_t xs_addr = XS4 ? xs_window_addr(lo) : 0u;
 
-    for(int pos = lo; pos < hi; ++pos)
+    for(int kb = lo; kb < hi; ++kb)
     {
-        if((pos & 63) == 0 && pos != 0)
-        {
-#pragma unroll
-            for(int g = 0; g < SG; ++g)
-                ws_vec[g] = ring_ws_window<C>(src.ws_row[g], src.kblocks, pos, lane);
-        }
-        float wsc[SG];
-#pragma unroll
-        for(int g = 0; g < SG; ++g)
-            wsc[g] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ws_vec[g]), pos & 63));
+        if((kb & 63) == 0 && kb != 0)
+            ws_vec = ring_ws_window(src.ws_row, src.kblocks, kb, lane);
+        const float wsc = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ws_vec), kb & 63));
 
         aw[0] = read_w(stage, 0);
-        float sc[SG][4];
+        float sc[4];
 #pragma unroll
         for(int j = 0; j < 4; ++j)
         {
             const float xsv = XS4 ? *(lds_f32_ptr)(smem3 + xs_addr + j * 256) : *(lds_f32_ptr)(smem3 + stage + xs_lds + j * 64);
-#pragma unroll
-            for(int g = 0; g < SG; ++g)
-                sc[g][j] = xsv * wsc[g];
+            sc[j]           = xsv * wsc;
         }
 #pragma unroll
         for(int q = 0; q < 4 * NF; ++q)
         {
-            if(H > 1 && q == 2)
+            if(q == 2)
                 aw[1] = read_w(stage, 1);
             if(q < D) // deferred tile (H + q % H, q / H) of the previous K block
                 FP8BS_MFMA(P[q & 3], aw[H + q % H], bx[q / H]);
@@ -322,22 +266,20 @@ __device__ __forceinline__ void ring_multiply(lds_byte_ptr smem3, const RingSour
                 aw[q - D + NF] = read_w(stage, q - D + NF);
             if(XS4 && q == D)
             {
-                xs_addr = xs_window_addr(pos + 1);
+                xs_addr = xs_window_addr(kb + 1);
                 asm volatile("" : "+v"(xs_addr)); // here, between two slots
             }
             // fold in the product issued two slots ago
             if(q < 2)
-                FP8BS_FMA4(acc[H - 1][2 + q], P[2 + q], scp[0][2 + q]);
+                FP8BS_FMA4(acc[H - 1][2 + q], P[2 + q], scp[2 + q]);
             else if(q < D + 2)
-                FP8BS_FMA4(acc[H + (q - 2) % H][(q - 2) / H], P[(q - 2) & 3], scp[SG - 1][(q - 2) / H]);
+                FP8BS_FMA4(acc[H + (q - 2) % H][(q - 2) / H], P[(q - 2) & 3], scp[(q - 2) / H]);
             else
-                FP8BS_FMA4(acc[(q - 2 - D) >> 2][(q - 2 - D) & 3], P[(q - 2) & 3], sc[0][(q - 2 - D) & 3]);
+                FP8BS_FMA4(acc[(q - 2 - D) >> 2][(q - 2 - D) & 3], P[(q - 2) & 3], sc[(q - 2 - D) & 3]);
         }
 #pragma unroll
-        for(int g = 0; g < SG; ++g)
-#pragma unroll
-            for(int j = 0; j < 4; ++j)
-                scp[g][j] = sc[g][j];
+        for(int j = 0; j < 4; ++j)
+            scp[j] = sc[j];
         stage = stage == (T::kStages - 1u) * T::kStageBytes ? 0u : stage + (uint32_t)T::kStageBytes;
         // (every fragment of this K block is in registers, or on its way there: the barrier waits for outstanding LDS
         // reads) the next one is in LDS behind it
@@ -349,14 +291,14 @@ __device__ __forceinline__ void ring_multiply(lds_byte_ptr smem3, const RingSour
     {
         FP8BS_MFMA(P[q & 3], aw[H + q % H], bx[q / H]);
         if(q < 2)
-            FP8BS_FMA4(acc[H - 1][2 + q], P[2 + q], scp[0][2 + q]);
+            FP8BS_FMA4(acc[H - 1][2 + q], P[2 + q], scp[2 + q]);
         else
-            FP8BS_FMA4(acc[H + (q - 2) % H][(q - 2) / H], P[(q - 2) & 3], scp[SG - 1][(q - 2) / H]);
+            FP8BS_FMA4(acc[H + (q - 2) % H][(q - 2) / H], P[(q - 2) & 3], scp[(q - 2) / H]);
     }
     asm volatile("s_nop 15\n s_nop 15\n s_nop 15" ::: "memory"); // >= 11 wait states after the last MFMA
 #pragma unroll
     for(int q = D; q < D + 2; ++q)
-        FP8BS_FMA4(acc[H + (q - 2) % H][(q - 2) / H], P[(q - 2) & 3], scp[SG - 1][(q - 2) / H]);
+        FP8BS_FMA4(acc[H + (q - 2) % H][(q - 2) / H], P[(q - 2) & 3], scp[(q - 2) / H]);
 #undef FP8BS_MFMA
 #undef FP8BS_FMA4
 }

@@ -83,9 +83,9 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmKernelParam
         }
         float          acc[T::kFrags][4][4];
         const uint32_t nb = min((uint32_t)(n0 + wn * 64) >> 7, (uint32_t)((p.N + 127) / 128 - 1));
-        src.ws_row[0] = src.ws_row[1] = p.ws + (size_t)nb * p.kblocks;
+        src.ws_row = p.ws + (size_t)nb * p.kblocks;
         const bool busy = m0 + wm * 64 < p.M && n0 + wn * 64 < p.N;
-        float      ws_vec[1] = {ring_ws_window<0>(src.ws_row[0], p.kblocks, 0, lane)};
+        float      ws_vec = ring_ws_window(src.ws_row, p.kblocks, 0, lane);
         auto zero = [&] {
 #pragma unroll
             for(int q = 0; q < 16; ++q)
@@ -101,12 +101,12 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmKernelParam
             const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
                 (uint8_t*)parked + (size_t)blockIdx.x * kParkedBytes, 0, (int)kParkedBytes, 0x00020000);
             const int at = t * 4;
-            ring_multiply<T, SHUF, XS4, 1>(smem3, src, wave, lane, 0, fold_kb, busy, ws_vec, acc);
+            ring_multiply<T, SHUF, XS4>(smem3, src, wave, lane, 0, fold_kb, busy, ws_vec, acc);
 #pragma unroll
             for(int q = 0; q < 64; ++q)
                 __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[q >> 4][(q >> 2) & 3][q & 3]), rsrc, at, q * 2048, 0);
             zero();
-            ring_multiply<T, SHUF, XS4, 1>(smem3, src, wave, lane, fold_kb, p.kblocks, busy, ws_vec, acc);
+            ring_multiply<T, SHUF, XS4>(smem3, src, wave, lane, fold_kb, p.kblocks, busy, ws_vec, acc);
             // (all requested before the first is added: left to itself the compiler may wait for them one by one)
             float back[64];
 #pragma unroll
@@ -118,7 +118,7 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmKernelParam
                 acc[q >> 4][(q >> 2) & 3][q & 3] = back[q] + acc[q >> 4][(q >> 2) & 3][q & 3];
         }
         else
-            ring_multiply<T, SHUF, XS4, 1>(smem3, src, wave, lane, 0, p.kblocks, busy, ws_vec, acc);
+            ring_multiply<T, SHUF, XS4>(smem3, src, wave, lane, 0, p.kblocks, busy, ws_vec, acc);
 
         const uint32_t ebase = (uint32_t)wave * (64u * kOutPitch);
         typedef u32x2 __attribute__((address_space(3)))*       lds_u2_ptr;

@@ -533,6 +533,24 @@ def test_fmoe_tiles_with_more_items_than_workgroups(tokens, dim, inter, experts,
         assert torch.equal(want.view(torch.int16), got.view(torch.int16))
 
 
+@pytest.mark.parametrize("dim", [256, 768, 1280, 8448])  # 2, 6, 10 and 66 K blocks: less than a round of chains, and past a window
+@pytest.mark.parametrize("per_expert,experts", [
+    (70, 260),   # 260 tiles: 32 or 33 items per XCD, the last in quarters of a tile's rows (3 blocks: one of them twice)
+    (33, 300),   # 300: 5 or 6 of them left, two blocks each
+    (128, 320),  # 320: 8 left, in quarters of one block
+    (100, 352),  # 352: 12 left, in halves
+    (20, 400),   # 400: 18 left, one block each, as they are
+])
+def test_fmoe_tiles_of_the_last_round_are_cut(dim, per_expert, experts):
+    # one group of columns; every expert has the same number of rows.  The additions do not depend on how rows are dealt out
+    p = make_moe(per_expert * experts // 2, dim, 128, experts, 2, seed=dim + experts)
+    p["ti"] = (torch.arange(per_expert * experts, dtype=torch.int32) % experts).view(-1, 2)
+    want = run_moe(p, bf16_input=True, kernel_name="tiles=0,down=rows")
+    for _ in range(2):
+        got = run_moe(p, bf16_input=True, kernel_name="tiles=1")
+        assert torch.equal(want.view(torch.int16), got.view(torch.int16))
+
+
 def test_fmoe_tiles_leave_few_tokens_to_the_column_kernel():
     # 500 tokens, top-16: rows and items enough for tiles, but the column kernel's tables still fit: it sums in fp32
     p = make_moe(500, 512, 128, 64, 16, seed=5)
