@@ -1705,7 +1705,11 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const void* __restrict
 // is known whether the position table's entry counts: it only has to lie inside the sorted array.
 // kChunk: slots per pass, topk (rounded up to even) where it is at most 10: a slot too many costs a request (8000 tokens,
 // top-2, the layer: 76.9 us with ten, 74.2 with two).
-template <In16 DT, int kChunk>
+// STREAM: the rows are read past the caches.  Bound by memory: more rows than the last-level cache holds are not there any more
+// when they are read, and what is allocated for them displaces the rows that still are.  us without / with, by what the rows
+// take: 940 MB (8192 tokens, top-8, dim 7168) 238 / 191 (5.5 TB/s), 402 MB 112 / 86, 268 MB 57 / 57; less than the cache:
+// 235 MB 50 / 48, 196 MB 35 / 41, 123 MB 24 / 29.
+template <In16 DT, int kChunk, bool STREAM>
 __global__ __launch_bounds__(256) void moe_combine8_kernel(const uint16_t* __restrict__ y, const float* __restrict__ sorted_weights,
                                                            const int32_t* __restrict__ where,
                                                            const int32_t* __restrict__ sorted_ids,
@@ -1734,7 +1738,8 @@ __global__ __launch_bounds__(256) void moe_combine8_kernel(const uint16_t* __res
             const int32_t r  = in ? at : 0; // (row 0 exists; what is read there is not used)
             ok[i]            = in && sorted_ids[r] == ((k << 24) | token);
             w[i]             = sorted_weights[r];
-            v[i]             = *(const u32x4*)(y + (size_t)r * dim + (size_t)q * 8);
+            const u32x4* row = (const u32x4*)(y + (size_t)r * dim + (size_t)q * 8);
+            v[i]             = STREAM ? __builtin_nontemporal_load(row) : *row;
         }
 #pragma unroll
         for(int i = 0; i < kChunk; ++i)
@@ -1930,15 +1935,16 @@ size_t moe_workspace_bytes(const MoeArgs& a)
     return b;
 }
 
-template <In16 DT>
+template <In16 DT, bool STREAM>
 static auto combine8_kernel(int topk)
 {
-    return topk <= 2   ? moe_combine8_kernel<DT, 2>
-           : topk <= 4 ? moe_combine8_kernel<DT, 4>
-           : topk <= 6 ? moe_combine8_kernel<DT, 6>
-           : topk <= 8 ? moe_combine8_kernel<DT, 8>
-                       : moe_combine8_kernel<DT, 10>;
+    return topk <= 2   ? moe_combine8_kernel<DT, 2, STREAM>
+           : topk <= 4 ? moe_combine8_kernel<DT, 4, STREAM>
+           : topk <= 6 ? moe_combine8_kernel<DT, 6, STREAM>
+           : topk <= 8 ? moe_combine8_kernel<DT, 8, STREAM>
+                       : moe_combine8_kernel<DT, 10, STREAM>;
 }
+constexpr size_t kLastLevelCacheBytes = (size_t)256 << 20;
 
 // out[token] += the token's rows, weighted, in slot order
 static hipError_t launch_combine(const MoeArgs& a, const void* y, bool y32, const int32_t* where, hipStream_t stream)
@@ -1946,7 +1952,10 @@ static hipError_t launch_combine(const MoeArgs& a, const void* y, bool y32, cons
     if(!y32 && (a.dim & 7) == 0 && (a.out_stride & 7) == 0 && ((uintptr_t)a.out & 15) == 0 && ((uintptr_t)y & 15) == 0)
     {
         const dim3 grid8((unsigned)a.M, (unsigned)((a.dim / 8 + 255) / 256));
-        auto combine8 = a.out_dtype == In16::bf16 ? combine8_kernel<In16::bf16>(a.topk) : combine8_kernel<In16::fp16>(a.topk);
+        const bool stream_rows = (size_t)a.M * a.topk * a.dim * 2 >= kLastLevelCacheBytes;
+        auto       combine8    = a.out_dtype == In16::bf16
+                                     ? (stream_rows ? combine8_kernel<In16::bf16, true>(a.topk) : combine8_kernel<In16::bf16, false>(a.topk))
+                                     : (stream_rows ? combine8_kernel<In16::fp16, true>(a.topk) : combine8_kernel<In16::fp16, false>(a.topk));
         hipLaunchKernelGGL(combine8, grid8, dim3(256), 0, stream, (const uint16_t*)y, a.sorted_weights, where, a.sorted_ids,
                            a.num_valid, a.max_padded, (uint16_t*)a.out, a.M, a.topk, a.dim, a.out_stride, a.overwrite);
         return hipGetLastError();

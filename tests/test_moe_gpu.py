@@ -551,6 +551,20 @@ def test_fmoe_tiles_of_the_last_round_are_cut(dim, per_expert, experts):
         assert torch.equal(want.view(torch.int16), got.view(torch.int16))
 
 
+@pytest.mark.parametrize("below,dim,topk", [(2340, 7168, 8), (3276, 8192, 5), (16383, 4096, 2)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_fmoe_sum_of_more_rows_than_the_last_level_cache_holds(below, dim, topk, dtype):
+    # 256 MiB of rows lie between `below` tokens and one more; a token's sum does not depend on how many there are
+    assert below * topk * dim * 2 < 256 << 20 <= (below + 1) * topk * dim * 2
+    p = make_moe(below + 1, dim, 128, 8, topk, seed=below)
+    more = run_moe(p, dtype=dtype, bf16_input=True)
+    for name in ("x", "ti", "tw"):
+        p[name] = p[name][:below].contiguous()
+    fewer = run_moe(p, dtype=dtype, bf16_input=True)
+    assert torch.equal(more[:below].view(torch.int16), fewer.view(torch.int16))
+    assert more[below].float().norm() > 0
+
+
 def test_fmoe_tiles_leave_few_tokens_to_the_column_kernel():
     # 500 tokens, top-16: rows and items enough for tiles, but the column kernel's tables still fit: it sums in fp32
     p = make_moe(500, 512, 128, 64, 16, seed=5)
