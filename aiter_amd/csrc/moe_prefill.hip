@@ -926,8 +926,9 @@ hipError_t launch_moe_prefill_gemms(const MoeArgs& a, hipStream_t stream, void* 
     d.lda       = a.inter;
     if(d.kblocks <= 2)
     {
-        // each wave of an item walks about seven groups of columns: enough to amortise the tile's rows, and enough items
-        d.col_splits = std::max(1, a.dim / 64 / (7 * kDownWaves));
+        const int64_t pairs = (int64_t)a.M * a.topk;
+        const int64_t all   = routed_experts(pairs, a.topk, a.block_rows << a.expert_shift, a.max_padded, a.experts);
+        d.col_splits        = down_col_splits((double)pairs / (double)all, a.experts, a.dim / 64, kDownWaves);
         const size_t lds = down_lds_bytes(d.kblocks, f32);
         auto kernel = d.kblocks == 1 ? (f32 ? moe_prefill_down_kernel<1, true> : moe_prefill_down_kernel<1, false>)
                                      : (f32 ? moe_prefill_down_kernel<2, true> : moe_prefill_down_kernel<2, false>);

@@ -44,4 +44,23 @@ inline bool tiles_win(int64_t pairs, int64_t all, int experts, int inter)
     return rows >= least && items >= 80.0;
 }
 
+// Second GEMM with its rows in LDS: the parts that a tile's groups of 64 columns are cut into, one item each, of which the
+// workgroup's waves take a group at a time.  More items fill 512 workgroups evenly and keep more requests in flight, but each
+// brings the tile's rows into LDS.  us with 7, 4, 2 and 1 groups per wave (tokens, experts, topk, dim, inter; items with one):
+//   (1000, 32, 5, 5120, 256)   1160: 39 / - / 24 / 22     (2500, 40, 6, 4352, 256)  2400: 64 / 58 / 54 / 46
+//   (2795, 64, 6, 2816, 256)   1826: 59 / - / 41 / 36     (1184, 8, 2, 6400, 128)    500: 27 / 17 / 15 / 12
+//   (5184, 256, 8, 2048, 256)  3616: 75 / 68 / 71 / 69    (3000, 128, 8, 4096, 128) 4000: 58 / 53 / 52 / 55
+//   (2048, 256, 8, 7168, 256)  7170: 156 / - / 144 / 142  (4096, 256, 8, 4096, 256) 6140: 123 / 108 / 109 / 117
+//   (8192, 256, 8, 3072, 128)  7680: 115 / 98 / 92 / 95   (8192, 256, 8, 7168, 256) 17920: 304 / - / 307 / 327
+inline int down_col_splits(double rows_per_expert, int experts, int groups, int waves)
+{
+    const double tiles = (rows_per_expert / kTileRowsOfExpert + 0.5) * experts; // an expert's last one is half full on average
+    auto splits = [&](int per_wave) { return groups <= per_wave * waves ? 1 : (groups + per_wave * waves - 1) / (per_wave * waves); };
+    if(tiles * splits(1) <= 3800.0)
+        return splits(1);
+    if(tiles * splits(2) <= 5000.0)
+        return splits(2);
+    return groups <= 7 * waves ? 1 : groups / (7 * waves);
+}
+
 } // namespace fp8bs

@@ -46,6 +46,14 @@ int main()
         EXPECT(!tiles_win((int64_t)m * 8, routed_experts((int64_t)m * 8, 8, 32, padded((int64_t)m * 8, 8, 32, 256), e), e, 2048));
     m = 8192;
     EXPECT(tiles_win((int64_t)m * 8, 256, e, 256) && tiles_win((int64_t)m * 8, 256, 256, 256));
+    // parts of the second GEMM's columns: at least one, never more than the workgroup's waves have groups for
+    for(e = 1; e <= 512; e += 7)
+        for(m = 1; m <= 4096; m = m * 2 + 1) // rows per expert
+            for(int groups = 4; groups <= 256; groups += 4)
+            {
+                const int splits = down_col_splits(m, e, groups, 4);
+                EXPECT(splits >= 1 && splits * 4 <= groups);
+            }
     std::printf("OK\n");
     return 0;
 }

@@ -565,6 +565,19 @@ def test_fmoe_sum_of_more_rows_than_the_last_level_cache_holds(below, dim, topk,
     assert more[below].float().norm() > 0
 
 
+@pytest.mark.parametrize("tokens,dim,inter,experts,topk", [
+    (700, 256, 128, 3, 2),     # one group of columns per wave: four groups, one part
+    (700, 2816, 256, 12, 6),   # eleven parts
+    (2500, 4864, 128, 40, 6),  # two groups per wave: ten parts of seven or eight of the 76 groups
+    (8000, 5120, 128, 64, 8),  # seven: two parts of forty
+])
+def test_fmoe_tiles_whose_columns_are_cut_into_parts(tokens, dim, inter, experts, topk):
+    p = make_moe(tokens, dim, inter, experts, topk, seed=tokens + dim)
+    want = run_moe(p, bf16_input=True, kernel_name="tiles=0,down=rows")
+    got = run_moe(p, bf16_input=True, kernel_name="tiles=1")
+    assert torch.equal(want.view(torch.int16), got.view(torch.int16))
+
+
 def test_fmoe_tiles_leave_few_tokens_to_the_column_kernel():
     # 500 tokens, top-16: rows and items enough for tiles, but the column kernel's tables still fit: it sums in fp32
     p = make_moe(500, 512, 128, 64, 16, seed=5)
