@@ -18,7 +18,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_NAME = "libaiter_fp8bs.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 
-SOURCES = ["abi.hip", "workspace.hip", "norm_quant_kernels.hip", "gemm_blockscale_kernels.hip", "gemm_prefill.hip", "gemm_ring.hip", "gemm_decode.hip",
+SOURCES = ["abi.hip", "workspace.hip", "norm_quant_kernels.hip", "gemm_blockscale_kernels.hip", "gemm_prefill.hip", "gemm_ring.hip", "gemm_band.hip", "gemm_decode.hip",
            "gemm_mid.hip", "moe_kernels.hip", "moe_prefill.hip"]
 
 # -ffp-contract=off: the quantiser's rounding sequence must stay one IEEE operation per step.

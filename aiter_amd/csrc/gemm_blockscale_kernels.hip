@@ -298,6 +298,8 @@ static hipError_t dispatch(const GemmArgs& a, const GemmKernelParams& p, hipStre
     ctx.stream      = stream;
     ctx.why         = why;
     ctx.static_only = a.static_scratch;
+    // bands of weight rows in place of what was chosen here with K in one range: the same sums
+    const int band = gemm_prefill_supports(p) ? gemm_band_rows(p, 256) : 0;
     switch(k.family)
     {
     case Family::tile:
@@ -320,6 +322,8 @@ static hipError_t dispatch(const GemmArgs& a, const GemmKernelParams& p, hipStre
             *why = "the mid_* kernels need operand matrices below 4 GiB";
             return hipErrorInvalidValue;
         }
+        if(!named && req.split_k_log2 < 0 && band && gemm_mid_ranges(p) == 1)
+            return launch_gemm_band(p, DT, ctx, band);
         return launch_gemm_mid(p, DT, req.split_k_log2, ctx, k.tile, k.splits);
     case Family::prefill:
         if(!gemm_prefill_supports(p))
@@ -331,6 +335,8 @@ static hipError_t dispatch(const GemmArgs& a, const GemmKernelParams& p, hipStre
         // unless ":s=" pins the K ranges per tile; chosen automatically, the launcher decides -- but for
         // 256 x 128 tiles, which may stand for a plan of another family.
         // splitK is a hint this kernel has no use for.
+        if(!named && band && (k.tile == 128 || gemm_prefill_plan(p, 256).splits == 1))
+            return launch_gemm_band(p, DT, ctx, band);
         return launch_gemm_prefill(p, DT, ctx, k.splits > 0 ? k.splits : (named ? 1 : 0), named || k.tile == 128 ? k.tile : 0);
     }
     *why = kUnknownName;

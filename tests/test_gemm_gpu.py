@@ -433,6 +433,38 @@ def test_narrow_prefill_tiles_as_the_library_chooses_them(m, n, k, expect):
     assert torch.equal(pre.view(torch.int16), named.view(torch.int16))
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (203, 36864, 7168),   # bands of 144 rows of weights, 256 workgroups: K blocks in windows of four; rows to 208
+    (65, 32772, 128),     # one K block, fewer than the stages of either ring; a last band of 84 columns, rows not 16-byte aligned
+    (256, 36856, 256),    # two
+    (70, 32784, 384),     # an odd number of them
+    (129, 36860, 640),
+    (257, 16400, 1152),   # two rows of tiles, the second with one row in it
+    (1000, 9216, 512),    # four
+    (2044, 4480, 8320),   # eight; 65 K blocks: past one window of w_scale
+    (150, 16512, 5120),   # bands of 96: 172 workgroups, 40 K blocks
+    (33, 24576, 5248),    # 41: odd; 128 MiB of weights, past the caches; two of the eight waves have rows
+    (100, 24572, 5632),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_bands_of_weight_rows_carry_out_plans_of_one_range(m, n, k, dtype):
+    # what the library chooses, against the kernel that keeps a tile's K in one workgroup: the same products in the same order
+    assert ":s=" not in _ffi.gemm_choice(m, n, k) or _ffi.gemm_choice(m, n, k).endswith(":s=1")
+    xq, wq, xs, ws = _gpu_problem(m, n, k, seed=m + n + k, outliers=True)
+    tile = torch.empty(m, n, dtype=dtype, device=DEV)
+    aiter_amd.gemm_a8w8_blockscale_ck(xq, wq, xs, ws, tile, kernelName="tile_128x128")
+    out = torch.full((m, n), float("nan"), dtype=dtype, device=DEV)
+    aiter_amd.gemm_a8w8_blockscale_ck(xq, wq, xs, ws, out, splitK=-1)
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), tile.view(torch.int16))
+    if n % 16 == 0:
+        wsh = aiter_amd.shuffle_weight(wq.view(torch.uint8)).view(wq.dtype)
+        out.fill_(float("nan"))
+        aiter_amd.gemm_a8w8_blockscale_bpreshuffle_ck(xq, wsh, xs.t().contiguous().view(*xs.shape), ws, out)
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), tile.view(torch.int16))
+
+
 @pytest.mark.parametrize("m,n,k", [(4352, 4096, 256), (4352, 4352, 128), (4100, 4360, 256)])
 def test_prefill_kernel_more_tiles_than_compute_units(m, n, k):
     # 272 / 289 / 306 tiles of 256x256 on 256 compute units: workgroups take a second tile (a
