@@ -23,6 +23,7 @@
 // slots in slot order, weighted, into `out`.  Both are deterministic, unlike atomic accumulation.
 #include "gemm_common.h"
 #include "moe_launch.h"
+#include "moe_rules.h"
 
 #include <algorithm>
 #include <atomic>
@@ -1814,10 +1815,16 @@ bool moe_down_by_columns(const MoeArgs& a)
                       a.max_blocks <= kColsMaxBlocks && a.dim % (16 * kColsTiles) == 0;
     if(a.down_mode == 1 || !fits)
         return false;
-    // measured on the DeepSeek-V3 layer against rows through memory: with two walkers 4 % faster at 1 token,
-    // 6 % at 16-192, 8 % at 256 and 264 (275 against 297 us); with one walker (the tables of two no longer
-    // fit) 2 % slower at 288-320 tokens
-    return a.down_mode == 2 || cols_walkers(a) == 2;
+    if(a.down_mode == 2)
+        return true;
+    // with one walker (the tables of two no longer fit) 2 % slower at 288-320 tokens of the DeepSeek-V3 layer
+    if(cols_walkers(a) != 2)
+        return false;
+    // Rows that would wait in bf16 are the column kernel's as long as it fits.  In fp32 they are summed with one rounding less per
+    // product: against 64 bits 5.4e-8 to 6.2e-8 for topk 6 and 8 and inter 128 and 256, in columns 5.8e-8 to 6.8e-8.
+    const int64_t pairs = (int64_t)a.M * a.topk;
+    return !moe_rows_in_f32(a) || !rows_beat_columns(pairs, routed_experts(pairs, a.topk, a.block_rows << a.expert_shift, a.max_padded, a.experts),
+                                                     a.experts, a.dim, a.inter);
 }
 
 template <typename T>

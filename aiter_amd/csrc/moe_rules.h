@@ -2,6 +2,7 @@
 // be compiled and tested on the host.
 #pragma once
 
+#include <math.h>
 #include <stdint.h>
 
 namespace fp8bs {
@@ -61,6 +62,28 @@ inline int down_col_splits(double rows_per_expert, int experts, int groups, int 
     if(tiles * splits(2) <= 5000.0)
         return splits(2);
     return groups <= 7 * waves ? 1 : groups / (7 * waves);
+}
+
+// Whether few tokens' rows, kept in fp32, go through memory to a kernel of their own for the per-token sum, where the kernel that owns
+// 32 columns and sums in LDS would fit too.  That one walks every block of rows in each of its dim / 32 workgroups: a block's
+// K block takes it 0.13 us, more than memory needs for all columns' weights below dim 5000, and a pair of token and expert
+// 0.02 us; rows through memory cost a launch (with some margin 6.5 us), are written and read, and their weights arrive 6 % more slowly.
+// Over 100 drawn layers (1 to 300 tokens, inter 128 and 256) this takes 0.5 % longer than the better of the two on average and 14 %
+// at worst, where columns stay.  us in columns / through memory, sort excluded (tokens, experts, topk, dim, inter):
+//   (140, 64, 6, 1536, 128)  47 / 35    (204, 64, 6, 3840, 128)  64 / 53    (29, 256, 8, 1024, 128)  47 / 30
+//   (295, 128, 8, 4096, 256) 169 / 109  (18, 256, 8, 1280, 256)  48 / 38    (61, 256, 8, 3840, 256) 114 / 107
+//   (16, 256, 8, 7168, 256)  89 / 94    (128, 256, 8, 7168, 256) 199 / 213  (66, 256, 8, 4864, 256) 131 / 133
+//   (1, 256, 8, 1024, 256)   17 / 20    (3, 32, 5, 6400, 256)    24 / 26    (110, 256, 8, 5376, 256) 164 / 168
+// Measured from dim 1024 on; below, columns as long as they fit.
+inline bool rows_beat_columns(int64_t pairs, int64_t all, int experts, int dim, int inter)
+{
+    if(dim < 1024)
+        return false;
+    const double rows = (double)pairs / (double)all, here = rows * experts, kblocks = inter / 128;
+    const double blocks  = experts * (1.0 - exp(-rows)) + here / 32.0; // an even routing's, of up to 32 rows each
+    const double weights = dim * 25.6e-6;                              // us per block and K block, at 5 TB/s
+    const double in_columns = blocks * kblocks * (weights < 0.13 ? 0.13 - weights : 0.0) + here * 0.02;
+    return in_columns > 6.5 + here * dim * 2e-6 + blocks * kblocks * weights * 0.06;
 }
 
 } // namespace fp8bs

@@ -54,6 +54,12 @@ int main()
                 const int splits = down_col_splits(m, e, groups, 4);
                 EXPECT(splits >= 1 && splits * 4 <= groups);
             }
+    // Few tokens: rows through memory where a narrow layer leaves the column kernel few workgroups, columns for the rest.  A rank that
+    // holds a part of the experts counts its own pairs
+    m = 140, e = 64;
+    EXPECT(rows_beat_columns(140 * 6, 64, 64, 1536, 128) && !rows_beat_columns(140 * 6, 64, 64, 512, 128));
+    EXPECT(!rows_beat_columns(16 * 8, 256, 256, 7168, 256) && !rows_beat_columns(128 * 8, 256, 256, 7168, 256));
+    EXPECT(!rows_beat_columns(5, 32, 32, 1024, 256) && !rows_beat_columns(140 * 6, 64, 4, 1536, 128));
     std::printf("OK\n");
     return 0;
 }

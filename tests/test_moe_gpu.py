@@ -585,6 +585,25 @@ def test_fmoe_tiles_leave_few_tokens_to_the_column_kernel():
     assert torch.equal(want.view(torch.int16), run_moe(p, bf16_input=True).view(torch.int16))
 
 
+@pytest.mark.parametrize("tokens,dim,inter,experts,topk,rows", [
+    (140, 1536, 128, 64, 6, True),
+    (140, 768, 128, 64, 6, False),   # a dim below those that were measured
+    (16, 5120, 256, 64, 8, False),   # wide enough that columns cover the chip
+    (29, 1024, 128, 256, 8, True),   # experts with one row or none
+    (3, 1024, 256, 32, 5, False),    # a launch more than it saves
+    (270, 1280, 256, 5, 3, True),    # the most tokens that two walkers' tables fit
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_fmoe_few_tokens_take_columns_or_rows(tokens, dim, inter, experts, topk, rows, dtype):
+    p = make_moe(tokens, dim, inter, experts, topk, seed=tokens + dim, w_std=0.05)
+    auto = run_moe(p, dtype=dtype, bf16_input=True)
+    for hint in ("down=cols", "down=rows"):
+        got = run_moe(p, dtype=dtype, bf16_input=True, kernel_name=hint)
+        assert_close(got, reference(p), hint)
+        if (hint == "down=rows") == rows:
+            assert torch.equal(auto.view(torch.int16), got.view(torch.int16))
+
+
 @pytest.mark.parametrize("block", [64, 128])
 def test_fmoe_pairs_of_blocks_in_arrays_sorted_in_larger_blocks(block):
     # sorted in blocks of 64 or 128 rows, the kernels' 32-row blocks of one sorted block share an expert id:
