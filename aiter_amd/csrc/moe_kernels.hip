@@ -136,7 +136,8 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__
 // the chunks, one wave per expert; a stable scatter, one wave per chunk, so that pairs keep their (token, slot) order, in
 // which every wave works out for itself where the experts' runs start.  (8192 tokens, top-8 of 256: the scan 4.7 us
 // and the scatter 8.4; 21.1 and 7.1 with one workgroup for the whole scan and the padding behind each expert's run entry by
-// entry.)  Up to kSortChunk pairs one workgroup does it all (500 tokens: 13.4 us, 17.5 with that padding).
+// entry.)  Up to kSortChunk pairs one workgroup does it all, bound by its own instructions and by what it waits for in turn: 500
+// tokens, top-8 of 256: 10.7 us (13.4 with divisions per pair, ten bits of expert ids and loads asked for where they are used).
 struct SortParams
 {
     const int32_t* topk_ids;     // [M][topk], row stride id_stride
@@ -168,6 +169,41 @@ __device__ __forceinline__ int32_t sort_rows(const SortParams& p)
     }
     return rows < p.w_rows ? rows : p.w_rows;
 }
+
+// (token, slot) of pair `first` + i, i < 2^20.  The sorts turn pairs into tokens and slots several times each; an integer division is
+// some 35 instructions (with 64 bits 100), which in a workgroup or two that do it all are microseconds.  One at the front, and for
+// the rest a product: i + 0.5 stays half a step of 1 / topk away from the next multiple, 2^-22 of it is less below 2^21.
+struct PairIndex
+{
+    int32_t token, slot, topk;
+    float   inv;
+    __device__ __forceinline__ PairIndex(int64_t first, int32_t topk_) : topk(topk_), inv(1.f / (float)topk_)
+    {
+        token = (int32_t)(first / topk_);
+        slot  = (int32_t)(first - (int64_t)token * topk_);
+    }
+    __device__ __forceinline__ void at(int i, int32_t& t, int32_t& s) const
+    {
+        const int32_t x = slot + i, q = (int32_t)(((float)x + 0.5f) * inv);
+        t = token + q;
+        s = x - q * topk;
+    }
+};
+
+// The lanes whose expert is this lane's, out of `in` (ids below 2^bits)
+__device__ __forceinline__ uint64_t lanes_of_expert(uint64_t in, int32_t e, int bits)
+{
+    uint32_t lo = (uint32_t)in, hi = (uint32_t)(in >> 32);
+    for(int b = 0; b < bits; ++b)
+    {
+        const uint64_t bal  = __ballot((e >> b) & 1);
+        const uint32_t mine = (uint32_t)__builtin_amdgcn_sbfe(e, b, 1); // all ones where the bit is set
+        lo &= ~((uint32_t)bal ^ mine);
+        hi &= ~((uint32_t)(bal >> 32) ^ mine);
+    }
+    return (uint64_t)hi << 32 | lo;
+}
+__device__ __forceinline__ int expert_bits(int experts) { return 32 - __builtin_clz((uint32_t)(experts > 1 ? experts - 1 : 1)); }
 
 // The output buffer of the expert layer has to come back zeroed.  Rather than a launch of its own,
 // the workgroups of the first sorting launch beyond the `first` that sort clear it.
@@ -206,12 +242,14 @@ __global__ __launch_bounds__(1024) void moe_sort_count_kernel(SortParams p)
     __syncthreads();
     const int64_t n = (int64_t)sort_rows(p) * p.topk;
     const int64_t lo = (int64_t)blockIdx.x * p.chunk_pairs;
+    const PairIndex pairs(lo, p.topk);
     for(int i = threadIdx.x; i < p.chunk_pairs; i += blockDim.x)
     {
-        const int64_t f = lo + i;
-        if(f >= n)
+        if(lo + i >= n)
             break;
-        const int32_t e = p.topk_ids[(f / p.topk) * p.id_stride + (f % p.topk)];
+        int32_t token, slot;
+        pairs.at(i, token, slot);
+        const int32_t e = p.topk_ids[(size_t)token * p.id_stride + slot];
         if(e >= 0 && e < p.experts)
             atomicAdd(&hist[e], 1);
     }
@@ -298,29 +336,24 @@ __global__ __launch_bounds__(256) void moe_sort_scan_kernel(SortParams p)
 // a pair's rank among the earlier pairs of its expert comes from ballots over the bits of the
 // expert id, and `running[e]` (LDS) carries the expert's fill level from one step to the next.
 __device__ __forceinline__ void scatter_chunk(const SortParams& p, const int32_t* ids, const float* wts,
-                                              const int32_t* begin, int32_t* running, int cnt, int64_t first)
+                                              const int32_t* begin, int32_t* running, int cnt, const PairIndex& pairs)
 {
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, bits = expert_bits(p.experts);
     for(int base = 0; base < cnt; base += 64)
     {
         const int  i  = base + lane;
         const int  e  = i < cnt ? ids[i] : -1;
         const bool in = e >= 0 && e < p.experts && begin[e] >= 0;
-        uint64_t   same = __ballot(in);
-#pragma unroll
-        for(int b = 0; b < 10; ++b)
-        {
-            const uint64_t bal = __ballot((e >> b) & 1);
-            same &= ((e >> b) & 1) ? bal : ~bal;
-        }
+        const uint64_t same = lanes_of_expert(__ballot(in), e, bits);
         if(in)
         {
             const int     rank = __popcll(same & ((1ull << lane) - 1ull));
             const int     n    = __popcll(same);
             const int32_t fill = running[e];
             const int32_t at   = begin[e] + fill + rank;
-            const int64_t f    = first + i;
-            p.sorted_ids[at]     = ((int32_t)(f % p.topk) << 24) | (int32_t)(f / p.topk);
+            int32_t       token, slot;
+            pairs.at(i, token, slot);
+            p.sorted_ids[at]     = slot << 24 | token;
             p.sorted_weights[at] = wts[i];
             if(rank == n - 1)
                 running[e] = fill + n;
@@ -339,11 +372,13 @@ __global__ __launch_bounds__(64) void moe_sort_scatter_kernel(SortParams p)
     const int64_t      n  = (int64_t)sort_rows(p) * p.topk;
     const int64_t      lo = (int64_t)blockIdx.x * p.chunk_pairs;
     const int          cnt = !scatters ? 0 : (int)((n - lo) < p.chunk_pairs ? (n - lo > 0 ? n - lo : 0) : p.chunk_pairs);
+    const PairIndex pairs(lo, p.topk);
     for(int i = lane; i < cnt; i += 64)
     {
-        const int64_t f = lo + i;
-        ids[i]          = p.topk_ids[(f / p.topk) * p.id_stride + (f % p.topk)];
-        wts[i]          = p.topk_weights[(f / p.topk) * p.w_stride + (f % p.topk)];
+        int32_t token, slot;
+        pairs.at(i, token, slot);
+        ids[i] = p.topk_ids[(size_t)token * p.id_stride + slot];
+        wts[i] = p.topk_weights[(size_t)token * p.w_stride + slot];
     }
     if(scatters)
         for(int e = lane; e < p.experts; e += 64)
@@ -378,7 +413,7 @@ __global__ __launch_bounds__(64) void moe_sort_scatter_kernel(SortParams p)
         p.num_valid_ids[1] = sort_rows(p);
     }
     __syncthreads();
-    scatter_chunk(p, ids, wts, begin, running, cnt, lo);
+    scatter_chunk(p, ids, wts, begin, running, cnt, pairs);
 }
 
 // All of it in one workgroup, for up to kSortChunk pairs (the decode regime).  The pairs are cut
@@ -388,19 +423,30 @@ __global__ __launch_bounds__(64) void moe_sort_scatter_kernel(SortParams p)
 constexpr int kSortWaves = 8;
 constexpr int kSortRunSteps = kSortChunk / kSortWaves / 64; // 64-pair steps of the longest run
 
-// scatter_chunk for one run of the one-workgroup sort: the weights come from memory, all of the
-// run's requested before the first step (they would otherwise cost a round trip per step)
-__device__ __forceinline__ void scatter_run(const SortParams& p, const int32_t* ids, const int32_t* begin,
-                                            int32_t* running, int cnt, int first)
+// What a lane scatters of its wave's run: asked for before anything else, a round trip per step costs more than the rest.
+struct SortRun
+{
+    float   w[kSortRunSteps];
+    int32_t id[kSortRunSteps]; // as it is stored
+};
+__device__ __forceinline__ void load_run(const SortParams& p, const PairIndex& pairs, int cnt, int first, SortRun& run)
 {
     const int lane = threadIdx.x & 63;
-    float     w[kSortRunSteps];
 #pragma unroll
     for(int st = 0; st < kSortRunSteps; ++st)
     {
-        const int f = first + st * 64 + lane;
-        w[st]       = st * 64 + lane < cnt ? p.topk_weights[(size_t)(f / p.topk) * p.w_stride + (f % p.topk)] : 0.f;
+        int32_t token, slot;
+        pairs.at(first + st * 64 + lane, token, slot);
+        run.w[st]  = st * 64 + lane < cnt ? p.topk_weights[(size_t)token * p.w_stride + slot] : 0.f;
+        run.id[st] = slot << 24 | token;
     }
+}
+
+// scatter_chunk for one run of the one-workgroup sort
+__device__ __forceinline__ void scatter_run(const SortParams& p, const int32_t* ids, const int32_t* begin,
+                                            int32_t* running, int cnt, const SortRun& run)
+{
+    const int lane = threadIdx.x & 63, bits = expert_bits(p.experts);
 #pragma unroll
     for(int st = 0; st < kSortRunSteps; ++st)
     {
@@ -409,22 +455,15 @@ __device__ __forceinline__ void scatter_run(const SortParams& p, const int32_t* 
         const int  i  = st * 64 + lane;
         const int  e  = i < cnt ? ids[i] : -1;
         const bool in = e >= 0 && e < p.experts && begin[e] >= 0;
-        uint64_t   same = __ballot(in);
-#pragma unroll
-        for(int b = 0; b < 10; ++b)
-        {
-            const uint64_t bal = __ballot((e >> b) & 1);
-            same &= ((e >> b) & 1) ? bal : ~bal;
-        }
+        const uint64_t same = lanes_of_expert(__ballot(in), e, bits);
         if(in)
         {
             const int     rank = __popcll(same & ((1ull << lane) - 1ull));
             const int     n    = __popcll(same);
             const int32_t fill = running[e];
             const int32_t at   = begin[e] + fill + rank;
-            const int     f    = first + i;
-            p.sorted_ids[at]     = ((int32_t)(f % p.topk) << 24) | (int32_t)(f / p.topk);
-            p.sorted_weights[at] = w[st];
+            p.sorted_ids[at]     = run.id[st];
+            p.sorted_weights[at] = run.w[st];
             if(rank == n - 1)
                 running[e] = fill + n;
         }
@@ -443,18 +482,37 @@ __global__ __launch_bounds__(1024) void moe_sort_single_kernel(SortParams p)
     __shared__ int32_t count[1024], begin[1024], local[1024];
     const int rows = sort_rows(p);
     const int cnt  = rows * p.topk; // <= kSortChunk, checked at launch
-    const int run_len = ((cnt + kSortWaves - 1) / kSortWaves + 63) / 64 * 64;
+    const int run_len = max(64, ((cnt + kSortWaves - 1) / kSortWaves + 63) / 64 * 64);
+    // every load of the pairs leaves before the first of them is waited for
+    const PairIndex pairs(0, p.topk);
+    const int       wave = threadIdx.x >> 6, first = wave * run_len;
+    const int       run_pairs = wave >= kSortWaves ? 0 : cnt - first < run_len ? cnt - first : run_len;
+    constexpr int   kPerThread = kSortChunk / 1024;
+    int32_t         mine[kPerThread];
+    SortRun         run;
+#pragma unroll
+    for(int u = 0; u < kPerThread; ++u)
+    {
+        const int i = u * 1024 + threadIdx.x;
+        int32_t   token, slot;
+        pairs.at(i, token, slot);
+        mine[u] = i < cnt ? p.topk_ids[(size_t)token * p.id_stride + slot] : -1;
+    }
+    if(run_pairs > 0)
+        load_run(p, pairs, run_pairs, first, run);
     fill_padding(p, (int)threadIdx.x, (int)blockDim.x);
     for(int i = threadIdx.x; i < kSortWaves * 1024; i += blockDim.x)
         (&fill[0][0])[i] = 0;
     __syncthreads();
-    for(int i = threadIdx.x; i < cnt; i += blockDim.x)
+#pragma unroll
+    for(int u = 0; u < kPerThread; ++u)
     {
-        const int     r = i / p.topk, k = i - r * p.topk;
-        const int32_t e = p.topk_ids[(size_t)r * p.id_stride + k];
-        ids[i]          = e;
-        if(e >= 0 && e < p.experts)
-            atomicAdd(&fill[i / run_len][e], 1);
+        const int i = u * 1024 + threadIdx.x;
+        if(i < cnt)
+            ids[i] = mine[u];
+        const int of = __builtin_amdgcn_readfirstlane(i) / run_len; // (runs are whole waves)
+        if(mine[u] >= 0 && mine[u] < p.experts)
+            atomicAdd(&fill[of][mine[u]], 1);
     }
     __syncthreads();
     if((int)threadIdx.x < p.experts)
@@ -487,14 +545,8 @@ __global__ __launch_bounds__(1024) void moe_sort_single_kernel(SortParams p)
         p.num_valid_ids[1] = rows;
     }
     __syncthreads();
-    const int wave = threadIdx.x >> 6;
-    if(wave < kSortWaves)
-    {
-        const int lo = wave * run_len;
-        const int n  = cnt - lo < run_len ? cnt - lo : run_len;
-        if(n > 0)
-            scatter_run(p, ids + lo, begin, fill[wave], n, lo);
-    }
+    if(run_pairs > 0)
+        scatter_run(p, ids + first, begin, fill[wave], run_pairs, run);
 }
 
 

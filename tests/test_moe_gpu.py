@@ -155,6 +155,15 @@ def test_moe_sorting_in_three_launches(tokens, experts, topk, block):
     check_sorting(ids, w, experts, block=block, num_local_tokens=0)
 
 
+@pytest.mark.parametrize("tokens,experts,topk", [
+    (64, 2, 2), (65, 3, 1), (63, 8, 5), (4096, 5, 1), (4097, 5, 1), (819, 1000, 5), (1366, 1024, 3), (586, 33, 7), (128, 256, 32),
+    (129, 257, 32), (20000, 129, 9),
+])
+def test_moe_sorting_runs_that_end_inside_a_token(tokens, experts, topk):
+    # of 64 pairs in one launch and of 256 in three, up to one pair more than one launch takes; expert ids of one bit to ten
+    check_sorting(*routed(tokens, experts, topk, tokens + experts), experts)
+
+
 def test_moe_sorting_strided_inputs_and_repeat_calls():
     ids, w = routed(100, 16, 4, 3)
     wide_i = torch.full((100, 8), -5, dtype=torch.int32)
