@@ -613,6 +613,14 @@ def test_fmoe_few_tokens_take_columns_or_rows(tokens, dim, inter, experts, topk,
             assert torch.equal(auto.view(torch.int16), got.view(torch.int16))
 
 
+@pytest.mark.parametrize("topk", [1, 2, 3, 5, 8, 9, 10, 11, 23])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_fmoe_sum_of_fp32_rows(topk, dtype):
+    # slots per pass: 2, 4, 6, 8 or 10, the last pass partly empty; a second pass; 288 lanes' worth of columns
+    p = make_moe(37, 1280, 128, 24, topk, seed=topk, w_std=0.05)
+    assert_close(run_moe(p, dtype=dtype, kernel_name="down=rows"), reference(p), f"top-{topk}")
+
+
 @pytest.mark.parametrize("block", [64, 128])
 def test_fmoe_pairs_of_blocks_in_arrays_sorted_in_larger_blocks(block):
     # sorted in blocks of 64 or 128 rows, the kernels' 32-row blocks of one sorted block share an expert id:
