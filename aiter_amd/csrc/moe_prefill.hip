@@ -832,7 +832,7 @@ bool moe_prefill_wanted(const MoeArgs& a)
         return false;
     const int64_t pairs = (int64_t)a.M * a.topk;
     const int64_t all   = routed_experts(pairs, a.topk, a.block_rows << a.expert_shift, a.max_padded, a.experts);
-    return tiles_win(pairs, all, a.experts, a.inter);
+    return tiles_win(pairs, all, a.experts, a.inter, a.dim);
 }
 
 size_t moe_prefill_workspace_bytes(const MoeArgs& a)

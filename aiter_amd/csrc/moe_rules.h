@@ -19,30 +19,34 @@ inline int64_t routed_experts(int64_t pairs, int topk, int unit, int64_t padded,
 }
 
 // Tiles win where an expert has enough rows that the block-wise kernels' repeated passes over its weights cost more than a
-// tile's padding -- fewer with a longer K of the second GEMM, where those kernels have nothing in flight while they multiply --
-// and where there are enough items (a tile's 128 columns of the product; an expert's last tile is half full on average) for
-// the chip.  Over 1139 drawn layers (5 to 256 experts, 8 to 1200 rows each, dim 1024 to 7168) this takes 0.5 % longer than
-// the better of the two on average, 5 % and more in 43 and 23 % at worst.  us block by block / in tiles (experts, topk, dim,
-// inter):
-//   (256, 8, 3072, 128)  64 rows per expert (256 items): 181 / 198, 80 (288): 215 / 206, 128: 299 / 236
-//   (256, 8, 7168, 256)  48 (448): 468 / 490, 52: 494 / 479, 64: 553 / 515, 256: 1724 / 1044
-//   (128, 8, 7168, 256)  64 (256): 294 / 319, 80 (288): 342 / 341, 96: 385 / 343
-//   (32, 5, 4096, 256)   96 (80): 92 / 106, 112 (88): 109 / 108, 160: 137 / 113
-//   (8, 2, 1024, 256)    640 (88): 72 / 75, 768 (104): 79 / 75, 1024: 88 / 77
-//   (128, 8, 4096, 384)  48 (336): 208 / 214, 56 (360): 231 / 212, 128: 392 / 291
-//   (256, 8, 2048, 512)  32 (768): 241 / 254, 40 (832): 273 / 255, 256: 1055 / 609
-//   (64, 6, 7168, 512)   48 (224): 238 / 275, 64 (256): 283 / 291, 80: 328 / 296
-//   (32, 8, 7168, 1024)  32 (192): 183 / 198, 48 (224): 207 / 192, 128: 414 / 291
-//   (16, 4, 4096, 2048)  32 (192): 121 / 112, 128: 284 / 180
-//   (32 held of 256, 8, 7168, 2048)  2: 245 / 273, 16 (320): 293 / 299, 32 (384): 396 / 319, 256: 1635 / 815
-//   (64 held of 256, 8, 4096, 1024)  16: 187 / 219, 32 (384): 226 / 229, 64: 337 / 252
+// tile's padding -- fewer with a longer K of the second GEMM, where those kernels have nothing in flight while they multiply, and
+// fewer on narrower layers, whose items are shorter -- and where there are enough items (a tile's 128 columns of the product;
+// an expert's last tile is half full on average) for the chip.  Over 211
+// layers (8 to 256 experts, 12 to 1024 rows each, dim 1024 to 7168, 150 of them drawn) this takes 1.2 % longer than the better of
+// the two on average, 5 % and more in 20, 26 % at worst; with the first condition alone 3.8 %, 52 and 31 %.  us block by block / in tiles (experts, topk, dim, inter):
+//   (256, 8, 3072, 128)  40 rows per expert (208 items): 128 / 130, 56 (240): 153 / 141, 128: 283 / 196
+//   (256, 8, 7168, 256)  40 (416): 402 / 408, 52: 462 / 426, 64: 530 / 441, 256: 1652 / 900
+//   (128, 8, 7168, 256)  48 (224): 228 / 257, 56 (240): 254 / 259, 64: 277 / 260, 96: 365 / 288
+//   (32, 5, 4096, 256)   48 (56): 61 / 61, 64 (64): 76 / 62, 112: 92 / 64, 160: 119 / 68
+//   (8, 2, 1024, 256)    384 (56): 43 / 40, 512 (72): 52 / 41, 1024: 72 / 49
+//   (128, 8, 4096, 384)  40 (312): 168 / 188, 48 (336): 187 / 184, 128: 377 / 252
+//   (256, 8, 2048, 512)  24 (704): 190 / 195, 32 (768): 219 / 212, 256: 1016 / 492
+//   (64, 6, 7168, 512)   48 (224): 218 / 240, 64 (256): 267 / 247, 80: 298 / 248
+//   (32, 8, 7168, 1024)  32 (192): 182 / 195, 48 (224): 212 / 186, 128: 394 / 261
+//   (16, 4, 4096, 2048)  16 (160): 88 / 95, 24 (176): 116 / 100, 128: 257 / 140
+//   (32 held of 256, 8, 7168, 2048)  2: 197 / 238, 16 (320): 301 / 286, 32 (384): 340 / 326, 256: 2004 / 865
+//   (64 held of 256, 8, 4096, 1024)  16: 180 / 190, 32 (384): 210 / 190, 64: 321 / 227
 // `all`: the experts that the pairs are spread over, as routed_experts says.
-inline bool tiles_win(int64_t pairs, int64_t all, int experts, int inter)
+inline bool tiles_win(int64_t pairs, int64_t all, int experts, int inter, int dim = 7168)
 {
     const double rows  = (double)pairs / (double)all;
     const double items = (rows / kTileRowsOfExpert + 0.5) * experts * (inter / 128);
     const double least = inter <= 128 ? 80.0 : inter <= 256 ? 64.0 : inter <= 512 ? 40.0 : inter <= 1024 ? 28.0 : 24.0;
-    return rows >= least && items >= 80.0;
+    if(rows >= least && items >= 80.0)
+        return true;
+    // fewer rows where the items fill the chip and are short
+    const double filled = (items < 256.0 ? items : 256.0) / 256.0;
+    return items >= 40.0 && rows * pow(filled, 0.3) > 22.5 * sqrt((dim > 1024 ? dim : 1024) / 1024.0) * pow(128.0 / (inter < 1024 ? inter : 1024), 0.2);
 }
 
 // Second GEMM with its rows in LDS: the parts that a tile's groups of 64 columns are cut into, one item each, of which the
