@@ -1892,32 +1892,41 @@ int cols_walkers(const MoeArgs& a)
 
 } // namespace
 
-// The second GEMM's rows wait in memory for the per-token sum: in fp32 while the real rows
-// (tokens x topk) take at most 32 MiB -- the decode regime, where the bf16 rounding of rows that
-// largely cancel in the sum is avoided at no measurable cost -- and in bf16 beyond, where writing
-// them between the weight reads costs 5 % of the layer's time in fp32.
-bool moe_rows_in_f32(const MoeArgs& a) { return (size_t)a.M * a.topk * a.dim * 4 <= ((size_t)32 << 20); }
+static bool cols_fit(const MoeArgs& a)
+{
+    const int kblocks = a.inter / 128;
+    return kblocks <= 4 && (size_t)kColsTiles * kblocks * (a.M + 16) * 64 <= kColsTableBytes && a.max_blocks <= kColsMaxBlocks &&
+           a.dim % (16 * kColsTiles) == 0;
+}
+static bool few_rows(const MoeArgs& a) { return (size_t)a.M * a.topk * a.dim * 4 <= ((size_t)32 << 20); }
 
-// Decode-size batches take the second GEMM that owns output columns and sums per token in LDS
-// (moe_down_cols_kernel): its tables and its unit list have to fit the LDS.  Beyond, rows go through
-// memory and moe_combine_kernel adds them.  down_mode 1 / 2 force the one / the other (2 only where it fits).
+// Rows through memory, in fp32, where the column kernel fits but takes longer.  (With one walker, where the tables of two no
+// longer fit, it is behind anyhow: 2 % at 288-320 tokens of the DeepSeek-V3 layer.  A call that names its tiles, or rows through
+// memory, has rows in fp32 up to 32 MiB only.)  In fp32 rows are summed with one rounding less per product: against 64 bits 5.4e-8 to 6.2e-8 for topk 6 and 8 and
+// inter 128 and 256, in columns 5.8e-8 to 6.8e-8.
+static bool rows_in_place_of_columns(const MoeArgs& a)
+{
+    if(a.down_mode != 0 || !cols_fit(a) || cols_walkers(a) != 2 || (a.tiles128 == 1 && !few_rows(a)))
+        return false;
+    const int64_t pairs = (int64_t)a.M * a.topk;
+    return rows_beat_columns(pairs, routed_experts(pairs, a.topk, a.block_rows << a.expert_shift, a.max_padded, a.experts), a.experts,
+                             a.dim, a.inter);
+}
+
+// The second GEMM's rows wait in memory for the per-token sum: in fp32 while the real rows (tokens x topk) take at most 32 MiB, or
+// where they stand in for the column kernel, whose sums never leave it -- the decode regime, where the bf16 rounding of rows
+// that largely cancel in the sum is avoided at no measurable cost -- and in bf16 beyond, where writing them between the weight
+// reads costs 5 % of the layer's time in fp32.
+bool moe_rows_in_f32(const MoeArgs& a) { return few_rows(a) || rows_in_place_of_columns(a); }
+
+// Decode-size batches may take the second GEMM that owns output columns and sums per token in LDS (moe_down_cols_kernel): its
+// tables and its unit list have to fit the LDS.  Else, rows go through memory and a kernel of its own adds them.
+// down_mode 1 / 2 force the one / the other (2 only where it fits).
 bool moe_down_by_columns(const MoeArgs& a)
 {
-    const int  kblocks = a.inter / 128;
-    const bool fits    = kblocks <= 4 && (size_t)kColsTiles * kblocks * (a.M + 16) * 64 <= kColsTableBytes &&
-                      a.max_blocks <= kColsMaxBlocks && a.dim % (16 * kColsTiles) == 0;
-    if(a.down_mode == 1 || !fits)
+    if(a.down_mode == 1 || !cols_fit(a))
         return false;
-    if(a.down_mode == 2)
-        return true;
-    // with one walker (the tables of two no longer fit) 2 % slower at 288-320 tokens of the DeepSeek-V3 layer
-    if(cols_walkers(a) != 2)
-        return false;
-    // Rows that would wait in bf16 are the column kernel's as long as it fits.  In fp32 they are summed with one rounding less per
-    // product: against 64 bits 5.4e-8 to 6.2e-8 for topk 6 and 8 and inter 128 and 256, in columns 5.8e-8 to 6.8e-8.
-    const int64_t pairs = (int64_t)a.M * a.topk;
-    return !moe_rows_in_f32(a) || !rows_beat_columns(pairs, routed_experts(pairs, a.topk, a.block_rows << a.expert_shift, a.max_padded, a.experts),
-                                                     a.experts, a.dim, a.inter);
+    return a.down_mode == 2 || (cols_walkers(a) == 2 && !rows_in_place_of_columns(a));
 }
 
 template <typename T>

@@ -78,6 +78,9 @@ inline int down_col_splits(double rows_per_expert, int experts, int groups, int 
 //   (295, 128, 8, 4096, 256) 169 / 109  (18, 256, 8, 1280, 256)  48 / 38    (61, 256, 8, 3840, 256) 114 / 107
 //   (16, 256, 8, 7168, 256)  89 / 94    (128, 256, 8, 7168, 256) 199 / 213  (66, 256, 8, 4864, 256) 131 / 133
 //   (1, 256, 8, 1024, 256)   17 / 20    (3, 32, 5, 6400, 256)    24 / 26    (110, 256, 8, 5376, 256) 164 / 168
+// and whole layers, whose rows take more than 32 MiB and wait in fp32 all the same:
+//   (400, 256, 8, 2304, 128) 146 / 92   (554, 128, 8, 3840, 128) 160 / 121  (264, 256, 8, 4608, 256) 198 / 183
+//   (270, 64, 6, 7168, 256)  127 / 128
 // Measured from dim 1024 on; below, columns as long as they fit.
 inline bool rows_beat_columns(int64_t pairs, int64_t all, int experts, int dim, int inter)
 {
@@ -87,7 +90,7 @@ inline bool rows_beat_columns(int64_t pairs, int64_t all, int experts, int dim, 
     const double blocks  = experts * (1.0 - exp(-rows)) + here / 32.0; // an even routing's, of up to 32 rows each
     const double weights = dim * 25.6e-6;                              // us per block and K block, at 5 TB/s
     const double in_columns = blocks * kblocks * (weights < 0.13 ? 0.13 - weights : 0.0) + here * 0.02;
-    return in_columns > 6.5 + here * dim * 2e-6 + blocks * kblocks * weights * 0.06;
+    return in_columns > 6.5 + here * dim * 2.1e-6 + blocks * kblocks * weights * 0.06;
 }
 
 } // namespace fp8bs

@@ -613,10 +613,21 @@ def test_fmoe_few_tokens_take_columns_or_rows(tokens, dim, inter, experts, topk,
             assert torch.equal(auto.view(torch.int16), got.view(torch.int16))
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_fmoe_rows_in_place_of_columns_stay_in_fp32(dtype):
+    # 62 MB of them: in bf16 an fp16 result would be several times as far off (by name, rows beyond 32 MiB wait in bf16)
+    p = make_moe(540, 3584, 128, 64, 8, seed=540, w_std=0.05)
+    ref = reference(p, compute=torch.float64)[0].double()
+    error = {h: ((run_moe(p, dtype=dtype, bf16_input=True, kernel_name=h).cpu().double() - ref).norm() / ref.norm()).item()
+             for h in ("", "down=cols", "down=rows,tiles=0")}
+    assert error[""] < error["down=cols"] * (1 + 1e-4)
+    assert error[""] < error["down=rows,tiles=0"] * (1 if dtype == torch.bfloat16 else 0.8)
+
+
 @pytest.mark.parametrize("topk", [1, 2, 3, 5, 8, 9, 10, 11, 23])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_fmoe_sum_of_fp32_rows(topk, dtype):
-    # slots per pass: 2, 4, 6, 8 or 10, the last pass partly empty; a second pass; 288 lanes' worth of columns
+    # slots per pass: 2, 4, 6, 8 or 10, the last pass partly empty; a second pass; a second, partly empty workgroup per token
     p = make_moe(37, 1280, 128, 24, topk, seed=topk, w_std=0.05)
     assert_close(run_moe(p, dtype=dtype, kernel_name="down=rows"), reference(p), f"top-{topk}")
 
