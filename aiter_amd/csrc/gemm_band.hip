@@ -13,7 +13,7 @@
 // weights take what is left: four to six.  A wave's loads are counted in the order they were issued, so that each operand
 // has its own fetching waves (two and two) and waits for its own depth.
 //
-// Bound by, up to 64 rows, the weights (36864 x 7168: 44 us, 6.1 TB/s); beyond, by what a compute unit takes in and multiplies
+// Bound by, with few rows, the weights (64 x 36864 x 7168, were it one range: 44 us, 6.1 TB/s); beyond, by what a compute unit takes in and multiplies
 // per K block: 203 rows 71 us, 256 rows 73.  us before (192-wide tiles, mid_* tilings) / here, K in one range:
 //   203 x 36864 x 7168 92 / 71   512 x 18432 x 7168 88 / 68   1024 x 9216 x 7168 86 / 71   75 x 34496 x 1920 28 / 17
 //   86 x 35136 x 1152 20 / 13    288 x 17024 x 2816 33 / 26   2044 x 4480 x 1024 18 / 16   1439 x 5760 x 3072 34 / 28
