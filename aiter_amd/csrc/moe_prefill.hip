@@ -1,7 +1,7 @@
 // Block-scale mixture of experts, many rows per expert: the two grouped GEMMs on 128-row tiles.
 //
 // DeepSeek-V3's routed experts (256, top-8, dim 7168, inter 256), the layer on 2048 / 4096 / 8192 tokens: 563 / 958 / 1764
-// us block by block, 469 / 641 / 965 in tiles, with the same bits.
+// us block by block, 464 / 610 / 926 in tiles, with the same bits.
 //
 // The kernels of moe_kernels.hip walk the sorted rows in blocks of 32 (or pairs of them) and stream an expert's weights
 // once per block: right while the weights are what the layer reads, but with hundreds of rows per expert the same
