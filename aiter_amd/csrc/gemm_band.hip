@@ -19,6 +19,7 @@
 //   86 x 35136 x 1152 20 / 13    288 x 17024 x 2816 33 / 26   2044 x 4480 x 1024 18 / 16   1439 x 5760 x 3072 34 / 28
 // Taken out again: two stages of rows (203 x 36864 x 7168 81 us: a K block then waits for L2).
 #include "gemm_ring.h"
+#include "gemm_rules.h"
 
 #include <algorithm>
 #include <atomic>
@@ -30,7 +31,7 @@ namespace {
 
 constexpr int kMulWaves = 8, kFetchWaves = 4; // two that fetch weights, two that fetch rows and their scales
 constexpr int kBandThreads = 64 * (kMulWaves + kFetchWaves);
-constexpr int kBandRows    = 32 * kMulWaves;
+static_assert(kBandRows == 32 * kMulWaves, "32 rows per multiplying wave");
 constexpr int kXStages     = 3; // K blocks of rows in LDS
 
 struct BandLayout // LDS, in bytes
@@ -135,8 +136,6 @@ __global__ __launch_bounds__(kBandThreads) void gemm_band_kernel(GemmKernelParam
             uint32_t stage = 0;
             auto issue = [&](int kb) { // past the end the last block again, unused, so that every K block has its loads
                 const uint8_t* src = p.wq + (size_t)min(kb, n - 1) * (SHUF ? 2048 : 128);
-                // (weights that one workgroup reads, and that take more than half of the last-level cache: past the caches, which
-                // the rows then have for themselves.  64 x 36864 x 7168: 50 us, 44 this way; 203 rows 74 and 71)
                 if(lds.stream_w)
                 {
 #pragma unroll
@@ -405,7 +404,7 @@ BandLayout band_layout(const GemmKernelParams& p, int nf, bool xs4)
     l.w_at     = kXStages * l.rows * 128;
     l.xs_at    = l.w_at + l.w_stages * stage;
     l.total    = std::max(l.xs_at + scales, kMulWaves * 32 * (16 * nf * 2 + 16));
-    l.stream_w = p.M <= kBandRows && (int64_t)p.N * p.K >= (int64_t)128 << 20;
+    l.stream_w = gemm_band_streams_weights(p.M, p.N, p.K);
     return l;
 }
 
@@ -418,25 +417,6 @@ auto band_kernel(bool shuffled, bool xs4, bool bf)
 }
 
 } // namespace
-
-// 144 where tiles of 128 rows take a second round of workgroups and these do not: ahead in all 10 of 70 drawn sizes, by 12 %
-// (2044 x 4480 x 1024) to 38 % (75 x 34496 x 1920); where 128 fit one round as well, up to 24 % behind gemm_ring.hip's.  From
-// 65 rows on: up to 64, one row of 64 x 64 tiles, two of them on a compute unit, reads the weights once as well
-// (34 x 32960 x 512: 7.8 us there, 9.1 here).
-// 96 for up to 256 rows and 40 K blocks or more where that covers two thirds of the chip, in place of tilings that read
-// the weights more than once or cover less of it: 68 x 21632 x 5760 30.3 / 28.6 us, 151 x 17984 x 5504 41.4 / 37.4,
-// 130 x 20480 x 6144 43.3 / 38.7, 100 x 24576 x 7168 44.9 / 39.4; with fewer K blocks 110 x 17984 x 2432 13.8 / 15.0, 256 x 16512 x
-// 2560 19.0 / 22.0, on less of the chip 37 x 14464 x 2688 (151 workgroups) 11.2 / 13.7, for more rows 392 x 7872 x 6272 31 / 38.
-int gemm_band_rows(const GemmKernelParams& p, int cus)
-{
-    const int64_t tiles_m = (p.M + kBandRows - 1) / kBandRows;
-    auto tiles = [&](int rows) { return tiles_m * ((p.N + rows - 1) / rows); };
-    if(p.M > 64 && tiles(128) > cus && tiles(144) <= cus)
-        return 144;
-    if(tiles_m == 1 && p.kblocks >= 40 && tiles(96) <= cus && tiles(96) * 3 >= cus * 2)
-        return 96;
-    return 0;
-}
 
 // band: 96 or 144 weight rows per workgroup.  Operands as gemm_prefill_supports says.
 hipError_t launch_gemm_band(const GemmKernelParams& p, In16 out_dtype, const LaunchCtx& ctx, int band)

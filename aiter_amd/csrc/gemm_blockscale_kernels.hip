@@ -13,6 +13,7 @@
 // one scalar per lane, xs[m,kb]*ws[nb,kb], and (b) its output 4 consecutive 16-bit values.
 #include "fp8bs_launch.h"
 #include "gemm_common.h"
+#include "gemm_rules.h"
 #include <cstdio>
 #include <cstdlib>
 
@@ -299,7 +300,7 @@ static hipError_t dispatch(const GemmArgs& a, const GemmKernelParams& p, hipStre
     ctx.why         = why;
     ctx.static_only = a.static_scratch;
     // bands of weight rows in place of what was chosen here with K in one range: the same sums
-    const int band = gemm_prefill_supports(p) ? gemm_band_rows(p, 256) : 0;
+    const int band = gemm_prefill_supports(p) ? gemm_band_rows(p.M, p.N, p.K, k.family == Family::prefill && k.tile == 192, 256) : 0;
     switch(k.family)
     {
     case Family::tile:

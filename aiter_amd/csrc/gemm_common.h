@@ -100,8 +100,6 @@ hipError_t launch_gemm_prefill(const GemmKernelParams& p, In16 out_dtype, const 
                                int want_tile_n = 0);
 bool       gemm_prefill_supports(const GemmKernelParams& p);
 hipError_t launch_gemm_ring(const GemmKernelParams& p, In16 out_dtype, const LaunchCtx& ctx, int kb_per_range, int device, int cus);
-// gemm_band.hip: the rows of weights per workgroup with which it carries out a plan of one K range, 0 where it does not
-int        gemm_band_rows(const GemmKernelParams& p, int cus);
 hipError_t launch_gemm_band(const GemmKernelParams& p, In16 out_dtype, const LaunchCtx& ctx, int band);
 hipError_t launch_gemm_decode(const GemmKernelParams& p, In16 out_dtype, int split_k_log2, const LaunchCtx& ctx,
                               const char* tuning = nullptr);

@@ -81,3 +81,15 @@ def test_choice_below_65_rows_against_measured_durations():
         if r[other] > 1.25 * r[chosen] or r[chosen] > 1.25 * r[other]:
             assert r[chosen] < r[other], (r, chosen)
     assert sum(losses) / len(losses) <= 0.01, sum(losses) / len(losses)
+
+
+def test_where_bands_of_weight_rows_take_over(tmp_path):
+    """The edges of the rule by which bands of 96 and 144 weight rows carry out a plan of one K range:
+    aiter_amd/csrc/gemm_rules.h on the host."""
+    import subprocess
+
+    exe = str(tmp_path / "gemm_rules_check")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-o", exe,
+                           os.path.join(os.path.dirname(os.path.abspath(__file__)), "host_math", "gemm_rules_check.cpp")])
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0 and out.stdout.startswith("OK"), out.stdout + out.stderr
