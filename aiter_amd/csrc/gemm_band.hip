@@ -1,8 +1,8 @@
 // Block-scale FP8 GEMM, up to 256 activation rows by a band of 96 or 144 weight rows per workgroup: one round of workgroups
 // that covers the chip where 128-row tiles do not, with the weights requested several K blocks further ahead than the rows.
 //
-// Carries out, where it is faster, what was chosen for other kernels with K in one range; the additions are the same, so the
-// bits are too.
+// Carries out, where it is faster (gemm_rules.h), what was chosen for other kernels with K in one range; the additions are the same,
+// so the bits are too.  By name it takes any size that the prefill_* kernels take.
 //
 // Why bands of 144.  With 256 rows of weights per workgroup 36864 of them are 144 workgroups, with 192 they are 192, with 128
 // a round and a fragment of one; with 144 they are 256, and a workgroup's K block is 18 KiB of weights beside the rows'.

@@ -164,7 +164,7 @@ static hipError_t launch_tile(const GemmKernelParams& p, hipStream_t stream)
 
 static const char* const kKernelNames =
     "tile_16x256,tile_64x128,tile_128x128,mid_64x64,mid_64x128,mid_128x128,prefill_256x256,prefill_256x192,prefill_256x128,"
-    "decode_stream";
+    "band_256x144,band_256x96,decode_stream";
 
 const char* gemm_kernel_names() { return kKernelNames; }
 
@@ -184,7 +184,7 @@ const char* gemm_kernel_names() { return kKernelNames; }
 // That decides the K ranges, and with them the bits.  Where it means one range, one round of the 256 x 128 tiles of
 // gemm_ring.hip takes the place of mid_* tilings that are modelled no faster: the same sums (425 x 8896 x 2816: 31 us there, 20
 // here; 5712 x 704 x 3584: 37 and 23).
-static const char* automatic_choice(const GemmKernelParams& p)
+static const char* choice_of_ranges(const GemmKernelParams& p)
 {
     const PrefillPlan plan = gemm_prefill_plan(p, 256); // fitted on a 256-CU part, like the mid model
     if(p.M <= 64 && gemm_decode_supports(p) && (!gemm_mid_supports(p) || gemm_mid_estimate_us(p) >= gemm_decode_estimate_us(p)))
@@ -198,6 +198,23 @@ static const char* automatic_choice(const GemmKernelParams& p)
     if(gemm_prefill_supports(p))
         return plan.tile_n == 128 ? "prefill_256x128" : plan.tile_n == 192 ? "prefill_256x192" : "prefill_256x256";
     return "tile_128x128";
+}
+
+// ... and where that is one range, bands of weight rows take over: the same sums.  split_k_log2: the caller's K ranges, -1 for none;
+// mid_* tilings heed them, the prefill_* ones and bands do not.
+static const char* automatic_choice(const GemmKernelParams& p, int split_k_log2)
+{
+    const char* const name = choice_of_ranges(p);
+    const bool        mid  = strcmp(name, "mid_auto") == 0;
+    if(!gemm_prefill_supports(p) || (!mid && strncmp(name, "prefill_", 8) != 0))
+        return name;
+    const int band = gemm_band_rows(p.M, p.N, p.K, strcmp(name, "prefill_256x192") == 0, 256);
+    if(!band)
+        return name;
+    // (256 x 128 tiles may stand for a plan of another family, and are one range in any case)
+    const bool one_range = mid ? split_k_log2 < 0 && gemm_mid_ranges(p) == 1
+                               : strcmp(name, "prefill_256x128") == 0 || gemm_prefill_plan(p, 256).splits == 1;
+    return !one_range ? name : band == 144 ? "band_256x144" : "band_256x96";
 }
 
 // Names of the reference's own kernel zoo ("a8w8_blockscale_1x128x128_256x16x128x256_..."), as
@@ -222,8 +239,9 @@ static KernelRequest resolve_request(const GemmArgs& a, const GemmKernelParams& 
     const bool named = a.kernel_name && a.kernel_name[0] && !foreign_kernel_name(a.kernel_name);
     if(named)
         return KernelRequest{a.kernel_name, a.split_k_log2};
-    const bool foreign = a.kernel_name && a.kernel_name[0];
-    return KernelRequest{automatic_choice(p), (foreign || a.split_k_log2 <= 0) ? -1 : a.split_k_log2};
+    const bool foreign      = a.kernel_name && a.kernel_name[0];
+    const int  split_k_log2 = (foreign || a.split_k_log2 <= 0) ? -1 : a.split_k_log2;
+    return KernelRequest{automatic_choice(p, split_k_log2), split_k_log2};
 }
 
 // One of this library's kernel names, taken apart.
@@ -232,12 +250,13 @@ enum class Family
     tile,
     decode,
     mid,
-    prefill
+    prefill,
+    band
 };
 struct ParsedKernel
 {
     Family      family;
-    int         tile;   // tile: 16256 / 64128 / 128128; mid: 0 (choose) / 64 / 64128 / 128
+    int         tile;   // tile: 16256 / 64128 / 128128; mid: 0 (choose) / 64 / 64128 / 128; prefill, band: weight rows
     int         splits; // ":s=<n>" of mid_* and prefill_*, 0 when absent
     const char* tuning; // what follows "decode_stream:", or null
 };
@@ -256,6 +275,12 @@ static bool parse_kernel_name(const char* name, ParsedKernel* out)
     {
         out->family = Family::decode;
         out->tuning = name[13] == ':' ? name + 14 : nullptr;
+        return true;
+    }
+    if(strcmp(name, "band_256x144") == 0 || strcmp(name, "band_256x96") == 0)
+    {
+        out->family = Family::band;
+        out->tile   = name[9] == '1' ? 144 : 96;
         return true;
     }
     const char*  colon = strchr(name, ':');
@@ -299,8 +324,6 @@ static hipError_t dispatch(const GemmArgs& a, const GemmKernelParams& p, hipStre
     ctx.stream      = stream;
     ctx.why         = why;
     ctx.static_only = a.static_scratch;
-    // bands of weight rows in place of what was chosen here with K in one range: the same sums
-    const int band = gemm_prefill_supports(p) ? gemm_band_rows(p.M, p.N, p.K, k.family == Family::prefill && k.tile == 192, 256) : 0;
     switch(k.family)
     {
     case Family::tile:
@@ -323,8 +346,6 @@ static hipError_t dispatch(const GemmArgs& a, const GemmKernelParams& p, hipStre
             *why = "the mid_* kernels need operand matrices below 4 GiB";
             return hipErrorInvalidValue;
         }
-        if(!named && req.split_k_log2 < 0 && band && gemm_mid_ranges(p) == 1)
-            return launch_gemm_band(p, DT, ctx, band);
         return launch_gemm_mid(p, DT, req.split_k_log2, ctx, k.tile, k.splits);
     case Family::prefill:
         if(!gemm_prefill_supports(p))
@@ -336,9 +357,15 @@ static hipError_t dispatch(const GemmArgs& a, const GemmKernelParams& p, hipStre
         // unless ":s=" pins the K ranges per tile; chosen automatically, the launcher decides -- but for
         // 256 x 128 tiles, which may stand for a plan of another family.
         // splitK is a hint this kernel has no use for.
-        if(!named && band && (k.tile == 128 || gemm_prefill_plan(p, 256).splits == 1))
-            return launch_gemm_band(p, DT, ctx, band);
         return launch_gemm_prefill(p, DT, ctx, k.splits > 0 ? k.splits : (named ? 1 : 0), named || k.tile == 128 ? k.tile : 0);
+    case Family::band:
+        // (a tile's K in one workgroup, as the tile_* kernels: splitK is a hint these have no use for)
+        if(!gemm_prefill_supports(p))
+        {
+            *why = "the band_* kernels need N % 4 == 0 and operand matrices below 4 GiB";
+            return hipErrorInvalidValue;
+        }
+        return launch_gemm_band(p, DT, ctx, k.tile);
     }
     *why = kUnknownName;
     return hipErrorInvalidValue;
@@ -368,7 +395,7 @@ hipError_t launch_gemm_blockscale(const GemmArgs& a, hipStream_t stream, const c
                                      : dispatch<In16::fp16>(a, p, stream, why);
 }
 
-void gemm_describe_choice(int64_t M, int64_t N, int64_t K, bool shuffled, char* buf, size_t n)
+static GemmKernelParams contiguous_problem(int64_t M, int64_t N, int64_t K, bool shuffled)
 {
     GemmKernelParams p{};
     p.M          = (int32_t)M;
@@ -378,7 +405,12 @@ void gemm_describe_choice(int64_t M, int64_t N, int64_t K, bool shuffled, char* 
     p.ldb        = K;
     p.kblocks    = (int32_t)(K / 128);
     p.w_shuffled = shuffled ? 1 : 0;
-    const char* name = automatic_choice(p);
+    return p;
+}
+
+// `name`, as automatic_choice has it, with the tiling and the K ranges that it means
+static void describe(const GemmKernelParams& p, const char* name, char* buf, size_t n)
+{
     if(strcmp(name, "mid_auto") == 0)
         gemm_mid_describe(p, buf, n);
     else
@@ -391,21 +423,20 @@ void gemm_describe_choice(int64_t M, int64_t N, int64_t K, bool shuffled, char* 
     }
 }
 
+void gemm_describe_choice(int64_t M, int64_t N, int64_t K, bool shuffled, char* buf, size_t n)
+{
+    const GemmKernelParams p = contiguous_problem(M, N, K, shuffled);
+    describe(p, automatic_choice(p, -1), buf, n);
+}
+
 // "<kernel>;splitK=<n>": what the pair (kernelName, splitK) of a call resolves to for contiguous
 // operands of this shape (n = -1: the kernel chooses its K ranges).  False with *why set when the
 // name is neither one of this library's nor one of the reference's zoo.
 bool gemm_describe_request(int64_t M, int64_t N, int64_t K, bool shuffled, int split_k_log2, const char* kernel_name,
                            char* buf, size_t n, const char** why)
 {
-    GemmKernelParams p{};
-    p.M          = (int32_t)M;
-    p.N          = (int32_t)N;
-    p.K          = (int32_t)K;
-    p.lda        = K;
-    p.ldb        = K;
-    p.kblocks    = (int32_t)(K / 128);
-    p.w_shuffled = shuffled ? 1 : 0;
-    GemmArgs a{};
+    const GemmKernelParams p = contiguous_problem(M, N, K, shuffled);
+    GemmArgs               a{};
     a.kernel_name        = kernel_name;
     a.split_k_log2       = split_k_log2;
     const KernelRequest r = resolve_request(a, p);
@@ -418,7 +449,7 @@ bool gemm_describe_request(int64_t M, int64_t N, int64_t K, bool shuffled, int s
     if(r.name != kernel_name) // chosen here: say which tiling and K ranges the choice means
     {
         char chosen[48];
-        gemm_describe_choice(M, N, K, shuffled, chosen, sizeof chosen);
+        describe(p, r.name, chosen, sizeof chosen);
         if(r.split_k_log2 >= 0) // the caller's ranges replace the choice's
             if(char* colon = strchr(chosen, ':'))
                 *colon = 0;

@@ -443,13 +443,14 @@ def test_narrow_prefill_tiles_as_the_library_chooses_them(m, n, k, expect):
     (1000, 9216, 512),    # four
     (2044, 4480, 8320),   # eight; 65 K blocks: past one window of w_scale
     (150, 16512, 5120),   # bands of 96: 172 workgroups, 40 K blocks
-    (33, 24576, 5248),    # 41: odd; 128 MiB of weights, past the caches; two of the eight waves have rows
-    (100, 24572, 5632),
+    (33, 24576, 5248),    # 41: odd; two of the eight waves have rows
+    (100, 24572, 5632),   # more than 128 MiB of weights, past the caches
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_bands_of_weight_rows_carry_out_plans_of_one_range(m, n, k, dtype):
     # what the library chooses, against the kernel that keeps a tile's K in one workgroup: the same products in the same order
     assert ":s=" not in _ffi.gemm_choice(m, n, k) or _ffi.gemm_choice(m, n, k).endswith(":s=1")
+    assert _ffi.gemm_choice(m, n, k) == ("band_256x96" if k >= 5120 and k != 7168 and m < 256 else "band_256x144")
     xq, wq, xs, ws = _gpu_problem(m, n, k, seed=m + n + k, outliers=True)
     tile = torch.empty(m, n, dtype=dtype, device=DEV)
     aiter_amd.gemm_a8w8_blockscale_ck(xq, wq, xs, ws, tile, kernelName="tile_128x128")
@@ -463,6 +464,44 @@ def test_bands_of_weight_rows_carry_out_plans_of_one_range(m, n, k, dtype):
         aiter_amd.gemm_a8w8_blockscale_bpreshuffle_ck(xq, wsh, xs.t().contiguous().view(*xs.shape), ws, out)
         torch.cuda.synchronize()
         assert torch.equal(out.view(torch.int16), tile.view(torch.int16))
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 16, 128),       # one row, less than a band
+    (16, 288, 384),     # whole bands of either width
+    (17, 148, 640),     # a second band of 4 or 52 columns; a row in the second fragment
+    (31, 1744, 1152),   # nine K blocks: scales one by one
+    (240, 432, 1024),   # eight: in windows of four; the fewest stages of weights
+    (257, 304, 256),    # a second tile of one row
+    (700, 592, 8320),   # three tiles of rows; 65 K blocks: past one window of w_scale
+])
+@pytest.mark.parametrize("band", ["band_256x144", "band_256x96"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_bands_by_name(m, n, k, band, dtype):
+    # any size, whatever the library would choose; splitK is a hint that they ignore
+    xq, wq, xs, ws = _gpu_problem(m, n, k, seed=m + n + k, outliers=True)
+    tile = torch.empty(m, n, dtype=dtype, device=DEV)
+    aiter_amd.gemm_a8w8_blockscale_ck(xq, wq, xs, ws, tile, kernelName="tile_128x128")
+    out = torch.full((m, n), float("nan"), dtype=dtype, device=DEV)
+    for split in (-1, 0, 2):
+        out.fill_(float("nan"))
+        aiter_amd.gemm_a8w8_blockscale_ck(xq, wq, xs, ws, out, splitK=split, kernelName=band)
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), tile.view(torch.int16))
+    if n % 16 == 0:
+        wsh = aiter_amd.shuffle_weight(wq.view(torch.uint8)).view(wq.dtype)
+        out.fill_(float("nan"))
+        aiter_amd.gemm_a8w8_blockscale_bpreshuffle_ck(xq, wsh, xs.t().contiguous().view(*xs.shape), ws, out, band)
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), tile.view(torch.int16))
+
+
+def test_bands_by_name_reject_what_they_cannot_do():
+    with pytest.raises(RuntimeError, match="band_.*N % 4"):
+        run_gpu(*make_problem(16, 255, 256), kernel="band_256x144")
+    for name in ("band_256x144:s=2", "band_256x128", "band_"):
+        with pytest.raises(RuntimeError, match="unknown kernelName"):
+            run_gpu(*make_problem(128, 256, 256), kernel=name)
 
 
 @pytest.mark.parametrize("m,n,k", [(4352, 4096, 256), (4352, 4352, 128), (4100, 4360, 256)])

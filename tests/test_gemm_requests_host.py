@@ -93,3 +93,23 @@ def test_where_bands_of_weight_rows_take_over(tmp_path):
                            os.path.join(os.path.dirname(os.path.abspath(__file__)), "host_math", "gemm_rules_check.cpp")])
     out = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0 and out.stdout.startswith("OK"), out.stdout + out.stderr
+
+
+@pytest.mark.parametrize("m,n,k,expect", [
+    (203, 36864, 7168, "band_256x144"),      # in place of 256 x 192 tiles
+    (70, 32784, 384, "band_256x144"),        # of mid_* tilings with K in one range
+    (4096, 2112, 7168, "band_256x144"),
+    (150, 16512, 5120, "band_256x96"),       # of 256 x 128 tiles
+    (12, 24576, 7168, "band_256x96"),
+    (4096, 2112, 1024, "prefill_256x192"),   # left to what was there
+    (256, 16384, 8064, "mid_128x128:s=1"),
+    (8, 22480, 5248, "mid_64x128:s=1"),
+    (2048, 4096, 7168, "prefill_256x256:s=2"),
+])
+def test_choice_names_the_bands_that_run(m, n, k, expect):
+    # what a call without a name launches is decided by the name that is reported here
+    assert _ffi.gemm_choice(m, n, k) == expect and _ffi.gemm_choice(m, n, k, n % 16 == 0) == expect
+    assert _ffi.gemm_resolve(m, n, k, -1, "") == (expect, -1) and _ffi.gemm_resolve(m, n, k, 0, expect) == (expect, 0)
+    # K ranges that a caller asks for keep the mid_* tilings, which heed them
+    if (m, n) in ((70, 32784), (12, 24576)):
+        assert _ffi.gemm_resolve(m, n, k, 2, "")[0].startswith("mid_")
