@@ -36,8 +36,16 @@ inline int64_t routed_experts(int64_t pairs, int topk, int unit, int64_t padded,
 //   (16, 4, 4096, 2048)  16 (160): 88 / 95, 24 (176): 116 / 100, 128: 257 / 140
 //   (32 held of 256, 8, 7168, 2048)  2: 197 / 238, 16 (320): 301 / 286, 32 (384): 340 / 326, 256: 2004 / 865
 //   (64 held of 256, 8, 4096, 1024)  16: 180 / 190, 32 (384): 210 / 190, 64: 321 / 227
+// Below 48 items the line depends on how full the tiles are: an expert with a hundred rows or fewer has one ragged tile, and a chip
+// that is a sixth full waits for the longest of them.  Time block by block over time in tiles, fewer than 112 rows: (322, 12
+// experts, top-3, 6144, 384; 40 items) 0.84, (415, 16, 4, 4096, 256; 41) 0.92, (432, 8, 2, 3840, 512; 43) 0.92, (355, 24, 4, 2816, 256; 46)
+// 0.96, (430, 12, 3, 4096, 384; 48) 1.10; more: (604, 12, 3, 2816, 256; 40) 0.94, (638, 12, 3, 6912, 256; 41) 1.10, (474, 16, 4, 5120, 256;
+// 45) 1.17, (2362, 8, 2, 6144, 128; 40) 1.23.
+// Three K blocks of the second GEMM (inter 384) take the ring there, and with 0.8 to 1.25 rounds of items need more rows to make up for
+// it: (608, 96, 6, 4096; 229 items) 0.87, (618, 128, 8, 4096; 308) 0.94, (476, 112, 8, 3072; 257) 0.96, (380, 80, 8, 3072; 191) 1.21.
+// (The average over 211 layers is from before these two.)
 // `all`: the experts that the pairs are spread over, as routed_experts says.
-inline bool tiles_win(int64_t pairs, int64_t all, int experts, int inter, int dim = 7168)
+inline bool tiles_win(int64_t pairs, int64_t all, int experts, int inter, int dim)
 {
     const double rows  = (double)pairs / (double)all;
     const double items = (rows / kTileRowsOfExpert + 0.5) * experts * (inter / 128);
@@ -46,7 +54,10 @@ inline bool tiles_win(int64_t pairs, int64_t all, int experts, int inter, int di
         return true;
     // fewer rows where the items fill the chip and are short
     const double filled = (items < 256.0 ? items : 256.0) / 256.0;
-    return items >= 40.0 && rows * pow(filled, 0.3) > 22.5 * sqrt((dim > 1024 ? dim : 1024) / 1024.0) * pow(128.0 / (inter < 1024 ? inter : 1024), 0.2);
+    const double fewest = rows >= 256.0 ? 40.0 : rows >= 112.0 ? 41.0 : 48.0;
+    const double ring   = inter == 384 && items > 205.0 && items < 320.0 ? 1.2 : 1.0;
+    return items >= fewest &&
+           rows * pow(filled, 0.3) > 22.5 * ring * sqrt((dim > 1024 ? dim : 1024) / 1024.0) * pow(128.0 / (inter < 1024 ? inter : 1024), 0.2);
 }
 
 // Second GEMM with its rows in LDS: the parts that a tile's groups of 64 columns are cut into, one item each, of which the

@@ -17,6 +17,9 @@
 
 using namespace fp8bs;
 
+// a layer of the widest dim that was measured
+static bool tiles_win(int64_t pairs, int64_t all, int held, int inter) { return fp8bs::tiles_win(pairs, all, held, inter, 7168); }
+
 // slots as the sort's arrays are sized, in whole blocks
 static int64_t padded(int64_t pairs, int topk, int unit, int all) { return (pairs + (int64_t)all * unit - topk) / unit * unit; }
 
@@ -60,6 +63,28 @@ int main()
     EXPECT(rows_beat_columns(140 * 6, 64, 64, 1536, 128) && !rows_beat_columns(140 * 6, 64, 64, 512, 128));
     EXPECT(!rows_beat_columns(16 * 8, 256, 256, 7168, 256) && !rows_beat_columns(128 * 8, 256, 256, 7168, 256));
     EXPECT(!rows_beat_columns(5, 32, 32, 1024, 256) && !rows_beat_columns(140 * 6, 64, 4, 1536, 128));
+    // Tiles on both sides of where they were measured to win: (rows per expert, experts, dim, inter)
+    auto tiles = [](int rows, int experts, int dim, int inter) { return fp8bs::tiles_win((int64_t)rows * experts, experts, experts, inter, dim); };
+    struct
+    {
+        int experts, dim, inter, no, yes;
+    } const lines[] = {
+        {256, 3072, 128, 40, 56},  {256, 7168, 256, 40, 52},  {128, 7168, 256, 48, 56},  {32, 4096, 256, 48, 64}, {8, 1024, 256, 240, 384},
+        {256, 2048, 512, 22, 32},  {16, 4096, 2048, 12, 24},  {64, 1536, 256, 26, 49},   {128, 1280, 128, 24, 36}, {64, 1024, 384, 18, 25},
+        {32, 7168, 1024, 24, 48},  {128, 4096, 384, 38, 40},  {96, 4096, 384, 38, 40},   {80, 3072, 384, 34, 38},
+        {16, 4096, 256, 104, 118}, {8, 3840, 512, 108, 117},  {12, 6144, 384, 95, 112},  {24, 2304, 256, 59, 64},  {8, 6144, 128, 560, 580},
+    };
+    for(auto& l : lines)
+    {
+        m = l.dim, e = l.experts;
+        EXPECT(!tiles(l.no, l.experts, l.dim, l.inter) && tiles(l.yes, l.experts, l.dim, l.inter));
+    }
+    // a narrower layer takes tiles from no more rows than a wide one
+    for(int inter : {128, 256, 512, 1024})
+        for(e = 8; e <= 256; e *= 2)
+            for(int rows = 8; rows <= 1024; rows += 8)
+                for(m = 1024; m < 7168; m += 512)
+                    EXPECT(tiles(rows, e, m, inter) || !tiles(rows, e, m + 512, inter));
     std::printf("OK\n");
     return 0;
 }
