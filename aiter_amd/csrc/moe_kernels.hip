@@ -1892,6 +1892,28 @@ int cols_walkers(const MoeArgs& a)
 
 } // namespace
 
+// floats per sorted row in the buffer the quantiser writes its scales to: a row record while the
+// second GEMM's K has at most four scale blocks, the bare scales beyond
+size_t scale_floats_per_slot(const MoeArgs& a) { return a.inter / 128 <= 4 ? (size_t)kRowInfo : (size_t)(a.inter / 128); }
+
+static size_t block_wise_workspace_bytes(const MoeArgs& a, bool rows_in_f32)
+{
+    const size_t slots = (size_t)a.max_padded;
+    size_t       b     = 0;
+    b += align_up(slots * a.inter * 2);          // activation product, bf16
+    b += align_up(slots * a.inter);              // the same as fp8
+    b += align_up(slots * scale_floats_per_slot(a) * 4); // its scales, or the row records that hold them
+    b += align_up(slots * a.dim * (rows_in_f32 ? 4 : 2)); // second GEMM's rows
+    b += align_up((size_t)a.M * a.topk * 4);     // sorted position of each (token, slot)
+    b += align_up((size_t)a.max_blocks * 4);     // real rows of each block
+    if(a.x16)
+    {
+        b += align_up((size_t)a.M * a.dim);             // quantised tokens
+        b += align_up((size_t)a.M * (a.dim / 128) * 4); // their scales
+    }
+    return b;
+}
+
 static bool cols_fit(const MoeArgs& a)
 {
     const int kblocks = a.inter / 128;
@@ -1904,9 +1926,13 @@ static bool few_rows(const MoeArgs& a) { return (size_t)a.M * a.topk * a.dim * 4
 // longer fit, it is behind anyhow: 2 % at 288-320 tokens of the DeepSeek-V3 layer.  A call that names its tiles, or rows through
 // memory, has rows in fp32 up to 32 MiB only.)  In fp32 rows are summed with one rounding less per product: against 64 bits 5.4e-8 to 6.2e-8 for topk 6 and 8 and
 // inter 128 and 256, in columns 5.8e-8 to 6.8e-8.
+// Columns stay where fp32 rows would take more scratch than a call can be recorded with (dim from 8192 on, and thousands of slots of
+// padding from sorting in blocks of 64 or 128; 513 tokens, 160 experts, top-24, 8960 x 128 in blocks of 128: 1.1 GiB, 406 us against 526).
 static bool rows_in_place_of_columns(const MoeArgs& a)
 {
     if(a.down_mode != 0 || !cols_fit(a) || cols_walkers(a) != 2 || (a.tiles128 == 1 && !few_rows(a)))
+        return false;
+    if(!few_rows(a) && std::max(block_wise_workspace_bytes(a, true), moe_prefill_workspace_bytes(a, true)) > kMaxCapturedLayerBytes)
         return false;
     const int64_t pairs = (int64_t)a.M * a.topk;
     return rows_beat_columns(pairs, routed_experts(pairs, a.topk, a.block_rows << a.expert_shift, a.max_padded, a.experts), a.experts,
@@ -2020,28 +2046,9 @@ hipError_t launch_moe_sorting(const MoeSortArgs& a, hipStream_t stream, const ch
     return hipGetLastError();
 }
 
-// floats per sorted row in the buffer the quantiser writes its scales to: a row record while the
-// second GEMM's K has at most four scale blocks, the bare scales beyond
-size_t scale_floats_per_slot(const MoeArgs& a) { return a.inter / 128 <= 4 ? (size_t)kRowInfo : (size_t)(a.inter / 128); }
-
 size_t moe_workspace_bytes(const MoeArgs& a)
 {
-    const size_t slots = (size_t)a.max_padded;
-    size_t       b     = 0;
-    if(moe_prefill_wanted(a))
-        return moe_prefill_workspace_bytes(a);
-    b += align_up(slots * a.inter * 2);          // activation product, bf16
-    b += align_up(slots * a.inter);              // the same as fp8
-    b += align_up(slots * scale_floats_per_slot(a) * 4); // its scales, or the row records that hold them
-    b += align_up(slots * a.dim * (moe_rows_in_f32(a) ? 4 : 2)); // second GEMM's rows
-    b += align_up((size_t)a.M * a.topk * 4);     // sorted position of each (token, slot)
-    b += align_up((size_t)a.max_blocks * 4);     // real rows of each block
-    if(a.x16)
-    {
-        b += align_up((size_t)a.M * a.dim);             // quantised tokens
-        b += align_up((size_t)a.M * (a.dim / 128) * 4); // their scales
-    }
-    return b;
+    return moe_prefill_wanted(a) ? moe_prefill_workspace_bytes(a, moe_rows_in_f32(a)) : block_wise_workspace_bytes(a, moe_rows_in_f32(a));
 }
 
 template <In16 DT, bool STREAM>

@@ -86,7 +86,7 @@ bool moe_down_by_columns(const MoeArgs& a);
 // moe_prefill.hip: whether this call takes its kernels, their scratch, and the launches up to the second GEMM's rows
 // (by sorted slot, bf16 or fp32 as moe_rows_in_f32 says) and the sorted position of each (token, slot) pair
 bool       moe_prefill_wanted(const MoeArgs& a);
-size_t     moe_prefill_workspace_bytes(const MoeArgs& a);
+size_t     moe_prefill_workspace_bytes(const MoeArgs& a, bool rows_in_f32);
 hipError_t launch_moe_prefill_gemms(const MoeArgs& a, hipStream_t stream, void* scratch, void** rows, int32_t** where);
 
 hipError_t launch_fmoe_blockscale(const MoeArgs& a, hipStream_t stream, const char** why);

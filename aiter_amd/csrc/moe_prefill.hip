@@ -835,10 +835,10 @@ bool moe_prefill_wanted(const MoeArgs& a)
     return tiles_win(pairs, all, a.experts, a.inter, a.dim);
 }
 
-size_t moe_prefill_workspace_bytes(const MoeArgs& a)
+size_t moe_prefill_workspace_bytes(const MoeArgs& a, bool rows_in_f32)
 {
     const size_t slots = (size_t)a.max_padded;
-    size_t       b     = align_up(slots * a.inter) + align_up(slots * row_floats(a.inter / 128) * 4) + align_up(slots * a.dim * (moe_rows_in_f32(a) ? 4 : 2)) +
+    size_t       b     = align_up(slots * a.inter) + align_up(slots * row_floats(a.inter / 128) * 4) + align_up(slots * a.dim * (rows_in_f32 ? 4 : 2)) +
                align_up((size_t)a.M * a.topk * 4) + tiles_bytes(a) + align_up((size_t)a.M * row_floats(a.dim / 128) * 4);
     if(a.x16)
         b += align_up((size_t)a.M * a.dim) + align_up((size_t)a.M * (a.dim / 128) * 4);

@@ -48,6 +48,9 @@ enum class WsKind : int
 constexpr size_t kStaticPartialBytes = (size_t)32 << 20;
 constexpr size_t kStaticTickets      = (size_t)1 << 20; // 32-bit words: 4 MiB
 
+// the largest expert-layer scratch that the graph scratch keeps up with: a call that needs more cannot be recorded
+constexpr size_t kMaxCapturedLayerBytes = (size_t)1 << 30;
+
 // What a launcher needs to know about the call it serves besides the operands.
 struct LaunchCtx
 {

@@ -45,7 +45,7 @@ constexpr size_t kMaxBytes[(int)WsKind::kinds] = {(size_t)2 << 30, (size_t)64 <<
 // largest eager request for which the capture arena is kept in step (graphs record decode-sized
 // calls; a prefill-sized expert layer would pin gigabytes twice)
 constexpr size_t kMaxCaptureBytes[(int)WsKind::kinds] = {(size_t)256 << 20, (size_t)64 << 20, (size_t)64 << 20,
-                                                         (size_t)1 << 30};
+                                                         kMaxCapturedLayerBytes};
 
 __global__ void __launch_bounds__(256) workspace_fill_zero_kernel(uint4* dst, size_t vecs)
 {

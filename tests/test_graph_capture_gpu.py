@@ -128,3 +128,36 @@ def test_moe_with_many_rows_per_expert_under_graph_replay(tokens, dim, inter, ex
         return [tw, ti, out]
 
     replay_and_compare(build, refill, run)
+
+
+def test_moe_sorted_in_long_blocks_under_graph_replay():
+    # 32 thousand slots of a wide layer, most of them padding: rows in 16 bits are below the 1 GiB of expert scratch up to which a call can be
+    # recorded, rows in fp32 would be above
+    tokens, dim, inter, experts, topk, block = 513, 8960, 128, 128, 32, 128
+    slots = tokens * topk + experts * block - topk
+    assert slots * dim * 2 < 1 << 30 < slots * dim * 4
+    g = torch.Generator(device=DEV).manual_seed(7)
+    weights = []
+    for rows, cols in ((2 * inter, dim), (dim, inter)):
+        w = (torch.randn(experts * rows, cols, generator=g, device=DEV) * 0.1).bfloat16()
+        q, s = aiter_amd.weight_per_128x128_quant(w)
+        weights.append(aiter_amd.shuffle_weight(q.view(experts, rows, cols).view(torch.uint8)).view(dtypes.fp8))
+        weights.append(s.view(experts, -1).contiguous())
+    w1, s1, w2, s2 = weights
+
+    def build():
+        return dict(x=torch.empty(tokens, dim, device=DEV, dtype=torch.bfloat16),
+                    score=torch.empty(tokens, experts, device=DEV))
+
+    def refill(t, i):
+        gg = torch.Generator(device=DEV).manual_seed(400 + i)
+        t["x"].copy_(torch.randn(tokens, dim, generator=gg, device=DEV).bfloat16())
+        t["score"].copy_(torch.randn(tokens, experts, generator=gg, device=DEV))
+
+    def run(t):
+        tw, ti = aiter_amd.fused_topk(t["x"], t["score"], topk, True)
+        s_ids, s_w, s_e, nv, out = aiter_amd.moe_sorting(ti, tw, experts, dim, torch.bfloat16, block_size=block)
+        aiter_amd.fmoe_fp8_blockscale_g1u1(out, t["x"], w1, w2, s_ids, s_w, s_e, nv, topk, None, s1, s2, "", 128, 128, None, 0, block)
+        return [tw, ti, out]
+
+    replay_and_compare(build, refill, run)
