@@ -1923,14 +1923,15 @@ static bool cols_fit(const MoeArgs& a)
 static bool few_rows(const MoeArgs& a) { return (size_t)a.M * a.topk * a.dim * 4 <= ((size_t)32 << 20); }
 
 // Rows through memory, in fp32, where the column kernel fits but takes longer.  (With one walker, where the tables of two no
-// longer fit, it is behind anyhow: 2 % at 288-320 tokens of the DeepSeek-V3 layer.  A call that names its tiles, or rows through
-// memory, has rows in fp32 up to 32 MiB only.)  In fp32 rows are summed with one rounding less per product: against 64 bits 5.4e-8 to 6.2e-8 for topk 6 and 8 and
+// longer fit, it is behind anyhow: 2 % at 288-320 tokens of the DeepSeek-V3 layer.)  Which kernels write the rows, by choice or by name,
+// has no say in this, so that tiles and blocks give the same bits; a call that names rows through memory ("down=rows") has them in fp32
+// up to 32 MiB only.  In fp32 rows are summed with one rounding less per product: against 64 bits 5.4e-8 to 6.2e-8 for topk 6 and 8 and
 // inter 128 and 256, in columns 5.8e-8 to 6.8e-8.
 // Columns stay where fp32 rows would take more scratch than a call can be recorded with (dim from 8192 on, and thousands of slots of
 // padding from sorting in blocks of 64 or 128; 513 tokens, 160 experts, top-24, 8960 x 128 in blocks of 128: 1.1 GiB, 406 us against 526).
 static bool rows_in_place_of_columns(const MoeArgs& a)
 {
-    if(a.down_mode != 0 || !cols_fit(a) || cols_walkers(a) != 2 || (a.tiles128 == 1 && !few_rows(a)))
+    if(a.down_mode != 0 || !cols_fit(a) || cols_walkers(a) != 2)
         return false;
     if(!few_rows(a) && std::max(block_wise_workspace_bytes(a, true), moe_prefill_workspace_bytes(a, true)) > kMaxCapturedLayerBytes)
         return false;

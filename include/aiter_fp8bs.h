@@ -308,12 +308,13 @@ int moe_sorting_fwd(aiter_tensor_t* topk_ids, aiter_tensor_t* topk_weights, aite
  *   fc2_smooth_scale must be NULL; kernel_name names the reference's tuned kernels and is only a
  *   tuning hint here ("nt=1|2|4", "dw=2|4|8", "dc=2|4|8", "down=rows", "down=cols", "pair=0|1", "tail=0",
  *   "stage=0", "ring=0", "tiles=0|1"; "out=write" stores the sums whatever out held; several joined by
- *   commas; anything else: choose).  No hint changes a result but the second GEMM's ("down=cols" sums in
- *   sorted order).
+ *   commas; anything else: choose).  No hint changes a result but those that name where rows are summed: "down=cols" sums in
+ *   sorted order; "down=rows", and "tiles=1" where the library would have chosen columns, in slot order, of rows that wait
+ *   in 16 bits where they take more than 32 MiB.
  * The product of the first GEMM is quantised 1x128 to fp8 for the second.  Each token's k
- * contributions are added in a fixed order (sorted order while the per-token tables of the second GEMM fit
- * the LDS, about 280 tokens at inter = 256; slot order beyond):
- * results do not depend on timing.  Scratch memory: see the top of this file.
+ * contributions are added in a fixed order (sorted order where the second GEMM owns columns: few tokens, up to about 280 at
+ * inter = 256, on layers wide enough for it; else slot order, of rows in fp32 up to 32 MiB and where they stand in for
+ * columns, in bf16 beyond): results do not depend on timing.  Scratch memory: see the top of this file.
  */
 int fmoe_fp8_blockscale_g1u1(aiter_tensor_t* out, aiter_tensor_t* input, aiter_tensor_t* gate, aiter_tensor_t* down,
                              aiter_tensor_t* sorted_token_ids, aiter_tensor_t* sorted_weights,

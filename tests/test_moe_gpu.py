@@ -624,6 +624,19 @@ def test_fmoe_rows_in_place_of_columns_stay_in_fp32(dtype):
     assert error[""] < error["down=rows,tiles=0"] * (1 if dtype == torch.bfloat16 else 0.8)
 
 
+@pytest.mark.parametrize("tokens,dim,experts,topk", [
+    (540, 3584, 64, 8),   # 62 MB of rows, in tiles by the library's own choice
+    (400, 3072, 256, 8),  # 39 MB, block by block
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_fmoe_rows_in_place_of_columns_whatever_kernels_write_them(tokens, dim, experts, topk, dtype):
+    # beyond 32 MiB, too: tiles asked for or refused by name give the bits of the library's own choice
+    p = make_moe(tokens, dim, 128, experts, topk, seed=tokens, w_std=0.05)
+    auto, block_wise, tiles = (run_moe(p, dtype=dtype, bf16_input=True, kernel_name=h) for h in ("", "tiles=0", "tiles=1"))
+    assert torch.equal(auto.view(torch.int16), block_wise.view(torch.int16))
+    assert torch.equal(auto.view(torch.int16), tiles.view(torch.int16))
+
+
 @pytest.mark.parametrize("topk", [1, 2, 3, 5, 8, 9, 10, 11, 23])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_fmoe_sum_of_fp32_rows(topk, dtype):
