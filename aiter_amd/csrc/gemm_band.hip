@@ -1,5 +1,5 @@
 // Block-scale FP8 GEMM, up to 256 activation rows by a band of 96 or 144 weight rows per workgroup: one round of workgroups
-// that covers the chip where 128-row tiles do not, with the weights requested several K blocks further ahead than the rows.
+// that covers the chip where 128-row tiles do not.
 //
 // Carries out, where it is faster (gemm_rules.h), what was chosen for other kernels with K in one range; the additions are the same,
 // so the bits are too.  By name it takes any size that the prefill_* kernels take.
@@ -7,17 +7,18 @@
 // Why bands of 144.  With 256 rows of weights per workgroup 36864 of them are 144 workgroups, with 192 they are 192, with 128
 // a round and a fragment of one; with 144 they are 256, and a workgroup's K block is 18 KiB of weights beside the rows'.
 //
-// Why two rings.  A stage of gemm_ring.h holds a K block of both operands, three stages fill the LDS, and two K blocks are all
-// that is ever on the way: 2 x 16 KiB of weights per compute unit, which at 2.5 us from memory under load is 3.7 TB/s over the
-// chip.  The rows come from L2 and need less of a head start.  With a ring of their own they keep three stages, and the
-// weights take what is left: four to six.  A wave's loads are counted in the order they were issued, so that each operand
-// has its own fetching waves (two and two) and waits for its own depth.
+// Why two rings.  The rows come from L2, the weights from memory, and a wave's loads are counted in the order they were issued: with
+// fetching waves of its own (two and two) each operand waits for its own depth only, and has a ring of its own.  The rows keep three
+// stages; the weights take what is left, up to six: bands of 144 four or more up to 208 rows (224 with scales that come K block by K
+// block), three beyond, where both operands are two K blocks ahead, as in gemm_ring.h.  The gain over other tilings does not
+// end there: 203, 224, 240 and 256 x 36864 x 7168 take 62.9, 64.1, 66.7 and 67.8 us, so most of it is the covered chip.
 //
-// Bound by, with few rows, the weights (64 x 36864 x 7168, were it one range: 44 us, 6.1 TB/s); beyond, by what a compute unit takes in and multiplies
-// per K block: 203 rows 71 us, 256 rows 73.  us before (192-wide tiles, mid_* tilings) / here, K in one range:
-//   203 x 36864 x 7168 92 / 71   512 x 18432 x 7168 88 / 68   1024 x 9216 x 7168 86 / 71   75 x 34496 x 1920 28 / 17
-//   86 x 35136 x 1152 20 / 13    288 x 17024 x 2816 33 / 26   2044 x 4480 x 1024 18 / 16   1439 x 5760 x 3072 34 / 28
-// Taken out again: two stages of rows (203 x 36864 x 7168 81 us: a K block then waits for L2).
+// Bound by, with few rows, the weights (64 x 36864 x 7168 by name: 45 us, 5.9 TB/s); beyond, by what a compute unit takes in and
+// multiplies per K block.  us of 192-wide tiles or mid_128x128, K in one range / here, calls in a loop over several copies of the weights
+// (among calls of other kinds 203 x 36864 x 7168 takes 104 / 72):
+//   203 x 36864 x 7168 102 / 63   512 x 18432 x 7168 94 / 66   1024 x 9216 x 7168 87 / 64   75 x 34496 x 1920 26 / 17
+//   86 x 35136 x 1152 18 / 13     288 x 17024 x 2816 39 / 25   2044 x 4480 x 1024 17 / 15   1439 x 5760 x 3072 34 / 28
+// Taken out again: two stages of rows (203 x 36864 x 7168 81 us among other calls: a K block then waits for L2).
 #include "gemm_ring.h"
 #include "gemm_rules.h"
 
@@ -394,13 +395,23 @@ __global__ __launch_bounds__(kBandThreads) void gemm_band_kernel(GemmKernelParam
 #undef FP8BS_MFMA
 #undef FP8BS_FMA4
 
+constexpr int kLds = 160 * 1024;
+constexpr int scale_bytes(bool xs4) { return xs4 ? 2 * kBandRows * 16 : 3 * kBandRows * 4; }
+constexpr int weight_stages(int rows, int nf, bool xs4)
+{
+    return std::min(6, (kLds - kXStages * rows * 128 - scale_bytes(xs4)) / (16 * nf * 128));
+}
+// The waits count w_stages - 2 K blocks of the youngest loads, at most four: three to six stages, fewest with the most rows
+static_assert(weight_stages(kBandRows, 9, true) == 3 && weight_stages(kBandRows, 9, false) == 3 && weight_stages(kBandRows, 6, true) == 4 &&
+              weight_stages(208, 9, true) == 4 && weight_stages(224, 9, true) == 3 && weight_stages(224, 9, false) == 4 &&
+              weight_stages(240, 9, false) == 3 && weight_stages(16, 9, true) == 6, "stages of weights");
+
 BandLayout band_layout(const GemmKernelParams& p, int nf, bool xs4)
 {
-    constexpr int kLds = 160 * 1024;
     BandLayout l{};
     l.rows     = std::min((p.M + 15) & ~15, kBandRows);
-    const int scales = xs4 ? 2 * kBandRows * 16 : 3 * kBandRows * 4, stage = 16 * nf * 128;
-    l.w_stages = std::min(6, (kLds - kXStages * l.rows * 128 - scales) / stage);
+    const int scales = scale_bytes(xs4), stage = 16 * nf * 128;
+    l.w_stages = weight_stages(l.rows, nf, xs4);
     l.w_at     = kXStages * l.rows * 128;
     l.xs_at    = l.w_at + l.w_stages * stage;
     l.total    = std::max(l.xs_at + scales, kMulWaves * 32 * (16 * nf * 2 + 16));

@@ -202,7 +202,8 @@ constexpr uint32_t kGateUpStage   = kGateUpX + kTileRows * 128;
 constexpr uint32_t kGateUpRingEnd = kGateUpRing + kGateUpStages * kGateUpStage;
 constexpr uint32_t kHPitch        = 272;                // bytes per row of the product (128 columns, bf16) in LDS
 constexpr size_t   kGateUpLds     = kGateUpRingEnd;
-static_assert(kGateUpLds <= 160 * 1024 && kTileRows * kHPitch <= kGateUpStages * kGateUpStage, "LDS");
+static_assert(kGateUpLds <= 160 * 1024, "LDS");
+static_assert(kTileRows * kHPitch <= kGateUpStage, "the product lies in one stage: the next item's first K blocks are landing in the others");
 static_assert((kGateUpWaves & (kGateUpWaves - 1)) == 0, "remainders by a mask");
 
 #define FP8BS_MFMA(P, A, B) asm volatile("v_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, 0" : "=&v"(P) : "v"(A), "v"(B))

@@ -63,6 +63,11 @@ int main()
     EXPECT(rows_beat_columns(140 * 6, 64, 64, 1536, 128) && !rows_beat_columns(140 * 6, 64, 64, 512, 128));
     EXPECT(!rows_beat_columns(16 * 8, 256, 256, 7168, 256) && !rows_beat_columns(128 * 8, 256, 256, 7168, 256));
     EXPECT(!rows_beat_columns(5, 32, 32, 1024, 256) && !rows_beat_columns(140 * 6, 64, 4, 1536, 128));
+    // the six layers whose bits test_fmoe_few_tokens_take_columns_or_rows compares: which side they are on
+    EXPECT(rows_beat_columns(140 * 6, 64, 64, 1536, 128) && rows_beat_columns(29 * 8, 256, 256, 1024, 128) && rows_beat_columns(270 * 3, 5, 5, 1280, 256));
+    EXPECT(!rows_beat_columns(140 * 6, 64, 64, 768, 128) && !rows_beat_columns(16 * 8, 64, 64, 5120, 256) && !rows_beat_columns(3 * 5, 32, 32, 1024, 256));
+    // and the ones beyond 32 MiB of rows
+    EXPECT(rows_beat_columns(540 * 8, 64, 64, 3584, 128) && rows_beat_columns(400 * 8, 256, 256, 3072, 128));
     // Tiles on both sides of where they were measured to win: (rows per expert, experts, dim, inter)
     auto tiles = [](int rows, int experts, int dim, int inter) { return fp8bs::tiles_win((int64_t)rows * experts, experts, experts, inter, dim); };
     struct
